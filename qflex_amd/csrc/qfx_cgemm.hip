@@ -1,7 +1,7 @@
-// Complex64 GEMM / GEMV / dot for the contraction path (gfx950).
+// Complex64 GEMM for the contraction path (gfx950).
 //
 // The reference hands every pairwise contraction to OpenBLAS
-// (cblas_cgemm / cgemv / cdotu_sub, reference src/tensor.cpp:960-1042).
+// (cblas_cgemm, reference src/tensor.cpp:960-980).
 //
 // MFMA form.  A complex A[m x k] (interleaved re,im) is read as a real
 // matrix Ahat[m x 2k].  B[k x n] is expanded, while staging from LDS, into
@@ -1411,73 +1411,13 @@ BigLayout tuned_layout(qfx_context* ctx, int precision, int am, uint64_t m, uint
   return best;
 }
 
-// ------------------------------------------------------------ GEMV / dot
+// ------------------------------------------------------------ vector-ALU forms
 __device__ __forceinline__ float2 cfma(float2 a, float2 b, float2 c) {
   c.x = fmaf(a.x, b.x, c.x);
   c.x = fmaf(-a.y, b.y, c.x);
   c.y = fmaf(a.x, b.y, c.y);
   c.y = fmaf(a.y, b.x, c.y);
   return c;
-}
-
-__device__ __forceinline__ float2 wave_sum(float2 v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    v.x += __shfl_xor(v.x, off);
-    v.y += __shfl_xor(v.y, off);
-  }
-  return v;
-}
-
-// y[m] = A[m x k] . x[k]; one wave per row, fixed lane-strided order.
-__global__ __launch_bounds__(256) void gemv_n_kernel(const float2* __restrict__ A,
-                                                     const float2* __restrict__ x,
-                                                     float2* __restrict__ y, uint64_t M,
-                                                     uint64_t K) {
-  const int lane = threadIdx.x & 63;
-  uint64_t row = uint64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  uint64_t rstride = uint64_t(gridDim.x) * 4;
-  for (; row < M; row += rstride) {
-    const float2* a = A + row * K;
-    float2 acc = make_float2(0.f, 0.f);
-    for (uint64_t k = lane; k < K; k += 64) acc = cfma(a[k], x[k], acc);
-    acc = wave_sum(acc);
-    if (lane == 0) y[row] = acc;
-  }
-}
-
-// y[c] = sum_r x[r] A[r][c] (A is m x k, row-major), split over rows.
-// Stage 1: block s reduces rows [s*rows_per, ...) for every column into
-// part[s][c]: 64 column lanes x 4 row groups, fixed order, LDS tree.
-__global__ __launch_bounds__(256) void gemv_t_partial_kernel(const float2* __restrict__ A,
-                                                             const float2* __restrict__ x,
-                                                             float2* __restrict__ part,
-                                                             uint64_t M, uint64_t K,
-                                                             uint64_t rows_per_split) {
-  __shared__ float2 red[4][64];
-  const uint64_t s = blockIdx.x;
-  const int cl = threadIdx.x & 63;
-  const int rg = threadIdx.x >> 6;
-  const uint64_t r0 = s * rows_per_split;
-  const uint64_t r1 = r0 + rows_per_split < M ? r0 + rows_per_split : M;
-  for (uint64_t c0 = 0; c0 < K; c0 += 64) {
-    const uint64_t c = c0 + cl;
-    float2 acc = make_float2(0.f, 0.f);
-    if (c < K)
-      for (uint64_t r = r0 + rg; r < r1; r += 4) acc = cfma(x[r], A[r * K + c], acc);
-    red[rg][cl] = acc;
-    __syncthreads();
-    if (rg == 0 && c < K) {
-      float2 t = red[0][cl];
-#pragma unroll
-      for (int g = 1; g < 4; ++g) {
-        t.x += red[g][cl].x;
-        t.y += red[g][cl].y;
-      }
-      part[s * K + c] = t;
-    }
-    __syncthreads();
-  }
 }
 
 // Stage 2 for few columns and many partials: one block per column, each
@@ -1534,29 +1474,6 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const float2* __restr
       y[c] = t;
     }
     __syncthreads();
-  }
-}
-
-// Block partial sums of x[i]*y[i] in a fixed per-lane order, then a tree.
-__global__ __launch_bounds__(256) void dot_partial_kernel(const float2* __restrict__ x,
-                                                          const float2* __restrict__ y,
-                                                          float2* __restrict__ part,
-                                                          uint64_t n) {
-  __shared__ float2 red[4];
-  float2 acc = make_float2(0.f, 0.f);
-  for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += uint64_t(gridDim.x) * blockDim.x)
-    acc = cfma(x[i], y[i], acc);
-  acc = wave_sum(acc);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float2 t = red[0];
-    for (int w = 1; w < 4; ++w) {
-      t.x += red[w].x;
-      t.y += red[w].y;
-    }
-    part[blockIdx.x] = t;
   }
 }
 
@@ -2078,67 +1995,6 @@ static int launch_smallk_splitk(qfx_context* ctx, const float2* A, const float2*
   return QFX_OK;
 }
 
-static int launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
-                         const float2* x, float2* y) {
-  // About 1024 row blocks of at least 16 rows each.
-  uint64_t nsplit = std::max<uint64_t>(1, std::min<uint64_t>(1024, (m + 15) / 16));
-  uint64_t rows_per = (m + nsplit - 1) / nsplit;
-  nsplit = (m + rows_per - 1) / rows_per;
-  void* ws = nullptr;
-  int st = qfx_workspace(ctx, nsplit * k * sizeof(float2), &ws);
-  if (st != QFX_OK) return st;
-  float2* part = static_cast<float2*>(ws);
-  gemv_t_partial_kernel<<<unsigned(nsplit), 256, 0, ctx->stream>>>(A, x, part, m, k, rows_per);
-  sum_partials_kernel<<<cap_grid((k + 63) / 64), 256, 0, ctx->stream>>>(part, y, nsplit, k);
-  QFX_HIP(hipGetLastError());
-  return QFX_OK;
-}
-
-extern "C" int qfx_cgemv_c64(qfx_context* ctx, int trans, uint64_t m, uint64_t k,
-                             const qfx_c64* A, const qfx_c64* x, qfx_c64* y) {
-  QFX_CHECK_CTX(ctx);
-  uint64_t ny = trans ? k : m;
-  if (ny == 0) return QFX_OK;
-  if (!A || !x || !y) return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemv_c64: null pointer");
-  if ((trans ? m : k) == 0) return qfx_zero(ctx, y, ny * sizeof(qfx_c64));
-  QFX_EXTENT(ctx, A, 8.0 * double(m) * double(k), "qfx_cgemv_c64: A");
-  QFX_EXTENT(ctx, x, 8.0 * double(trans ? m : k), "qfx_cgemv_c64: x");
-  QFX_EXTENT(ctx, y, 8.0 * double(ny), "qfx_cgemv_c64: y");
-  QfxLaunchScope scope(ctx, QFX_K_GEMV, 8.0 * (m * k + m + k), 8.0 * m * k);
-  const float2* A2 = reinterpret_cast<const float2*>(A);
-  const float2* x2 = reinterpret_cast<const float2*>(x);
-  float2* y2 = reinterpret_cast<float2*>(y);
-  if (!trans) {
-    gemv_n_kernel<<<cap_grid((m + 3) / 4), 256, 0, ctx->stream>>>(A2, x2, y2, m, k);
-    QFX_HIP(hipGetLastError());
-    return QFX_OK;
-  }
-  return launch_gemv_t(ctx, m, k, A2, x2, y2);
-}
-
-extern "C" int qfx_cdotu_c64(qfx_context* ctx, uint64_t n, const qfx_c64* x, const qfx_c64* y,
-                             qfx_c64* out) {
-  QFX_CHECK_CTX(ctx);
-  if (!out) return qfx_set_error(QFX_ERR_INVALID, "qfx_cdotu_c64: null output");
-  if (n == 0) return qfx_zero(ctx, out, sizeof(qfx_c64));
-  if (!x || !y) return qfx_set_error(QFX_ERR_INVALID, "qfx_cdotu_c64: null pointer");
-  QFX_EXTENT(ctx, x, 8.0 * double(n), "qfx_cdotu_c64: x");
-  QFX_EXTENT(ctx, y, 8.0 * double(n), "qfx_cdotu_c64: y");
-  QFX_EXTENT(ctx, out, 8.0, "qfx_cdotu_c64: out");
-  QfxLaunchScope scope(ctx, QFX_K_DOT, 16.0 * n, 8.0 * n);
-  uint64_t blocks = std::min<uint64_t>((n + 255) / 256, 1024);
-  void* ws = nullptr;
-  int st = qfx_workspace(ctx, blocks * sizeof(float2), &ws);
-  if (st != QFX_OK) return st;
-  float2* part = static_cast<float2*>(ws);
-  dot_partial_kernel<<<unsigned(blocks), 256, 0, ctx->stream>>>(
-      reinterpret_cast<const float2*>(x), reinterpret_cast<const float2*>(y), part, n);
-  sum_partials_kernel<<<1, 256, 0, ctx->stream>>>(part, reinterpret_cast<float2*>(out), blocks,
-                                                  1);
-  QFX_HIP(hipGetLastError());
-  return QFX_OK;
-}
-
 // Operand scales of the split-FP16 form: partial maxima of |A| and |B| in
 // one launch (at most 256 blocks per operand, at least 16 Ki elements
 // each), skipping an operand whose maxima its producer already wrote; the
@@ -2253,14 +2109,12 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
   if (precision == QFX_PREC_FP32_EXACT || !big) {
     if (n == 1 && precision != QFX_PREC_FP32_EXACT) {
       QfxLaunchScope scope(ctx, QFX_K_GEMV, bytes, flops);
-      gemv_n_kernel<<<cap_grid((m + 3) / 4), 256, 0, ctx->stream>>>(A2, B2, C2, m, k);
-      QFX_HIP(hipGetLastError());
-      return QFX_OK;
+      return qfx_launch_gemv_n(ctx, m, k, A2, B2, C2);
     }
     if (m == 1 && precision != QFX_PREC_FP32_EXACT) {
       QfxLaunchScope scope(ctx, QFX_K_GEMV, bytes, flops);
       // y[n] = sum_k a[k] B[k][n]: transposed GEMV of B (k x n) with x = A.
-      return launch_gemv_t(ctx, k, n, B2, A2, C2);
+      return qfx_launch_gemv_t(ctx, k, n, B2, A2, C2);
     }
     if (precision != QFX_PREC_FP32_EXACT && m * n <= 4096 && k >= 1024) {
       QfxLaunchScope scope(ctx, QFX_K_GEMV, bytes, flops);

@@ -1,0 +1,389 @@
+// Complex64 matrix-vector products and dot products of the contraction path
+// (gfx950): the closings cblas_cgemv / cblas_cdotu_sub of the reference
+// (src/tensor.cpp:982-1042).
+//
+// All of them read the matrix once and are bound by HBM (8 flop per 8
+// bytes), so the kernels only have to keep enough loads in flight on all
+// 256 CUs, for every aspect ratio: tall and narrow, short and wide.
+// Reductions run in a fixed order (no atomics): results are deterministic.
+// Measured against one wave per row (N) and against blocks that walked all
+// columns of 4 to 16 rows, 64 at a time (T), a plain copy running at 5.0 TB/s:
+//   T 4096 x 4096 (134 MB)   144 -> 32.5 us     N 4096 x 4096    36.7 -> 24.4 us
+//   T 227 x 37463 (68 MB)    842 -> 18.6 us     N 81 x 12430     51 -> 4.3 us
+//   T 16384 x 256 (34 MB)    74 -> 12.2 us      N 1000000 x 4    122 -> 7.8 us
+//   T 1000000 x 4 (32 MB)    141 -> 12.6 us     N 20000 x 2048   73.4 -> 62.1 us
+#include <algorithm>
+
+#include "qfx_internal.h"
+
+namespace {
+
+__device__ __forceinline__ float2 cfma(float2 a, float2 b, float2 c) {
+  c.x = fmaf(a.x, b.x, c.x);
+  c.x = fmaf(-a.y, b.y, c.x);
+  c.y = fmaf(a.x, b.y, c.y);
+  c.y = fmaf(a.y, b.x, c.y);
+  return c;
+}
+
+__device__ __forceinline__ float2 cadd(float2 a, float2 b) {
+  return make_float2(a.x + b.x, a.y + b.y);
+}
+
+// V complex values from p: one 16-byte load (V = 2) or one 8-byte load.
+template <int V>
+struct Vec {
+  float2 e[V];
+};
+template <int V>
+__device__ __forceinline__ Vec<V> load_vec(const float2* p) {
+  Vec<V> r;
+  if constexpr (V == 2) {
+    const float4 f = *reinterpret_cast<const float4*>(p);
+    r.e[0] = make_float2(f.x, f.y);
+    r.e[1] = make_float2(f.z, f.w);
+  } else {
+    r.e[0] = *p;
+  }
+  return r;
+}
+
+// y[m] = A[m x k] . x[k], many rows: groups of L = 2^llog lanes (L <= 64),
+// each R rows at a time, so that a load of x serves R rows and every lane
+// has R loads of A in flight.
+template <int V, int R>
+__global__ __launch_bounds__(256) void gemv_n_rows_kernel(const float2* __restrict__ A,
+                                                          const float2* __restrict__ x,
+                                                          float2* __restrict__ y, uint64_t M,
+                                                          uint64_t K, int llog) {
+  const int L = 1 << llog;
+  const int lane = threadIdx.x & (L - 1);
+  const uint64_t groups = uint64_t(256 >> llog) * gridDim.x;
+  const uint64_t units = K / V;  // loads per row (V divides K)
+  for (uint64_t g = (uint64_t(blockIdx.x) << (8 - llog)) + (threadIdx.x >> llog); g * R < M;
+       g += groups) {
+    const uint64_t r0 = g * R;
+    const float2* a[R];
+    float2 acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      a[r] = A + (r0 + r < M ? r0 + r : M - 1) * K;  // past the end: the last row again
+      acc[r] = make_float2(0.f, 0.f);
+    }
+    // U loads of x and U * R of A in flight per lane
+    constexpr int U = R == 1 ? 4 : 2;
+    uint64_t u = lane;
+    for (; u + (U - 1) * L < units; u += U * L) {
+      Vec<V> xv[U], av[U][R];
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        xv[j] = load_vec<V>(x + (u + j * L) * V);
+#pragma unroll
+        for (int r = 0; r < R; ++r) av[j][r] = load_vec<V>(a[r] + (u + j * L) * V);
+      }
+#pragma unroll
+      for (int j = 0; j < U; ++j)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int v = 0; v < V; ++v) acc[r] = cfma(av[j][r].e[v], xv[j].e[v], acc[r]);
+    }
+    for (; u < units; u += L) {
+      const Vec<V> xv = load_vec<V>(x + u * V);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const Vec<V> av = load_vec<V>(a[r] + u * V);
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[r] = cfma(av.e[v], xv.e[v], acc[r]);
+      }
+    }
+    for (int off = L >> 1; off > 0; off >>= 1)
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        acc[r].x += __shfl_xor(acc[r].x, off);
+        acc[r].y += __shfl_xor(acc[r].y, off);
+      }
+    if (lane == 0)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (r0 + r < M) y[r0 + r] = acc[r];
+  }
+}
+
+// y = A . x with few rows: one block per row, four loads in flight per
+// thread (the row is split over up to 16 waves instead of one).
+template <int V>
+__global__ __launch_bounds__(1024) void gemv_n_block_kernel(const float2* __restrict__ A,
+                                                            const float2* __restrict__ x,
+                                                            float2* __restrict__ y, uint64_t M,
+                                                            uint64_t K) {
+  __shared__ float2 red[16];
+  const uint64_t units = K / V, T = blockDim.x;
+  for (uint64_t row = blockIdx.x; row < M; row += gridDim.x) {
+    const float2* a = A + row * K;
+    float2 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = make_float2(0.f, 0.f);
+    uint64_t u = threadIdx.x;
+    for (; u + 3 * T < units; u += 4 * T) {
+      Vec<V> av[4], xv[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        av[j] = load_vec<V>(a + (u + j * T) * V);
+        xv[j] = load_vec<V>(x + (u + j * T) * V);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[j] = cfma(av[j].e[v], xv[j].e[v], acc[j]);
+    }
+    for (; u < units; u += T) {
+      const Vec<V> av = load_vec<V>(a + u * V), xv = load_vec<V>(x + u * V);
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[0] = cfma(av.e[v], xv.e[v], acc[0]);
+    }
+    float2 t = cadd(cadd(acc[0], acc[1]), cadd(acc[2], acc[3]));
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      t.x += __shfl_xor(t.x, off);
+      t.y += __shfl_xor(t.y, off);
+    }
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (unsigned w = 1; w < blockDim.x / 64; ++w) t = cadd(t, red[w]);
+      y[row] = t;
+    }
+    __syncthreads();
+  }
+}
+
+// Sum over the groups of a block of one value per thread, in a fixed tree:
+// thread t belongs to group t / CL (CL threads each, G = 256 / CL groups; the
+// threads past G * CL take no part).  The result is in group 0.
+__device__ __forceinline__ float2 group_sum(float2 v, float2* red, int CL, int G) {
+  const int t = threadIdx.x;
+  red[t] = v;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {  // group g takes over group g + w
+    if (t < w * CL && t + w * CL < G * CL) red[t] = cadd(red[t], red[t + w * CL]);
+    __syncthreads();
+  }
+  const float2 r = red[t];
+  __syncthreads();
+  return r;
+}
+
+// y[c] = sum_r x[r] A[r][c] (A is m x k, row-major).  Block (x, y): the
+// columns V * (CL x + lane) of the rows [rows_per * y, ...); its 256 threads
+// are G = 256 / CL row groups of CL column lanes, four rows in flight each.
+// A narrow matrix takes all its columns as the lanes (CL = k / V), so that
+// the block reads whole rows one after the other.  One split over the rows
+// writes y itself, several write part[split][c].
+template <int V>
+__global__ __launch_bounds__(256) void gemv_t_kernel(const float2* __restrict__ A,
+                                                     const float2* __restrict__ x,
+                                                     float2* __restrict__ out, uint64_t M,
+                                                     uint64_t K, uint64_t rows_per, int CL) {
+  __shared__ float2 red[256];
+  const int G = 256 / CL;
+  const int rg = threadIdx.x / CL, cl = threadIdx.x - rg * CL;
+  const uint64_t c = (uint64_t(blockIdx.x) * CL + cl) * V;
+  const uint64_t r0 = blockIdx.y * rows_per;
+  const uint64_t r1 = r0 + rows_per < M ? r0 + rows_per : M;
+  const bool in = rg < G && c < K;  // (V divides K)
+  float2 acc[4][V];  // one chain per row in flight
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[j][v] = make_float2(0.f, 0.f);
+  if (in) {
+    uint64_t r = r0 + rg;
+    for (; r + 3 * G < r1; r += 4 * G) {
+      Vec<V> a[4];
+      float2 xr[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        a[j] = load_vec<V>(A + (r + j * G) * K + c);
+        xr[j] = x[r + j * G];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[j][v] = cfma(xr[j], a[j].e[v], acc[j][v]);
+    }
+    for (; r < r1; r += G) {
+      const Vec<V> a = load_vec<V>(A + r * K + c);
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[0][v] = cfma(x[r], a.e[v], acc[0][v]);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    const float2 t = group_sum(cadd(cadd(acc[0][v], acc[1][v]), cadd(acc[2][v], acc[3][v])), red,
+                               CL, G);
+    if (rg == 0 && in) out[blockIdx.y * K + c + v] = t;
+  }
+}
+
+// y[c] = sum_s part[s][c]: CL columns per block, the splits shared by the
+// 256 / CL groups (CL a power of two).
+__global__ __launch_bounds__(256) void gemv_sum_kernel(const float2* __restrict__ part,
+                                                       float2* __restrict__ y, uint64_t nsplit,
+                                                       uint64_t K, int CL) {
+  __shared__ float2 red[256];
+  const int G = 256 / CL;
+  const int g = threadIdx.x / CL, cl = threadIdx.x - g * CL;
+  const uint64_t c = uint64_t(blockIdx.x) * CL + cl;
+  float2 acc = make_float2(0.f, 0.f);
+  if (c < K)
+    for (uint64_t s = g; s < nsplit; s += G) acc = cadd(acc, part[s * K + c]);
+  acc = group_sum(acc, red, CL, G);
+  if (g == 0 && c < K) y[c] = acc;
+}
+
+// Block partial sums of x[i]*y[i] in a fixed per-lane order, then a tree.
+__global__ __launch_bounds__(256) void dot_partial_kernel(const float2* __restrict__ x,
+                                                          const float2* __restrict__ y,
+                                                          float2* __restrict__ part,
+                                                          uint64_t n) {
+  __shared__ float2 red[256];
+  float2 acc = make_float2(0.f, 0.f);
+  for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += uint64_t(gridDim.x) * blockDim.x)
+    acc = cfma(x[i], y[i], acc);
+  acc = group_sum(acc, red, 1, 256);
+  if (threadIdx.x == 0) part[blockIdx.x] = acc;
+}
+
+// Smallest b with 2^b >= v (v >= 1), at most cap.
+int log2_ceil(uint64_t v, int cap) {
+  int b = 0;
+  while (b < cap && (uint64_t(1) << b) < v) ++b;
+  return b;
+}
+
+bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+void launch_sum(hipStream_t s, const float2* part, float2* y, uint64_t nsplit, uint64_t k) {
+  // Up to 16 columns per block (64 once k alone fills the chip), fewer where
+  // a thread would otherwise add up more than 8 partials one after the other.
+  int clog = k >= 65536 ? 6 : log2_ceil(k, 4);
+  while (clog > 1 && (nsplit << clog) > 8 * 256) --clog;
+  const int CL = 1 << clog;
+  gemv_sum_kernel<<<unsigned((k + CL - 1) / CL), 256, 0, s>>>(part, y, nsplit, k, CL);
+}
+
+template <int V>
+void launch_n(hipStream_t s, uint64_t m, uint64_t k, const float2* A, const float2* x, float2* y) {
+  const uint64_t units = k / V;
+  // Few rows: a block per row, if the row has enough loads to fill it (four
+  // per thread; below 512 rows one).  Otherwise the largest group of lanes
+  // that a row keeps four fifths busy (33 columns: 8 lanes, 5 loads each).
+  if ((m < 4096 && units >= 1024) || (m < 512 && units >= 256)) {
+    const unsigned threads = units >= 4096 && m <= 1024 ? 1024 : 256;
+    gemv_n_block_kernel<V><<<unsigned(m), threads, 0, s>>>(A, x, y, m, k);
+    return;
+  }
+  int llog = 6;
+  while (llog > 0 && 5 * units < 4 * ((((units - 1) >> llog) + 1) << llog)) --llog;
+  // rows per lane group: four share each load of x where there are enough rows
+  const uint64_t per_block = 256 >> llog;
+  const bool four = m >= 4 * per_block * 512;
+  const uint64_t groups = four ? (m + 3) / 4 : m;
+  const unsigned blocks =
+      unsigned(std::min<uint64_t>((groups + per_block - 1) / per_block, 65535));
+  if (four)
+    gemv_n_rows_kernel<V, 4><<<blocks, 256, 0, s>>>(A, x, y, m, k, llog);
+  else
+    gemv_n_rows_kernel<V, 1><<<blocks, 256, 0, s>>>(A, x, y, m, k, llog);
+}
+
+}  // namespace
+
+int qfx_launch_gemv_n(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A, const float2* x,
+                      float2* y) {
+  if (k % 2 == 0 && aligned16(A) && aligned16(x))
+    launch_n<2>(ctx->stream, m, k, A, x, y);
+  else
+    launch_n<1>(ctx->stream, m, k, A, x, y);
+  QFX_HIP(hipGetLastError());
+  return QFX_OK;
+}
+
+int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A, const float2* x,
+                      float2* y) {
+  const int V = k % 2 == 0 && aligned16(A) ? 2 : 1;
+  // column lanes: the whole row up to 128 loads (300000 x 33: 44 -> 20 us
+  // against 64 lanes, 31 of them idle), else tiles of 64
+  const uint64_t units = (k + V - 1) / V;
+  const int CL = units <= 128 ? int(units) : 64;
+  const uint64_t tile = uint64_t(V) * CL, tiles = (k + tile - 1) / tile;
+  // Row splits: about 2048 blocks in all (8 per CU), each row group of a
+  // block with at least 16 rows (four rounds of the four in flight: with 8,
+  // 16384 x 256 took 29 instead of 12 us, most of it adding up 1024
+  // partials), at most 1024 splits of at least 16 rows (the scratch is then
+  // never more than 1024 x k values).
+  const uint64_t G = 256 / CL;
+  const uint64_t want = (2048 + tiles - 1) / tiles;
+  uint64_t nsplit = std::min<uint64_t>({want, uint64_t(1024), (m + 16 * G - 1) / (16 * G),
+                                        (m + 15) / 16, uint64_t(65535)});
+  nsplit = std::max<uint64_t>(nsplit, 1);
+  const uint64_t rows_per = (m + nsplit - 1) / nsplit;
+  nsplit = (m + rows_per - 1) / rows_per;
+  if (tiles > 0x7fffffffULL) return qfx_set_error(QFX_ERR_UNSUPPORTED, "gemv: too many columns");
+  float2* out = y;
+  if (nsplit > 1) {
+    void* ws = nullptr;
+    const int st = qfx_workspace(ctx, nsplit * k * sizeof(float2), &ws);
+    if (st != QFX_OK) return st;
+    out = static_cast<float2*>(ws);
+  }
+  const dim3 g{unsigned(tiles), unsigned(nsplit), 1};
+  if (V == 2)
+    gemv_t_kernel<2><<<g, 256, 0, ctx->stream>>>(A, x, out, m, k, rows_per, CL);
+  else
+    gemv_t_kernel<1><<<g, 256, 0, ctx->stream>>>(A, x, out, m, k, rows_per, CL);
+  if (nsplit > 1) launch_sum(ctx->stream, out, y, nsplit, k);
+  QFX_HIP(hipGetLastError());
+  return QFX_OK;
+}
+
+extern "C" int qfx_cgemv_c64(qfx_context* ctx, int trans, uint64_t m, uint64_t k,
+                             const qfx_c64* A, const qfx_c64* x, qfx_c64* y) {
+  QFX_CHECK_CTX(ctx);
+  uint64_t ny = trans ? k : m;
+  if (ny == 0) return QFX_OK;
+  if (!A || !x || !y) return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemv_c64: null pointer");
+  if ((trans ? m : k) == 0) return qfx_zero(ctx, y, ny * sizeof(qfx_c64));
+  QFX_EXTENT(ctx, A, 8.0 * double(m) * double(k), "qfx_cgemv_c64: A");
+  QFX_EXTENT(ctx, x, 8.0 * double(trans ? m : k), "qfx_cgemv_c64: x");
+  QFX_EXTENT(ctx, y, 8.0 * double(ny), "qfx_cgemv_c64: y");
+  QfxLaunchScope scope(ctx, QFX_K_GEMV, 8.0 * (m * k + m + k), 8.0 * m * k);
+  const float2* A2 = reinterpret_cast<const float2*>(A);
+  const float2* x2 = reinterpret_cast<const float2*>(x);
+  float2* y2 = reinterpret_cast<float2*>(y);
+  return trans ? qfx_launch_gemv_t(ctx, m, k, A2, x2, y2) : qfx_launch_gemv_n(ctx, m, k, A2, x2, y2);
+}
+
+extern "C" int qfx_cdotu_c64(qfx_context* ctx, uint64_t n, const qfx_c64* x, const qfx_c64* y,
+                             qfx_c64* out) {
+  QFX_CHECK_CTX(ctx);
+  if (!out) return qfx_set_error(QFX_ERR_INVALID, "qfx_cdotu_c64: null output");
+  if (n == 0) return qfx_zero(ctx, out, sizeof(qfx_c64));
+  if (!x || !y) return qfx_set_error(QFX_ERR_INVALID, "qfx_cdotu_c64: null pointer");
+  QFX_EXTENT(ctx, x, 8.0 * double(n), "qfx_cdotu_c64: x");
+  QFX_EXTENT(ctx, y, 8.0 * double(n), "qfx_cdotu_c64: y");
+  QFX_EXTENT(ctx, out, 8.0, "qfx_cdotu_c64: out");
+  QfxLaunchScope scope(ctx, QFX_K_DOT, 16.0 * n, 8.0 * n);
+  uint64_t blocks = std::min<uint64_t>((n + 255) / 256, 1024);
+  void* ws = nullptr;
+  int st = qfx_workspace(ctx, blocks * sizeof(float2), &ws);
+  if (st != QFX_OK) return st;
+  float2* part = static_cast<float2*>(ws);
+  dot_partial_kernel<<<unsigned(blocks), 256, 0, ctx->stream>>>(
+      reinterpret_cast<const float2*>(x), reinterpret_cast<const float2*>(y), part, n);
+  launch_sum(ctx->stream, part, reinterpret_cast<float2*>(out), blocks, 1);
+  QFX_HIP(hipGetLastError());
+  return QFX_OK;
+}

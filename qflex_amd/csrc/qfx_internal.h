@@ -158,6 +158,14 @@ __device__ __forceinline__ uint64_t map_offset(const qfx_index_map& d, uint64_t 
   return off;
 }
 
+// Matrix-vector products of qfx_gemv.hip (pointers checked by the caller,
+// m, k > 0): y[m] = A[m x k] . x, without device scratch, and y[k] =
+// sum_r x[r] A[r][.].
+int qfx_launch_gemv_n(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A, const float2* x,
+                      float2* y);
+int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A, const float2* x,
+                      float2* y);
+
 // FP8 (E4M3, per-128x128-tile power-of-two scales) complex GEMM of
 // qfx_fp8.hip: whether the shape is large enough for its tiles, and the
 // launch (maps = {a_rows, a_cols, b_rows, b_cols} or null for row-major).

@@ -239,6 +239,32 @@ def test_cgemv(ctx, m, k):
     assert relerr(got.astype(np.complex128), xt.astype(np.complex128) @ a) < 2e-6
 
 
+# (m, k): one wave or block per row, lane groups per row, whole rows as column
+# lanes (k up to 128 loads) and column tiles, one and several row splits
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("m,k", [(1, 9), (511, 512), (513, 257), (600, 2049), (5000, 2048), (4097, 33),
+                                 (140000, 6), (131072, 1), (70000, 127), (65, 129), (33, 130), (40, 256),
+                                 (17, 258), (9000, 257), (3, 66000)])
+def test_cgemv_every_split(ctx, m, k, off):
+    """off = 1: A, x and y start 8 bytes past a 16-byte boundary."""
+    class At:
+        def __init__(self, buf):
+            self.ptr = buf.ptr + 8 * off
+
+    rng = np.random.default_rng(m + k)
+    a, x, xt = rand_c64(rng, (m * k + off,)), rand_c64(rng, (k + off,)), rand_c64(rng, (m + off,))
+    A, X, XT, Y = ctx.upload(a), ctx.upload(x), ctx.upload(xt), ctx.alloc((max(m, k) + off) * 8)
+    wide = a[off:].reshape(m, k).astype(np.complex128)
+    ctx.cgemv(0, m, k, At(A), At(X), At(Y))
+    got = ctx.download(Y, np.complex64, (m + off,))[off:]
+    assert relerr(got.astype(np.complex128), wide @ x[off:]) < 2e-6
+    ctx.cgemv(1, m, k, At(A), At(XT), At(Y))
+    got = ctx.download(Y, np.complex64, (k + off,))[off:]
+    assert relerr(got.astype(np.complex128), xt[off:] @ wide) < 2e-6
+    for buf in (A, X, XT, Y):
+        buf.free()
+
+
 @pytest.mark.parametrize("n", [1, 5, 256, 65537, 1 << 22])
 def test_cdotu_unconjugated(ctx, n):
     rng = np.random.default_rng(n)
