@@ -49,6 +49,31 @@ def test_mlp_forward_and_gradients_vs_oracle(ctx, B):
         b.free()
 
 
+@pytest.mark.parametrize("B", [31, 32, 33, 8191, 16417])
+def test_mlp_batches_around_the_row_tiles(ctx, B):
+    """Whole and ragged 32-row tiles, and more tiles than blocks (8192 rows
+    when training, 16384 forward): FP32 sums of up to 256 products, so y is
+    off by at most the odd activation rounded the other way (2^-9 of one of
+    256 terms); the batch sums average that out further."""
+    p, X, t = case(B, B)
+    P, DX, DT = ctx.upload(p), ctx.upload(X), ctx.upload(t)
+    Y, G, L = ctx.alloc(4 * B), ctx.alloc(4 * mlp.N_PARAMS), ctx.alloc(4)
+    ctx.mlp_forward(B, DX, P, Y)
+    y_ref, _ = mlp.forward(p, X, rounding=True)
+    assert relerr(ctx.download(Y, np.float32, (B,)), y_ref) < 2e-3
+    ctx.mlp_backward(B, DX, DT, P, G, L)
+    g = ctx.download(G, np.float32, (mlp.N_PARAMS,)).astype(np.float64)
+    loss_ref, g_ref = mlp.loss_and_grads(p, X, t, rounding=True)
+    assert abs(float(ctx.download(L, np.float32, (1,))[0]) - loss_ref) <= 2e-3 * loss_ref
+    o = 0
+    for name, shape in mlp.SIZES:
+        n = int(np.prod(shape))
+        assert relerr(g[o:o + n], g_ref[o:o + n]) < 2e-2, (B, name)
+        o += n
+    for b in (P, DX, DT, Y, G, L):
+        b.free()
+
+
 def test_mlp_adam_training_reduces_loss(ctx):
     # a smooth target of the features: the network must fit it
     rng = np.random.default_rng(0)
