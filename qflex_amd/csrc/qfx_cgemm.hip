@@ -326,17 +326,10 @@ __device__ __forceinline__ float absmax4(float4 v) {
   return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
 
-__global__ __launch_bounds__(256) void amax_partial_kernel(const float2* __restrict__ A,
-                                                           uint64_t na,
-                                                           const float2* __restrict__ B,
-                                                           uint64_t nb, int blocks_a,
-                                                           float* __restrict__ part) {
-  __shared__ float red[4];
-  const bool is_a = int(blockIdx.x) < blocks_a;
-  const float2* x = is_a ? A : B;
-  const uint64_t n = is_a ? na : nb;
-  const uint64_t nblk = is_a ? uint64_t(blocks_a) : uint64_t(gridDim.x - blocks_a);
-  const uint64_t b = is_a ? blockIdx.x : blockIdx.x - blocks_a;
+// Maximum over the elements block b of nblk takes of x, by the block's
+// thread 0 to *out; red holds 4 floats of LDS.
+__device__ __forceinline__ void amax_block(const float2* __restrict__ x, uint64_t n, uint64_t b,
+                                           uint64_t nblk, float* red, float* __restrict__ out) {
   const uint64_t stride = nblk * 256;
   float m = 0.f;
   if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
@@ -364,7 +357,19 @@ __global__ __launch_bounds__(256) void amax_partial_kernel(const float2* __restr
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  if (threadIdx.x == 0) *out = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+__global__ __launch_bounds__(256) void amax_partial_kernel(const float2* __restrict__ A,
+                                                           uint64_t na,
+                                                           const float2* __restrict__ B,
+                                                           uint64_t nb, int blocks_a,
+                                                           float* __restrict__ part) {
+  __shared__ float red[4];
+  const bool is_a = int(blockIdx.x) < blocks_a;
+  const uint64_t nblk = is_a ? uint64_t(blocks_a) : uint64_t(gridDim.x - blocks_a);
+  const uint64_t b = is_a ? blockIdx.x : blockIdx.x - blocks_a;
+  amax_block(is_a ? A : B, is_a ? na : nb, b, nblk, red, part + blockIdx.x);
 }
 
 // Partial maxima of the operands of one split-FP16 GEMM (from
@@ -1113,6 +1118,26 @@ __global__ __launch_bounds__(64 * WM * WN) void cgemm_split_chain_kernel(
       int(L % gy) * 16 * J * WN, L, gridDim.x, ntiles, gy);
 }
 
+// The last of `count` > 0 entries of a grouped launch whose first index (at
+// `first`, stride `bytes`, increasing, 0 at entry 0) is <= t.  Called by whole
+// waves: 64 entries are probed at a time, so 192 entries take two dependent
+// loads, where a binary search takes eight (4 us of each block's life).
+__device__ __forceinline__ int group_entry(const uint64_t* first, size_t bytes, int count,
+                                           uint64_t t) {
+  const int lane = threadIdx.x & 63;
+  int lo = 0, n = count;
+  while (n > 1) {
+    const int step = (n + 63) / 64;
+    const int i = lane * step;
+    const bool le = i < n && *reinterpret_cast<const uint64_t*>(
+                                 reinterpret_cast<const char*>(first) + size_t(lo + i) * bytes) <= t;
+    const int c = __popcll(__ballot(le)) - 1;  // the last probed entry <= t
+    lo += c * step;
+    n = min(step, n - c * step);
+  }
+  return __builtin_amdgcn_readfirstlane(lo);
+}
+
 // One problem of a grouped launch: row-major operands, 256 x 128 tiles.
 struct GroupTile {
   const float2* A;
@@ -1120,8 +1145,25 @@ struct GroupTile {
   float2* C;
   int M, N, K, tiles_m;
   uint64_t first_tile;  // index of the problem's first tile in the launch
+  uint64_t first_part;  // index of its first partial maximum (split FP16)
   AmaxRef amax;
 };
+
+// The operand maxima of all problems of a grouped launch: block b runs its
+// block of A or B of the problem whose partial maxima b is among.  (One
+// launch per problem cost 3 us each.)
+__global__ __launch_bounds__(256) void amax_grouped_kernel(const GroupTile* __restrict__ probs,
+                                                           int count, float* __restrict__ part) {
+  __shared__ float red[4];
+  const uint64_t t = blockIdx.x;
+  const GroupTile& g =
+      probs[group_entry(&probs[0].first_part, sizeof(GroupTile), count, t)];
+  const int b = int(t - g.first_part);
+  const bool is_a = b < g.amax.na;
+  const uint64_t m = uint64_t(g.M), n = uint64_t(g.N), k = uint64_t(g.K);
+  amax_block(is_a ? g.A : g.B, is_a ? m * k : k * n, is_a ? b : b - g.amax.na,
+             is_a ? g.amax.na : g.amax.nb, red, part + t);
+}
 
 // Persistent grouped launch: the blocks walk the tiles of all problems
 // (problems of any shape, tiles numbered problem by problem), each block
@@ -1131,13 +1173,8 @@ __global__ __launch_bounds__(512) void cgemm_split_grouped_kernel(const GroupTil
                                                                   int count, uint64_t total) {
   const qfx_index_map none{};
   for (uint64_t t = blockIdx.x; t < total; t += gridDim.x) {
-    int lo = 0, hi = count - 1;  // the last problem whose first tile is <= t
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (probs[mid].first_tile <= t) lo = mid;
-      else hi = mid - 1;
-    }
-    const GroupTile g = probs[lo];
+    const GroupTile g =
+        probs[group_entry(&probs[0].first_tile, sizeof(GroupTile), count, t)];
     const uint64_t local = t - g.first_tile;
     const int tm = int(local % uint64_t(g.tiles_m)), tn = int(local / uint64_t(g.tiles_m));
     split_big_tile<MODE, 4, 2, 4, 0>(g.A, g.B, g.C, g.M, g.N, g.K, g.amax, none, none, none, none,
@@ -1933,13 +1970,7 @@ struct RowsProb {
 __global__ __launch_bounds__(256) void cgemm_rows_grouped_kernel(const RowsProb* __restrict__ probs,
                                                                  int count) {
   const uint64_t b = blockIdx.x;
-  int lo = 0, hi = count - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (probs[mid].first_block <= b) lo = mid;
-    else hi = mid - 1;
-  }
-  const RowsProb p = probs[lo];
+  const RowsProb p = probs[group_entry(&probs[0].first_block, sizeof(RowsProb), count, b)];
   const qfx_index_map none{};
   rows_tile<false, false>(p.A, p.B, p.C, p.M, p.N, p.K, none, none, none, none, nullptr,
                           b - p.first_block);
@@ -2415,6 +2446,19 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
 
 // ------------------------------------------------------------ grouped products
 
+// A grouped launch's problem list to the device, through the staged uploads
+// and launched at once: in pieces of one 16-byte load per thread of an
+// upload's block, so that the whole list takes one trip over the bus.
+static int upload_problems(qfx_context* ctx, void* dev, const void* host, size_t bytes) {
+  for (size_t at = 0; at < bytes; at += 4096) {
+    const int st = qfx_copy_h2d_async(ctx, static_cast<char*>(dev) + at,
+                                      static_cast<const char*>(host) + at,
+                                      std::min<size_t>(4096, bytes - at));
+    if (st != QFX_OK) return st;
+  }
+  return qfx_flush_uploads(ctx);
+}
+
 // The row-kernel problems of a grouped call in one launch.  The problem
 // list goes to the device through the staged uploads (flushed right before
 // the launch) into the workspace.
@@ -2436,9 +2480,7 @@ static int launch_rows_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
   void* ws = nullptr;
   int st = qfx_workspace(ctx, probs.size() * sizeof(RowsProb), &ws);
   if (st != QFX_OK) return st;
-  st = qfx_copy_h2d_async(ctx, ws, probs.data(), probs.size() * sizeof(RowsProb));
-  if (st != QFX_OK) return st;
-  st = qfx_flush_uploads(ctx);
+  st = upload_problems(ctx, ws, probs.data(), probs.size() * sizeof(RowsProb));
   if (st != QFX_OK) return st;
   QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
   cgemm_rows_grouped_kernel<<<unsigned(blocks), 256, 0, ctx->stream>>>(
@@ -2497,12 +2539,14 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
     flops += 8.0 * double(d.m) * double(d.n) * double(d.k);
     bytes += 8.0 * (double(d.m) * d.k + double(d.k) * d.n + double(d.m) * d.n);
     if (precision == QFX_PREC_SPLIT_FP16) {
-      blocks[g][0] = int(std::min<uint64_t>(256, std::max<uint64_t>(1, (d.m * d.k + 16383) / 16384)));
-      blocks[g][1] = int(std::min<uint64_t>(256, std::max<uint64_t>(1, (d.k * d.n + 16383) / 16384)));
+      blocks[g][0] = int(std::min<uint64_t>(256, (d.m * d.k + 4095) / 4096));
+      blocks[g][1] = int(std::min<uint64_t>(256, (d.k * d.n + 4095) / 4096));
       nparts += size_t(blocks[g][0] + blocks[g][1]);
     }
   }
   QfxLaunchScope scope(ctx, QFX_K_CGEMM, bytes, flops);
+  if (nparts > 0x7fffffffULL)
+    return qfx_set_error(QFX_ERR_UNSUPPORTED, "qfx_cgemm_grouped_c64: too many operand blocks");
   const size_t part_bytes = (nparts * sizeof(float) + 255) / 256 * 256;
   const size_t desc_bytes = grouped.size() * sizeof(GroupTile);
   void* ws = nullptr;
@@ -2510,21 +2554,13 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
   if (st != QFX_OK) return st;
   float* part = static_cast<float*>(ws);
   GroupTile* dev = reinterpret_cast<GroupTile*>(static_cast<char*>(ws) + part_bytes);
-  // host staging of the problem list: the previous grouped call's copy
-  // must have been read before the staging buffer is rewritten
-  if (!ctx->group_ev) QFX_HIP(hipEventCreateWithFlags(&ctx->group_ev, hipEventDisableTiming));
-  else QFX_HIP(hipEventSynchronize(ctx->group_ev));
-  ctx->group_host.resize(desc_bytes);
-  GroupTile* host = reinterpret_cast<GroupTile*>(ctx->group_host.data());
-  uint64_t tile = 0;
-  size_t off = 0;
+  std::vector<GroupTile> host(grouped.size());
+  uint64_t tile = 0, off = 0;
   for (size_t g = 0; g < grouped.size(); ++g) {
     const qfx_gemm_desc& d = descs[grouped[g]];
-    const float2* A2 = reinterpret_cast<const float2*>(d.A);
-    const float2* B2 = reinterpret_cast<const float2*>(d.B);
-    GroupTile t{};
-    t.A = A2;
-    t.B = B2;
+    GroupTile& t = host[g];
+    t.A = reinterpret_cast<const float2*>(d.A);
+    t.B = reinterpret_cast<const float2*>(d.B);
     t.C = reinterpret_cast<float2*>(d.C);
     t.M = int(d.m);
     t.N = int(d.n);
@@ -2532,18 +2568,16 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
     t.tiles_m = int((d.m + 255) / 256);
     t.first_tile = tile;
     tile += uint64_t(t.tiles_m) * ((d.n + 127) / 128);
-    if (precision == QFX_PREC_SPLIT_FP16) {
-      const int ba = blocks[g][0], bb = blocks[g][1];
-      amax_partial_kernel<<<unsigned(ba + bb), 256, 0, ctx->stream>>>(A2, d.m * d.k, B2,
-                                                                      d.k * d.n, ba, part + off);
-      t.amax = AmaxRef{part + off, ba, part + off + ba, bb};
-      off += size_t(ba + bb);
-    }
-    host[g] = t;
+    const int ba = blocks[g][0], bb = blocks[g][1];
+    t.first_part = off;
+    t.amax = AmaxRef{part + off, ba, part + off + ba, bb};
+    off += uint64_t(ba + bb);
   }
+  st = upload_problems(ctx, dev, host.data(), desc_bytes);
+  if (st != QFX_OK) return st;
+  if (nparts > 0)
+    amax_grouped_kernel<<<unsigned(nparts), 256, 0, ctx->stream>>>(dev, int(host.size()), part);
   QFX_HIP(hipGetLastError());
-  QFX_HIP(hipMemcpyAsync(dev, host, desc_bytes, hipMemcpyHostToDevice, ctx->stream));
-  QFX_HIP(hipEventRecord(ctx->group_ev, ctx->stream));
   if (ctx->cus <= 0) {
     int cus = 0;
     QFX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));

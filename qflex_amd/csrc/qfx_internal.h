@@ -60,11 +60,7 @@ struct qfx_context {
   };
   std::vector<Upload> uploads;
   std::map<uintptr_t, uintptr_t> upload_at;
-  // Grouped products: host staging of the problem list, the event after its
-  // copy to the device, and the compute-unit count (grid of the launch).
-  std::vector<unsigned char> group_host;
-  hipEvent_t group_ev = nullptr;
-  int cus = 0;
+  int cus = 0;  // compute units of the device (0: not yet read)
   bool autotune = false;
   std::map<std::array<uint64_t, 5>, int> tuned;
   hipEvent_t tune_ev[2] = {nullptr, nullptr};

@@ -86,7 +86,6 @@ extern "C" int qfx_context_destroy(qfx_context* ctx) {
   if (ctx->timer_stop) hipEventDestroy(ctx->timer_stop);
   for (auto ev : ctx->tune_ev)
     if (ev) hipEventDestroy(ev);
-  if (ctx->group_ev) hipEventDestroy(ctx->group_ev);
   ctx->uploads.clear();  // their destinations are freed with the arena
   if (ctx->stage) hipHostFree(ctx->stage);
   hipStreamDestroy(ctx->stream);
