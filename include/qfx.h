@@ -158,7 +158,9 @@ int qfx_cgemm_noalloc_c64(qfx_context* ctx, int precision, uint64_t m, uint64_t 
  * such products (numbered product by product), so many small or uneven
  * products fill the GPU together; each result is bit-identical to that
  * product computed alone on the 256 x 128 tile (split FP16: one max-abs
- * launch over all of them precedes the grouped launch).  Products with k <= 16
+ * launch over all of them precedes the grouped launch).  The products with an
+ * odd k or n or 8-byte aligned operands that qfx_cgemm_c64 would run split
+ * share a second such launch, on 128 x 64 tiles (same bits).  Products with k <= 16
  * and n <= 16 (any precision) also share one launch, of the exact-FP32 row
  * kernel qfx_cgemm_c64 runs them on (same bits); the problem list reaches
  * the device through the staged uploads.  All other products run one by

@@ -23,6 +23,7 @@
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
@@ -434,7 +435,9 @@ typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
 
 // Same tiling as cgemm_bf16_mfma_kernel; two FP16 planes (hi, lo) of the
 // scaled operands, products hi*hi + hi*lo + lo*hi in one FP32 accumulator,
-// unscaled on output.
+// unscaled on output.  (Both kernels: 64-bit addressing, for operands beyond
+// the 32-bit offsets of split_big_tile that its large tiles don't take; the
+// same bits as those.)
 __global__ __launch_bounds__(256) void cgemm_fp16x2_mfma_kernel(
     const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C, int M,
     int N, int K, AmaxRef amax) {
@@ -642,8 +645,10 @@ __device__ __forceinline__ floatx16 mfma16(typename SplitTraits<MODE>::V a,
 // prologue overlaps the previous tile's last stages and C write-back.
 // cmax_slot then points at the per-tile maxima (slot L).  Needs an even
 // number of k-stages and whole-operand addressing (not WIDE).
+// ODD (AM 0): odd k or n, or operands at 8 bytes: a thread's two elements are
+// read by two 8-byte loads with their own bounds instead of one of 16 bytes.
 template <int MODE, int WM, int WN, int J, int AM, int I = 2, bool WIDE = false,
-          bool CHAIN = false>
+          bool CHAIN = false, bool ODD = false>
 __device__ __forceinline__ void split_big_tile(
     const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C, int M,
     int N, int K, AmaxRef amax, const qfx_index_map& a_rows, const qfx_index_map& a_cols,
@@ -651,6 +656,7 @@ __device__ __forceinline__ void split_big_tile(
     const int m0_first, const int n0_first, const unsigned L0 = 0, const unsigned Lstride = 0,
     const unsigned Lend = 0, const unsigned gy = 1) {
   static_assert(!(CHAIN && WIDE), "chained tiles use whole-operand addressing");
+  static_assert(!ODD || AM == 0, "digit maps have power-of-two runs");
   constexpr int NTH = 64 * WM * WN;  // threads of the block
   static_assert(NTH == 512 || NTH == 256, "8 or 4 waves");
   typedef typename SplitTraits<MODE>::T T;
@@ -674,11 +680,25 @@ __device__ __forceinline__ void split_big_tile(
   float sa = 1.f, sb = 1.f;
   int m0 = m0_first, n0 = n0_first;  // the tile being computed
 
-  // global -> register assignment (f = tid + 512*h, g = tid + 512*h)
+  // global -> register assignment (f = tid + NTH*h, g = tid + NTH*h)
   // A, AM 0/1: row = f >> 2, q = f & 3 (complex k = 2q, 2q+1 of the stage)
-  // A, AM 2:   kk = f & 7, row = 2*(f >> 3) (complex rows row, row+1)
-  // B: kk = g & 7 (consecutive lanes take consecutive k, so the LDS stores
-  //    are conflict-free), nq = g >> 3 (complex n = 2nq, 2nq+1)
+  // A, AM 2:   k = pair_k(f), rows 2*pair_i(f) and the next
+  // A, ODD:    k = f & 7, rows 2*(f >> 3) and the next
+  // B:         k = pair_k(g), columns 2*pair_i(g) and the next
+  // B, ODD:    k = (g >> 3) & 7, columns 16*(g >> 6) + (g & 7) and 8 after it
+  // pair_k, pair_i: four lanes read 64 contiguous bytes, and the half wave
+  // that stores to LDS at once still holds 8 k of 4 pairs, which is
+  // conflict-free.  ODD: eight lanes read 64 contiguous bytes.  (With k
+  // fastest over the lanes every 16 bytes were an access of their own: 4096^3
+  // with A read along m 1525 -> 1430 us, 131072 x 512 x 256 506 -> 479, 65536 x 256 x 256
+  // 138 -> 132; with A read along k the same time.)
+  auto pair_k = [](int g) { return (g >> 2) & 7; };
+  auto pair_i = [](int g) { return (g & 3) | ((g >> 3) & 4) | ((g >> 6) << 3); };
+  auto a_k = [&](int f) { return ODD ? f & 7 : AM == 2 ? pair_k(f) : 2 * (f & 3); };
+  auto a_row = [&](int f) { return ODD ? 2 * (f >> 3) : AM == 2 ? 2 * pair_i(f) : f >> 2; };
+  auto b_k = [&](int g) { return ODD ? (g >> 3) & 7 : pair_k(g); };
+  auto b_col = [&](int g) { return ODD ? 16 * (g >> 6) + (g & 7) : 2 * pair_i(g); };
+  constexpr int kBStep = ODD ? 8 : 1;  // from a thread's first column of B to its second
   // Each operand is read through a buffer resource with 32-bit offsets.
   // Normally (WIDE false) the resource covers the whole operand, made once.
   // WIDE: it is based at the block's first row (A) or column (B) and at the
@@ -729,16 +749,15 @@ __device__ __forceinline__ void split_big_tile(
   auto tile_rows = [&](int tm0, auto* aoff) {
 #pragma unroll
     for (int h = 0; h < kAH; ++h) {
-      const int f = tid + NTH * h;
-      const int row = AM == 1 ? (f >> 2) : 2 * (f >> 3);
+      const int row = a_row(tid + NTH * h);
       aoff[h] = map_offset(a_rows, uint64_t(WIDE ? row : tm0 + row));
     }
   };
   auto tile_cols = [&](int tn0, auto* boff) {
 #pragma unroll
     for (int h = 0; h < kBH; ++h) {
-      const int g = tid + NTH * h;
-      boff[h] = map_offset(b_cols, uint64_t(WIDE ? 2 * (g >> 3) : tn0 + 2 * (g >> 3)));
+      const int col = b_col(tid + NTH * h);
+      boff[h] = map_offset(b_cols, uint64_t(WIDE ? col : tn0 + col));
     }
   };
   auto set_next = [&]() {  // the chain's tile after Lc, if any
@@ -764,9 +783,9 @@ __device__ __forceinline__ void split_big_tile(
   };
   if constexpr (AM != 0) {
     tile_rows(m0, a_off);
-    a_coff = map_offset(a_cols, AM == 1 ? uint64_t(2 * (tid & 3)) : uint64_t(tid & 7));
+    a_coff = map_offset(a_cols, uint64_t(a_k(tid)));
     tile_cols(n0, b_off);
-    b_roff = map_offset(b_rows, uint64_t(tid & 7));
+    b_roff = map_offset(b_rows, uint64_t(b_k(tid)));
   }
   if constexpr (CHAIN) set_next();
   // Per-stage k offsets of A and B (uniform), behind the two LDS buffers,
@@ -798,6 +817,20 @@ __device__ __forceinline__ void split_big_tile(
     const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, int(byte_off), 0, 0);
     return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z),
                        __uint_as_float(v.w));
+  };
+  // a thread's two elements: side by side at off, or (ODD) `step` apart, each
+  // with its own bounds
+  auto load_pair = [&](__amdgpu_buffer_rsrc_t r, unsigned off, unsigned step, bool in0, bool in1) {
+    if constexpr (ODD) {
+      const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(
+          r, int(in0 ? off * unsigned(sizeof(float2)) : kOutside), 0, 0);
+      const u32x2 y = __builtin_amdgcn_raw_buffer_load_b64(
+          r, int(in1 ? (off + step) * unsigned(sizeof(float2)) : kOutside), 0, 0);
+      return make_float4(__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(y.x),
+                         __uint_as_float(y.y));
+    } else {
+      return load16(r, in0 ? off * unsigned(sizeof(float2)) : kOutside);
+    }
   };
   auto load_tile = [&](int kt, float4* ra, float4* rb, bool nx = false) {
     const int k0 = kt * kBBK;
@@ -833,29 +866,20 @@ __device__ __forceinline__ void split_big_tile(
 #pragma unroll
     for (int h = 0; h < kAH; ++h) {
       const int f = tid + NTH * h;
-      int gm, gk;
-      unsigned off;
       unsigned arow;
       if constexpr (kNextInLds)
         arow = nx ? next_slots()[h * NTH + tid] : unsigned(a_off[h]);
       else
         arow = CHAIN && nx ? a_offn[h] : unsigned(a_off[h]);
-      if constexpr (AM == 2) {
-        gm = tm0 + 2 * (f >> 3);
-        gk = k0 + (f & 7);
-        off = arow + a_kbase + unsigned(a_coff);
-      } else {
-        gm = tm0 + (f >> 2);
-        gk = k0 + 2 * (f & 3);
-        off = AM == 0 ? unsigned(gm - mo) * unsigned(K) + unsigned(gk - ko)
-                      : arow + a_kbase + unsigned(a_coff);
-      }
-      ra[h] = load16(rsrc_a, (gm < M && gk < K) ? off * unsigned(sizeof(float2)) : kOutside);
+      const int gm = tm0 + a_row(f), gk = k0 + a_k(f);
+      const unsigned off = AM == 0 ? unsigned(gm - mo) * unsigned(K) + unsigned(gk - ko)
+                                   : arow + a_kbase + unsigned(a_coff);
+      ra[h] = load_pair(rsrc_a, off, unsigned(K), gm < M && gk < K, gm + 1 < M && gk < K);
     }
 #pragma unroll
     for (int h = 0; h < kBH; ++h) {
       const int g = tid + NTH * h;
-      const int gk = k0 + (g & 7), gn = tn0 + 2 * (g >> 3);
+      const int gk = k0 + b_k(g), gn = tn0 + b_col(g);
       unsigned bcol;
       if constexpr (kNextInLds)
         bcol = nx ? next_slots()[(kAH + h) * NTH + tid] : unsigned(b_off[h]);
@@ -864,7 +888,7 @@ __device__ __forceinline__ void split_big_tile(
       const unsigned off = AM == 0 ? unsigned(gk - ko) * unsigned(N) + unsigned(gn - no)
                                    : b_kbase + unsigned(b_roff) + bcol;
       const bool in = (kBT % NTH == 0 || g < kBT) && gk < K && gn < N;
-      rb[h] = load16(rsrc_b, in ? off * unsigned(sizeof(float2)) : kOutside);
+      rb[h] = load_pair(rsrc_b, off, kBStep, in, in && gn + kBStep < N);
     }
   };
   typedef T T2 __attribute__((ext_vector_type(2)));
@@ -878,9 +902,9 @@ __device__ __forceinline__ void split_big_tile(
       T t3[4][3];
 #pragma unroll
       for (int e = 0; e < 4; ++e) split_terms<MODE>(v[e], t3[e]);
-      if constexpr (AM == 2) {
+      if constexpr (AM == 2 || ODD) {
         // (re, im) of rows row and row+1 at complex k = kk
-        const int row = 2 * (f >> 3), kk = f & 7;
+        const int row = a_row(f), kk = a_k(f);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           T2 w0 = {t3[0][t], t3[1][t]};
@@ -902,8 +926,8 @@ __device__ __forceinline__ void split_big_tile(
     for (int h = 0; h < kBH; ++h) {
       const int g = tid + NTH * h;
       if (kBT % NTH != 0 && g >= kBT) continue;
-      const int kk = g & 7, nq = g >> 3;
-      // (Br, Bi) of n, then of n+1
+      const int kk = b_k(g);
+      // (Br, Bi) of the thread's two columns
       float v[4] = {rb[h].x * sb, rb[h].y * sb, rb[h].z * sb, rb[h].w * sb};
       T t3[4][3];
 #pragma unroll
@@ -912,7 +936,7 @@ __device__ __forceinline__ void split_big_tile(
       for (int t = 0; t < NT; ++t) {
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-          const int n = 2 * nq + c;
+          const int n = b_col(g) + kBStep * c;
           const T br = t3[2 * c][t], bi = t3[2 * c + 1][t];
           T2 p0 = {br, static_cast<T>(-static_cast<float>(bi))};
           T2 p1 = {bi, br};
@@ -1087,7 +1111,7 @@ __device__ __forceinline__ void split_big_tile(
   }
 }
 
-template <int MODE, int WM, int WN, int J, int AM, int I = 2, bool WIDE = false>
+template <int MODE, int WM, int WN, int J, int AM, int I = 2, bool WIDE = false, bool ODD = false>
 __global__ __launch_bounds__(64 * WM * WN) void cgemm_split_big_kernel(
     const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C, int M,
     int N, int K, AmaxRef amax, qfx_index_map a_rows,
@@ -1098,7 +1122,7 @@ __global__ __launch_bounds__(64 * WM * WN) void cgemm_split_big_kernel(
   // products, the same on 4096^3; the tile computation is unchanged.
   const unsigned L = blockIdx.x + gridDim.x * blockIdx.y;
   const unsigned tn = L % gridDim.y, tm = L / gridDim.y;
-  split_big_tile<MODE, WM, WN, J, AM, I, WIDE>(
+  split_big_tile<MODE, WM, WN, J, AM, I, WIDE, false, ODD>(
       A, B, C, M, N, K, amax, a_rows, a_cols, b_rows, b_cols, cmax ? cmax + L : nullptr,
       int(tm) * 32 * I * WM, int(tn) * 16 * J * WN);
 }
@@ -1168,8 +1192,8 @@ __global__ __launch_bounds__(256) void amax_grouped_kernel(const GroupTile* __re
 // Persistent grouped launch: the blocks walk the tiles of all problems
 // (problems of any shape, tiles numbered problem by problem), each block
 // taking every gridDim.x-th tile.
-template <int MODE>
-__global__ __launch_bounds__(512) void cgemm_split_grouped_kernel(const GroupTile* __restrict__ probs,
+template <int MODE, int WM, int WN, int J, bool ODD>
+__global__ __launch_bounds__(64 * WM * WN) void cgemm_split_grouped_kernel(const GroupTile* __restrict__ probs,
                                                                   int count, uint64_t total) {
   const qfx_index_map none{};
   for (uint64_t t = blockIdx.x; t < total; t += gridDim.x) {
@@ -1177,8 +1201,9 @@ __global__ __launch_bounds__(512) void cgemm_split_grouped_kernel(const GroupTil
         probs[group_entry(&probs[0].first_tile, sizeof(GroupTile), count, t)];
     const uint64_t local = t - g.first_tile;
     const int tm = int(local % uint64_t(g.tiles_m)), tn = int(local / uint64_t(g.tiles_m));
-    split_big_tile<MODE, 4, 2, 4, 0>(g.A, g.B, g.C, g.M, g.N, g.K, g.amax, none, none, none, none,
-                                     nullptr, tm * 256, tn * 128);
+    split_big_tile<MODE, WM, WN, J, 0, 2, false, false, ODD>(
+        g.A, g.B, g.C, g.M, g.N, g.K, g.amax, none, none, none, none, nullptr, tm * 64 * WM,
+        tn * 16 * J * WN);
     __syncthreads();  // the next tile's prologue rewrites the LDS
   }
 }
@@ -1198,10 +1223,10 @@ size_t split_big_lds(uint64_t k) {
 }
 
 // Dynamic LDS above 64 KiB must be allowed per kernel once per process.
-template <int MODE, int WM, int WN, int J, int AM, int I = 2, bool WIDE = false>
+template <int MODE, int WM, int WN, int J, int AM, int I = 2, bool WIDE = false, bool ODD = false>
 hipError_t split_big_prepare() {
   static hipError_t e = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&cgemm_split_big_kernel<MODE, WM, WN, J, AM, I, WIDE>),
+      reinterpret_cast<const void*>(&cgemm_split_big_kernel<MODE, WM, WN, J, AM, I, WIDE, ODD>),
       hipFuncAttributeMaxDynamicSharedMemorySize,
       int(AM != 0 ? kMaxLds : split_big_smem<MODE, WM, WN, J, I>()));
   return e;
@@ -1379,6 +1404,40 @@ hipError_t launch_split_big_prec(int precision, BigLayout lay, hipStream_t strea
                                                 maps, cmax)
               : launch_split_big_mode<AM, false>(precision, lay, stream, A, B, C, m, n, k, amax,
                                                  maps, cmax);
+}
+
+// One row-major product on tiles of 64 WM x 16 J WN, one block each.
+template <int MODE, int WM, int WN, int J, bool ODD>
+hipError_t launch_split_rm(hipStream_t stream, const float2* A, const float2* B, float2* C,
+                           uint64_t m, uint64_t n, uint64_t k, AmaxRef amax) {
+  const hipError_t e = split_big_prepare<MODE, WM, WN, J, 0, 2, false, ODD>();
+  if (e != hipSuccess) return e;
+  const dim3 g{unsigned((m + 64 * WM - 1) / (64 * WM)), unsigned((n + 16 * J * WN - 1) / (16 * J * WN)),
+               1};
+  const qfx_index_map none{};
+  cgemm_split_big_kernel<MODE, WM, WN, J, 0, 2, false, ODD>
+      <<<g, 64 * WM * WN, split_big_lds<MODE, WM, WN, J, 0>(k), stream>>>(
+          A, B, C, int(m), int(n), int(k), amax, none, none, none, none, nullptr);
+  return hipGetLastError();
+}
+
+// Split products off the large tiles: odd k or n or 8-byte operands (`odd`),
+// or too few large tiles to fill the chip.  128 x 64 tiles of 4 waves, up to
+// three blocks per compute unit, or, where they take less time in all, 256 x
+// 128 tiles: a large tile does the work of four small ones in the time of
+// 2.7 of them (split FP16, per round of one block on every unit: 6145 x 515 x
+// 333 takes 48 us as 441 small and 64 as 125 large tiles, 9001 x 701 x 2001
+// 490 as 781 small and 353 as 216 large ones).  Whole-operand addressing only.
+template <int MODE>
+hipError_t launch_split_small(hipStream_t stream, const float2* A, const float2* B, float2* C,
+                              uint64_t m, uint64_t n, uint64_t k, AmaxRef amax, bool odd) {
+  auto rounds = [&](uint64_t bm, uint64_t bn) {
+    return (((m + bm - 1) / bm) * ((n + bn - 1) / bn) + device_cus() - 1) / device_cus();
+  };
+  if (odd && n >= 128 && 27 * rounds(256, 128) <= 10 * rounds(128, 64))
+    return launch_split_rm<MODE, 4, 2, 4, true>(stream, A, B, C, m, n, k, amax);
+  return odd ? launch_split_rm<MODE, 2, 2, 2, true>(stream, A, B, C, m, n, k, amax)
+             : launch_split_rm<MODE, 2, 2, 2, false>(stream, A, B, C, m, n, k, amax);
 }
 
 // Blocks (one partial maximum each) of a large-tile launch.
@@ -2175,12 +2234,12 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
   if (grid.y > 65535) return qfx_set_error(QFX_ERR_UNSUPPORTED, "qfx_cgemm_c64: n too large");
   // Large tiles (one block per CU) when there are enough of them to fill
   // the chip; float4 operand loads need even k and n and 16-byte alignment.
-  const BigLayout layout =
-      (precision != QFX_PREC_FP32 && precision != QFX_PREC_FP8 && (k % 2 == 0) && (n % 2 == 0) &&
-       big_operands_fit(m, n, k) &&
-       (reinterpret_cast<uintptr_t>(A) % 16 == 0) && (reinterpret_cast<uintptr_t>(B) % 16 == 0))
-          ? choose_big_layout(precision, m, n)
-          : kLayoutNone;
+  const bool split = precision != QFX_PREC_FP32 && precision != QFX_PREC_FP8;
+  const bool odd = k % 2 != 0 || n % 2 != 0 || reinterpret_cast<uintptr_t>(A) % 16 != 0 ||
+                   reinterpret_cast<uintptr_t>(B) % 16 != 0;
+  const BigLayout layout = split && !odd && big_operands_fit(m, n, k)
+                               ? choose_big_layout(precision, m, n)
+                               : kLayoutNone;
   AmaxRef amax{nullptr, 0, nullptr, 0};
   if (precision == QFX_PREC_SPLIT_FP16) {
     int st = launch_amax(ctx, A2, m * k, B2, k * n, &amax);
@@ -2200,6 +2259,16 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
     QFX_HIP(te);
     QFX_HIP(launch_split_big_prec<0>(precision, use, ctx->stream, A2, B2, C2, m, n, k, amax,
                                      nullptr, nullptr, wide));
+    return QFX_OK;
+  }
+  if (split && big_operands_whole(m, n, k)) {
+    auto go = [&](auto mode) {
+      return launch_split_small<decltype(mode)::value>(ctx->stream, A2, B2, C2, m, n, k, amax,
+                                                       odd);
+    };
+    QFX_HIP(precision == QFX_PREC_SPLIT_BF16X3 ? go(std::integral_constant<int, 0>{})
+            : precision == QFX_PREC_SPLIT_BF16 ? go(std::integral_constant<int, 1>{})
+                                               : go(std::integral_constant<int, 2>{}));
     return QFX_OK;
   }
   if (precision == QFX_PREC_SPLIT_FP16) {
@@ -2489,48 +2558,12 @@ static int launch_rows_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
   return QFX_OK;
 }
 
-extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
-                                     const qfx_gemm_desc* descs) {
-  QFX_CHECK_CTX(ctx);
-  QFX_NOT_CAPTURING(ctx, "qfx_cgemm_grouped_c64");
-  if (count < 0 || (count > 0 && !descs))
-    return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: invalid problem list");
-  if (precision < QFX_PREC_FP32 || precision > QFX_PREC_FP8)
-    return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: unknown precision");
-  const bool split = precision == QFX_PREC_SPLIT_FP16 || precision == QFX_PREC_SPLIT_BF16 ||
-                     precision == QFX_PREC_SPLIT_BF16X3;
-  // Problems for the large tiles go into one launch, and so do those of the
-  // row kernel (k, n <= 16, any precision: exact FP32, the kernel
-  // qfx_cgemm_c64 runs them on); the others (other precisions, odd sizes,
-  // unaligned or too large operands) run one by one exactly as
-  // qfx_cgemm_c64 would run them.
-  std::vector<int> grouped, rows;
-  for (int i = 0; i < count; ++i) {
-    const qfx_gemm_desc& d = descs[i];
-    if (d.m > 0 && d.n > 0 && d.k > 0 && d.k <= uint64_t(kSmallK) && d.n <= 16 && d.A && d.B &&
-        d.C && (d.m + 255) / 256 <= 0x7fffffffULL) {
-      rows.push_back(i);
-      continue;
-    }
-    const bool eligible = split && d.m > 0 && d.n > 0 && d.k > uint64_t(kSmallK) &&
-                          d.k % 2 == 0 && d.n % 2 == 0 && d.A && d.B && d.C &&
-                          reinterpret_cast<uintptr_t>(d.A) % 16 == 0 &&
-                          reinterpret_cast<uintptr_t>(d.B) % 16 == 0 &&
-                          big_operands_fit(d.m, d.n, d.k) && big_operands_whole(d.m, d.n, d.k) &&
-                          d.m <= 0x7fffffffULL &&
-                          d.n <= 0x7fffffffULL;
-    if (eligible) {
-      grouped.push_back(i);
-      continue;
-    }
-    const int st = qfx_cgemm_c64(ctx, precision, d.m, d.n, d.k, d.A, d.B, d.C);
-    if (st != QFX_OK) return st;
-  }
-  if (!rows.empty()) {
-    const int st = launch_rows_grouped(ctx, descs, rows);
-    if (st != QFX_OK) return st;
-  }
-  if (grouped.empty()) return QFX_OK;
+// The split products of a grouped call in one launch.
+template <bool ODD>
+static int launch_split_grouped(qfx_context* ctx, int precision, const qfx_gemm_desc* descs,
+                                const std::vector<int>& grouped) {
+  constexpr int WM = ODD ? 2 : 4, WN = 2, J = ODD ? 2 : 4;
+  constexpr uint64_t kTM = 64 * WM, kTN = 16 * J * WN;
   double flops = 0, bytes = 0;
   size_t nparts = 0;
   std::vector<std::array<int, 2>> blocks(grouped.size(), {0, 0});
@@ -2565,9 +2598,9 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
     t.M = int(d.m);
     t.N = int(d.n);
     t.K = int(d.k);
-    t.tiles_m = int((d.m + 255) / 256);
+    t.tiles_m = int((d.m + kTM - 1) / kTM);
     t.first_tile = tile;
-    tile += uint64_t(t.tiles_m) * ((d.n + 127) / 128);
+    tile += uint64_t(t.tiles_m) * ((d.n + kTN - 1) / kTN);
     const int ba = blocks[g][0], bb = blocks[g][1];
     t.first_part = off;
     t.amax = AmaxRef{part + off, ba, part + off + ba, bb};
@@ -2583,14 +2616,16 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
     QFX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
     ctx->cus = std::max(cus, 1);
   }
-  const unsigned grid = unsigned(std::min<uint64_t>(tile, uint64_t(ctx->cus)));
   auto go = [&](auto mode) -> hipError_t {
     constexpr int MODE = decltype(mode)::value;
+    constexpr int kLds = int(split_big_smem<MODE, WM, WN, J>());
     static hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&cgemm_split_grouped_kernel<MODE>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, int(split_big_smem<MODE, 4, 2, 4>()));
+        reinterpret_cast<const void*>(&cgemm_split_grouped_kernel<MODE, WM, WN, J, ODD>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (e != hipSuccess) return e;
-    cgemm_split_grouped_kernel<MODE><<<grid, 512, split_big_smem<MODE, 4, 2, 4>(), ctx->stream>>>(
+    const unsigned per_cu = unsigned(std::max<int>(1, int(kMaxLds) / kLds));
+    const unsigned grid = unsigned(std::min<uint64_t>(tile, uint64_t(ctx->cus) * per_cu));
+    cgemm_split_grouped_kernel<MODE, WM, WN, J, ODD><<<grid, 64 * WM * WN, kLds, ctx->stream>>>(
         dev, int(grouped.size()), tile);
     return hipGetLastError();
   };
@@ -2598,6 +2633,61 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
   else if (precision == QFX_PREC_SPLIT_BF16) QFX_HIP(go(std::integral_constant<int, 1>{}));
   else QFX_HIP(go(std::integral_constant<int, 2>{}));
   return QFX_OK;
+}
+
+extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
+                                     const qfx_gemm_desc* descs) {
+  QFX_CHECK_CTX(ctx);
+  QFX_NOT_CAPTURING(ctx, "qfx_cgemm_grouped_c64");
+  if (count < 0 || (count > 0 && !descs))
+    return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: invalid problem list");
+  if (precision < QFX_PREC_FP32 || precision > QFX_PREC_FP8)
+    return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: unknown precision");
+  const bool split = precision == QFX_PREC_SPLIT_FP16 || precision == QFX_PREC_SPLIT_BF16 ||
+                     precision == QFX_PREC_SPLIT_BF16X3;
+  // Problems for the large tiles go into one launch, and so do those of the
+  // row kernel (k, n <= 16, any precision: exact FP32, the kernel
+  // qfx_cgemm_c64 runs them on); the others (other precisions, odd sizes,
+  // unaligned or too large operands) run one by one exactly as
+  // qfx_cgemm_c64 would run them.
+  std::vector<int> grouped, grouped_odd, rows;
+  for (int i = 0; i < count; ++i) {
+    const qfx_gemm_desc& d = descs[i];
+    if (d.m > 0 && d.n > 0 && d.k > 0 && d.k <= uint64_t(kSmallK) && d.n <= 16 && d.A && d.B &&
+        d.C && (d.m + 255) / 256 <= 0x7fffffffULL) {
+      rows.push_back(i);
+      continue;
+    }
+    const bool fits = split && d.m > 0 && d.n > 0 && d.k > uint64_t(kSmallK) && d.A && d.B &&
+                      d.C && big_operands_fit(d.m, d.n, d.k) &&
+                      big_operands_whole(d.m, d.n, d.k) && d.m <= 0x7fffffffULL &&
+                      d.n <= 0x7fffffffULL;
+    const bool even = d.k % 2 == 0 && d.n % 2 == 0 &&
+                      reinterpret_cast<uintptr_t>(d.A) % 16 == 0 &&
+                      reinterpret_cast<uintptr_t>(d.B) % 16 == 0;
+    if (fits && even) {
+      grouped.push_back(i);
+      continue;
+    }
+    // the odd products that alone would run split on the matrix cores (the
+    // others are exact FP32 alone, and stay so)
+    if (fits && d.m >= 64 && d.n >= 16 && !smallk_splitk_fits(d.m, d.n, d.k)) {
+      grouped_odd.push_back(i);
+      continue;
+    }
+    const int st = qfx_cgemm_c64(ctx, precision, d.m, d.n, d.k, d.A, d.B, d.C);
+    if (st != QFX_OK) return st;
+  }
+  if (!rows.empty()) {
+    const int st = launch_rows_grouped(ctx, descs, rows);
+    if (st != QFX_OK) return st;
+  }
+  if (!grouped.empty()) {
+    const int st = launch_split_grouped<false>(ctx, precision, descs, grouped);
+    if (st != QFX_OK) return st;
+  }
+  return grouped_odd.empty() ? QFX_OK
+                             : launch_split_grouped<true>(ctx, precision, descs, grouped_odd);
 }
 
 // ------------------------------------------------------------ autotuner

@@ -25,7 +25,7 @@ static_assert(kParams == QFX_MLP_PARAMS, "parameter layout");
 // One training step's forward and backward pass is two launches.  As one
 // launch per GEMM, conversion, ReLU gradient and column sum it was about 20
 // of them, each a few us of launch and drain for well under 1 us of work (512
-// rows: 218 us a step).
+// rows: 218 us a step, 17 us now; 4096 rows: 1097 and 27).
 //
 // mlp_rows_kernel takes 32 rows of the batch at a time through the whole
 // network: forward, and for training the error and the two hidden layers'

@@ -124,6 +124,44 @@ def test_grouped_row_kernel_products_same_bits_as_alone(ctx, prec):
     free(probs)
 
 
+# Odd k or n, 8-byte operands, tile edges and remainders of the 128 x 64 and
+# 256 x 128 tiles.  Per element the split kernels sum the same products in the
+# same order whatever the tile, so alone, grouped, and padded to even sizes
+# with zeros (which add nothing) they give the same bits.
+ODD_SHAPES = [(64, 17, 17), (129, 65, 33), (127, 63, 4097), (6145, 515, 333), (20001, 257, 40),
+              (300, 64, 1001), (1025, 129, 18)]
+
+
+@pytest.mark.parametrize("prec", [capi.SPLIT_FP16, capi.SPLIT_BF16, capi.SPLIT_BF16X3])
+@pytest.mark.parametrize("m,n,k", ODD_SHAPES)
+def test_odd_split_products_same_bits_alone_grouped_and_padded(ctx, m, n, k, prec):
+    rng = np.random.default_rng(m + n + k)
+    a, b = rand_c(rng, (m, k)), rand_c(rng, (k, n))
+    n2, k2 = n + n % 2, k + k % 2
+    ap, bp = np.zeros((m, k2), np.complex64), np.zeros((k2, n2), np.complex64)
+    ap[:, :k], bp[:k, :n] = a, b
+    A, B, Ap, Bp = (ctx.upload(x) for x in (a, b, ap, bp))
+    C, G, P = ctx.alloc(m * n * 8), ctx.alloc(m * n * 8), ctx.alloc(m * n2 * 8)
+    ctx.cgemm(prec, m, n, k, A, B, C)
+    ctx.cgemm_grouped(prec, [(m, n, k, A, B, G), (m, n2, k2, Ap, Bp, P)])
+    got = ctx.download(C, np.complex64, (m, n))
+    assert np.array_equal(got, ctx.download(G, np.complex64, (m, n)))
+    assert np.array_equal(got, ctx.download(P, np.complex64, (m, n2))[:, :n])
+    ref = a.astype(np.complex128) @ b.astype(np.complex128)
+    assert np.linalg.norm(got - ref) / np.linalg.norm(ref) <= TOL[prec]
+    # the same operands at 8-byte addresses
+    A8, B8 = ctx.upload(np.concatenate([[0], a.ravel()]).astype(np.complex64)), ctx.upload(
+        np.concatenate([[0], b.ravel()]).astype(np.complex64))
+
+    class At8:
+        def __init__(self, buf):
+            self.ptr = buf.ptr + 8
+    ctx.cgemm(prec, m, n, k, At8(A8), At8(B8), G)
+    assert np.array_equal(got, ctx.download(G, np.complex64, (m, n)))
+    for buf in (A, B, Ap, Bp, C, G, P, A8, B8):
+        buf.free()
+
+
 # Products with at least two 256 x 128 (or 128 x 256, 512 x 32) tiles per
 # compute unit and an even number of 8-deep k-stages run as chains of tiles
 # (each block computes several tiles, loading the next tile's first stages
