@@ -54,6 +54,33 @@ def test_reorder_bit_exact(ctx, dims, perm):
     dst.free()
 
 
+# Dimensions that are no powers of two (boxes of contiguous runs): both
+# innermost axes in one box, the same innermost axis on both sides, axes cut
+# into blocks with and without remainder on one and both sides, boxes larger
+# than the tensor, many small axes, and a rank-2 transpose of long odd axes.
+BOX_CASES = [((3, 2), (1, 0)), ((5, 7, 3), (2, 1, 0)), ((16, 11, 16, 3, 16, 16, 5), (4, 1, 6, 0, 3, 2, 5)),
+             ((1009, 2003), (1, 0)), ((33, 4096), (1, 0)), ((4100, 3), (1, 0)), ((3, 100000), (1, 0)),
+             ((7, 301, 3), (1, 0, 2)), ((5, 3, 1001), (1, 0, 2)), ((3, 5, 67, 64), (1, 2, 0, 3)),
+             ((2,) * 9 + (3,) * 6, (14, 3, 8, 0, 11, 5, 13, 1, 9, 2, 12, 7, 4, 10, 6)),
+             ((100, 70, 90), (2, 0, 1)), ((65, 1, 65, 65), (3, 2, 1, 0)), ((2, 3, 513, 129), (3, 0, 2, 1)),
+             ((11, 16, 16, 16, 16, 7), (5, 0, 1, 2, 3, 4)), ((97, 101, 103), (2, 1, 0)),
+             ((3, 2) * 8, tuple(range(1, 16, 2)) + tuple(range(0, 16, 2)))]
+
+
+@pytest.mark.parametrize("dims,perm", BOX_CASES)
+def test_reorder_boxes_bit_exact(ctx, dims, perm):
+    rng = np.random.default_rng(len(dims) + sum(dims))
+    a = rand_c64(rng, dims)
+    src, dst = ctx.upload(a), ctx.alloc(a.nbytes)
+    ctx.zero(dst, a.nbytes)
+    ctx.reorder(src, dst, dims, perm)
+    want = np.ascontiguousarray(a.transpose(perm))
+    got = ctx.download(dst, np.complex64, want.shape)
+    assert np.array_equal(got.view(np.uint64), want.view(np.uint64))
+    src.free()
+    dst.free()
+
+
 def test_reorder_random_binary_permutations(ctx):
     rng = np.random.default_rng(7)
     for nbits in (11, 16, 20, 22):
