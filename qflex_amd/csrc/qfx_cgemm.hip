@@ -58,115 +58,6 @@ constexpr int kBN = 64;   // complex cols per block
 constexpr int kBK = 16;   // complex k per stage
 constexpr int kAStride = 2 * kBK + 1;  // floats per LDS row of the A tile
 
-__global__ __launch_bounds__(256) void cgemm_f32_mfma_kernel(const float2* __restrict__ A,
-                                                             const float2* __restrict__ B,
-                                                             float2* __restrict__ C, int M,
-                                                             int N, int K) {
-  __shared__ float As[2][kBM * kAStride];
-  __shared__ __align__(16) float2 Bs[2][kBK * kBN];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 1;  // wave row (0..1): 64 rows each
-  const int wn = wave & 1;   // wave col (0..1): 32 complex cols each
-  const int m0 = blockIdx.x * kBM;
-  const int n0 = blockIdx.y * kBN;
-
-  // Global -> register staging assignment.
-  // A: 128 rows x 16 k = 2048 complex; thread t loads rows t/16 + 16*h,
-  //    k = t%16 (h = 0..7): 16 consecutive threads read 128 B of one row.
-  // B: 16 k x 64 n = 1024 complex; thread t loads k = t/64 + 4*h, n = t%64.
-  float2 ra[8], rb[4];
-  auto load_tile = [&](int kt) {
-    const int k0 = kt * kBK;
-#pragma unroll
-    for (int h = 0; h < 8; ++h) {
-      int r = (tid >> 4) + 16 * h;
-      int kk = tid & 15;
-      int gm = m0 + r, gk = k0 + kk;
-      ra[h] = (gm < M && gk < K) ? A[uint64_t(gm) * K + gk] : make_float2(0.f, 0.f);
-    }
-#pragma unroll
-    for (int h = 0; h < 4; ++h) {
-      int kk = (tid >> 6) + 4 * h;
-      int nn = tid & 63;
-      int gk = k0 + kk, gn = n0 + nn;
-      rb[h] = (gk < K && gn < N) ? B[uint64_t(gk) * N + gn] : make_float2(0.f, 0.f);
-    }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int h = 0; h < 8; ++h) {
-      int r = (tid >> 4) + 16 * h;
-      int kk = tid & 15;
-      As[buf][r * kAStride + 2 * kk] = ra[h].x;
-      As[buf][r * kAStride + 2 * kk + 1] = ra[h].y;
-    }
-#pragma unroll
-    for (int h = 0; h < 4; ++h) {
-      int kk = (tid >> 6) + 4 * h;
-      int nn = tid & 63;
-      Bs[buf][kk * kBN + nn] = rb[h];
-    }
-  };
-
-  // Per-lane operand selectors.
-  const int half = lane >> 5;      // MFMA k index (0: real part row, 1: imag)
-  const int col = lane & 31;       // real column within a 32-wide MFMA tile
-  const int part = col & 1;        // 0: Cr column, 1: Ci column
-  const bool take_x = (half == part);
-  const float sgn = half ? -1.f : 1.f;
-
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  const int nkt = (K + kBK - 1) / kBK;
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
-  for (int kt = 0; kt < nkt; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < nkt) load_tile(kt + 1);
-    const float* as = As[buf];
-    const float2* bs = Bs[buf];
-#pragma unroll 4
-    for (int kk = 0; kk < kBK; ++kk) {
-      float a0 = as[(wm * 64 + col) * kAStride + 2 * kk + half];
-      float a1 = as[(wm * 64 + 32 + col) * kAStride + 2 * kk + half];
-      float2 b0v = bs[kk * kBN + wn * 32 + (col >> 1)];
-      float2 b1v = bs[kk * kBN + wn * 32 + 16 + (col >> 1)];
-      float b0 = take_x ? b0v.x : sgn * b0v.y;
-      float b1 = take_x ? b1v.x : sgn * b1v.y;
-      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc[1][1], 0, 0, 0);
-    }
-    if (kt + 1 < nkt) store_tile(buf ^ 1);
-    __syncthreads();
-  }
-
-  // Output: register r of lane l holds row 8*(r/4) + 4*(l/32) + r%4,
-  // real column l%32 of its 32x32 tile.
-  float* Cf = reinterpret_cast<float*>(C);
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        int row = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-        int cn = n0 + wn * 32 + j * 16 + (col >> 1);
-        if (row < M && cn < N) Cf[(uint64_t(row) * N + cn) * 2 + part] = acc[i][j][r];
-      }
-}
-
 // ------------------------------------------------------------ split-BF16 MFMA
 // Same block tile as the FP32 kernel.  Operands are split once, while they
 // are staged into LDS, into NT BF16 planes (hi, mid[, lo]):
@@ -1541,76 +1432,12 @@ __global__ __launch_bounds__(256) void sum_partials_narrow_kernel(const float2* 
   if (threadIdx.x == 0) y[c] = red[0];
 }
 
-// Stage 2: y[c] = sum_s part[s][c]; 64 columns x 4 split groups per block,
-// grid-stride over column tiles.
-__global__ __launch_bounds__(256) void sum_partials_kernel(const float2* __restrict__ part,
-                                                           float2* __restrict__ y,
-                                                           uint64_t nsplit, uint64_t K) {
-  __shared__ float2 red[4][64];
-  const int cl = threadIdx.x & 63;
-  const int sg = threadIdx.x >> 6;
-  for (uint64_t c0 = uint64_t(blockIdx.x) * 64; c0 < K; c0 += uint64_t(gridDim.x) * 64) {
-    const uint64_t c = c0 + cl;
-    float2 acc = make_float2(0.f, 0.f);
-    if (c < K)
-      for (uint64_t s = sg; s < nsplit; s += 4) {
-        float2 v = part[s * K + c];
-        acc.x += v.x;
-        acc.y += v.y;
-      }
-    red[sg][cl] = acc;
-    __syncthreads();
-    if (sg == 0 && c < K) {
-      float2 t = red[0][cl];
-#pragma unroll
-      for (int g = 1; g < 4; ++g) {
-        t.x += red[g][cl].x;
-        t.y += red[g][cl].y;
-      }
-      y[c] = t;
-    }
-    __syncthreads();
-  }
-}
-
-// Few outputs, long k: C[m x n] with m*n <= 4096.  Block (x = k chunk,
-// y = tile of 64 outputs): 4 groups of 64 lanes split the chunk, fixed
-// order, LDS tree; part[chunk][o] is then summed over chunks by
-// sum_partials_kernel.
-__global__ __launch_bounds__(256) void cgemm_splitk_partial_kernel(
-    const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ part,
-    uint64_t M, uint64_t N, uint64_t K, uint64_t chunk) {
-  __shared__ float2 red[4][64];
-  const int ol = threadIdx.x & 63;
-  const int kg = threadIdx.x >> 6;
-  const uint64_t o = uint64_t(blockIdx.y) * 64 + ol;
-  const uint64_t k0 = uint64_t(blockIdx.x) * chunk;
-  const uint64_t k1 = k0 + chunk < K ? k0 + chunk : K;
-  float2 acc = make_float2(0.f, 0.f);
-  if (o < M * N) {
-    const uint64_t m = o / N, n = o - m * N;
-    const float2* a = A + m * K;
-    for (uint64_t k = k0 + kg; k < k1; k += 4) acc = cfma(a[k], B[k * N + n], acc);
-  }
-  red[kg][ol] = acc;
-  __syncthreads();
-  if (kg == 0 && o < M * N) {
-    float2 t = red[0][ol];
-#pragma unroll
-    for (int g = 1; g < 4; ++g) {
-      t.x += red[g][ol].x;
-      t.y += red[g][ol].y;
-    }
-    part[uint64_t(blockIdx.x) * M * N + o] = t;
-  }
-}
-
 // Split-K for at most 8 x 8 outputs and long k (the final merges of a
 // contraction, e.g. 8 x 8 x 2^20).  Each thread keeps all 64 outputs in
 // registers over its k values (A rows and the B row of one k are
 // contiguous loads across lanes), then a butterfly reduce-scatter leaves
 // output o = i*8 + j on lane o of each wave; the 4 waves are summed in LDS
-// in fixed order and sum_partials_kernel adds the blocks' partials in
+// in fixed order and sum_partials_narrow_kernel adds the blocks' partials in
 // fixed order, so results are deterministic.
 constexpr int kTinyChunk = 2048;  // k values per block (a power of two >= 256)
 __global__ __launch_bounds__(256) void cgemm_tiny_mn_partial_kernel(
@@ -1671,9 +1498,6 @@ constexpr int kSmallK = 16;
 // MAPPED: operands through digit maps (offset tables in LDS); A is read
 // along m when a_mfast (a_rows digit 0 at stride 1), else along k; B along
 // n when b_nfast, else along k.
-// Split-K use (blockIdx.z = chunk > 0 or part != nullptr): the block covers
-// k in [16*z, 16*z + K) of a common dimension of length ldk and writes its
-// partial tile to part[z][m][n] (summed afterwards in fixed order).
 // Max of v over a 256-thread block, written by thread 0 (the partial maxima
 // a split-FP16 consumer of the output reduces instead of a max-abs pass).
 __device__ __forceinline__ void store_block_max(float v, float* slot) {
@@ -1689,9 +1513,7 @@ template <int BN, bool MAPPED>
 __global__ __launch_bounds__(256) void cgemm_smallk_kernel(
     const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C,
     uint64_t M, int N, int K, qfx_index_map a_rows, qfx_index_map a_cols, qfx_index_map b_rows,
-    qfx_index_map b_cols, bool a_mfast, bool b_nfast, uint64_t ldk, float2* __restrict__ part,
-    float* __restrict__ cmax) {
-  const uint64_t kbeg = uint64_t(blockIdx.z) * kSmallK;
+    qfx_index_map b_cols, bool a_mfast, bool b_nfast, float* __restrict__ cmax) {
   constexpr int TX = BN / 4;        // column groups
   constexpr int BM = 4 * 256 / TX;  // rows per block
   __shared__ float2 As[BM][kSmallK + 1];
@@ -1705,8 +1527,8 @@ __global__ __launch_bounds__(256) void cgemm_smallk_kernel(
     for (int i = threadIdx.x; i < BM; i += 256) arow[i] = map_offset(a_rows, m0 + i);
     for (int i = threadIdx.x; i < BN; i += 256) bcol[i] = map_offset(b_cols, uint64_t(n0 + i));
     if (threadIdx.x < K) {
-      acol[threadIdx.x] = map_offset(a_cols, kbeg + threadIdx.x);
-      brow[threadIdx.x] = map_offset(b_rows, kbeg + threadIdx.x);
+      acol[threadIdx.x] = map_offset(a_cols, threadIdx.x);
+      brow[threadIdx.x] = map_offset(b_rows, threadIdx.x);
     }
     __syncthreads();
   }
@@ -1721,7 +1543,7 @@ __global__ __launch_bounds__(256) void cgemm_smallk_kernel(
       c = e - r * K;
     }
     float2 v = make_float2(0.f, 0.f);
-    if (m0 + r < M) v = MAPPED ? A[arow[r] + acol[c]] : A[(m0 + r) * ldk + kbeg + c];
+    if (m0 + r < M) v = MAPPED ? A[arow[r] + acol[c]] : A[(m0 + r) * K + c];
     As[r][c] = v;
   }
   for (int e = threadIdx.x; e < K * BN; e += 256) {
@@ -1734,7 +1556,7 @@ __global__ __launch_bounds__(256) void cgemm_smallk_kernel(
       c = e - r * BN;
     }
     float2 v = make_float2(0.f, 0.f);
-    if (n0 + c < N) v = MAPPED ? B[brow[r] + bcol[c]] : B[(kbeg + r) * N + n0 + c];
+    if (n0 + c < N) v = MAPPED ? B[brow[r] + bcol[c]] : B[uint64_t(r) * N + n0 + c];
     Bs[r][c] = v;
   }
   __syncthreads();
@@ -1754,7 +1576,6 @@ __global__ __launch_bounds__(256) void cgemm_smallk_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = cfma(a[i], b[j], acc[i][j]);
   }
-  float2* out = part ? part + uint64_t(blockIdx.z) * M * N : C;
   float cm = 0.f;  // max |re|, |im| of the values this thread stores
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -1764,7 +1585,7 @@ __global__ __launch_bounds__(256) void cgemm_smallk_kernel(
     for (int j = 0; j < 4; ++j) {
       const int c = n0 + tx + TX * j;
       if (c < N) {
-        out[r * N + c] = acc[i][j];
+        C[r * N + c] = acc[i][j];
         cm = fmaxf(cm, fmaxf(fabsf(acc[i][j].x), fabsf(acc[i][j].y)));
       }
     }
@@ -2039,50 +1860,36 @@ unsigned cap_grid(uint64_t g) { return unsigned(std::max<uint64_t>(1, std::min<u
 
 }  // namespace
 
-// Small-output GEMMs with a longer common dimension (m*n <= 2^16,
-// 16 < k <= 4096, k a multiple of 16): split-K over chunks of 16 with the
-// vector-ALU tile kernel, partial tiles summed in fixed chunk order.
-// Enough blocks to fill the chip where one MFMA tile per output block
-// would leave most CUs idle.
-static bool smallk_splitk_fits(uint64_t m, uint64_t n, uint64_t k) {
-  return m * n <= (uint64_t(1) << 16) && k > uint64_t(kSmallK) && k <= 4096 &&
+static bool split_precision(int precision) {
+  return precision == QFX_PREC_SPLIT_FP16 || precision == QFX_PREC_SPLIT_BF16 ||
+         precision == QFX_PREC_SPLIT_BF16X3;
+}
+
+// At most 2^16 outputs over 16 < k <= 4096, k a multiple of 16.
+static bool small_output(uint64_t m, uint64_t n, uint64_t k) {
+  return m > 8 && n > 1 && m * n <= (uint64_t(1) << 16) && k > uint64_t(kSmallK) && k <= 4096 &&
          k % kSmallK == 0;
 }
 
-static int launch_smallk_splitk(qfx_context* ctx, const float2* A, const float2* B, float2* C,
-                                uint64_t m, uint64_t n, uint64_t k, bool mapped,
-                                const qfx_index_map* maps, bool a_mfast, bool b_nfast) {
-  const uint64_t nchunk = k / kSmallK;
-  void* ws = nullptr;
-  int st = qfx_workspace(ctx, nchunk * m * n * sizeof(float2), &ws);
-  if (st != QFX_OK) return st;
-  float2* part = static_cast<float2*>(ws);
-  const qfx_index_map none{};
-  const qfx_index_map& ar = mapped ? maps[0] : none;
-  const qfx_index_map& ac = mapped ? maps[1] : none;
-  const qfx_index_map& br = mapped ? maps[2] : none;
-  const qfx_index_map& bc = mapped ? maps[3] : none;
-  if (n <= 16) {
-    dim3 g{unsigned((m + 255) / 256), unsigned((n + 15) / 16), unsigned(nchunk)};
-    if (mapped)
-      cgemm_smallk_kernel<16, true><<<g, 256, 0, ctx->stream>>>(
-          A, B, C, m, int(n), kSmallK, ar, ac, br, bc, a_mfast, b_nfast, k, part, nullptr);
-    else
-      cgemm_smallk_kernel<16, false><<<g, 256, 0, ctx->stream>>>(
-          A, B, C, m, int(n), kSmallK, ar, ac, br, bc, false, true, k, part, nullptr);
-  } else {
-    dim3 g{unsigned((m + 63) / 64), unsigned((n + 63) / 64), unsigned(nchunk)};
-    if (mapped)
-      cgemm_smallk_kernel<64, true><<<g, 256, 0, ctx->stream>>>(
-          A, B, C, m, int(n), kSmallK, ar, ac, br, bc, a_mfast, b_nfast, k, part, nullptr);
-    else
-      cgemm_smallk_kernel<64, false><<<g, 256, 0, ctx->stream>>>(
-          A, B, C, m, int(n), kSmallK, ar, ac, br, bc, false, true, k, part, nullptr);
-  }
-  sum_partials_kernel<<<cap_grid((m * n + 63) / 64), 256, 0, ctx->stream>>>(part, C, nchunk,
-                                                                           m * n);
-  QFX_HIP(hipGetLastError());
-  return QFX_OK;
+// Products that run on the FP32 matrix-core kernel: all of FP32, the shapes
+// the split tiles don't take, and (`even`: sizes and addresses the split
+// kernels read in 16-byte pieces) those with too few large tiles whose
+// estimated time there is the shorter one.  The split kernels' 128 x 64 tile
+// takes 0.062 us per k and round of one block per CU (BF16x3: 0.088), and 3 us;
+// split FP16 also 4 us and a pass for the maxima; FP32 1.2 times the estimate
+// and 3 us.  Measured, split FP16 against FP32: 300^3 26.8 and 8.7 us, 1024 x
+// 1024 x 256 36.3 and 35.1, 1000^3 69 and 98; BF16x3: 700 x 700 x 2000 177 and
+// 121, 20000 x 100 x 100 21.5 and 29.8.  FP32 is the more exact one.
+static bool f32_route(int precision, uint64_t m, uint64_t n, uint64_t k, bool even) {
+  if (precision == QFX_PREC_FP32_EXACT || !qfx_f32_fits(m, n, k)) return false;
+  if (!split_precision(precision) || m < 64 || n < 16 || small_output(m, n, k)) return true;
+  if (!even || choose_big_layout(precision, m, n) != kLayoutNone) return false;
+  const uint64_t rounds = ((m + 127) / 128 * ((n + 63) / 64) + device_cus() - 1) / device_cus();
+  const bool fp16 = precision == QFX_PREC_SPLIT_FP16;
+  const double split =
+      (precision == QFX_PREC_SPLIT_BF16X3 ? 0.088 : 0.062) * double(k) * double(rounds) +
+      (fp16 ? 7 + 8.0 / 6e6 * (double(m) * k + double(k) * n) : 3);
+  return 1.2 * qfx_f32_time(m, n, k) + 3 < split;
 }
 
 // Operand scales of the split-FP16 form: partial maxima of |A| and |B| in
@@ -2162,20 +1969,14 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
     } else if (n <= 16) {
       dim3 g{unsigned((m + 255) / 256), unsigned((n + 15) / 16), 1};
       cgemm_smallk_kernel<16, false><<<g, 256, 0, ctx->stream>>>(A2, B2, C2, m, int(n), int(k),
-                                                                 {}, {}, {}, {}, false, true, k,
-                                                                 nullptr, nullptr);
+                                                                 {}, {}, {}, {}, false, true, nullptr);
     } else {
       dim3 g{unsigned((m + 63) / 64), unsigned((n + 63) / 64), 1};
       cgemm_smallk_kernel<64, false><<<g, 256, 0, ctx->stream>>>(A2, B2, C2, m, int(n), int(k),
-                                                                 {}, {}, {}, {}, false, true, k,
-                                                                 nullptr, nullptr);
+                                                                 {}, {}, {}, {}, false, true, nullptr);
     }
     QFX_HIP(hipGetLastError());
     return QFX_OK;
-  }
-  if (precision != QFX_PREC_FP32_EXACT && m > 8 && n > 1 && smallk_splitk_fits(m, n, k)) {
-    QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
-    return launch_smallk_splitk(ctx, A2, B2, C2, m, n, k, false, nullptr, false, true);
   }
   if (precision != QFX_PREC_FP32_EXACT && m <= 8 && n <= 8 && k >= 1024) {
     QfxLaunchScope scope(ctx, QFX_K_GEMV, bytes, flops);
@@ -2194,35 +1995,20 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
     QfxLaunchScope scope(ctx, QFX_K_CGEMM, bytes, flops);
     return qfx_cgemm_fp8(ctx, A2, B2, C2, m, n, k, nullptr);
   }
-  const bool big = m >= 64 && n >= 16 && k >= 8 && m <= 0x7fffffffULL &&
-                   n <= 0x7fffffffULL && k <= 0x7fffffffULL;
-  if (precision == QFX_PREC_FP32_EXACT || !big) {
-    if (n == 1 && precision != QFX_PREC_FP32_EXACT) {
-      QfxLaunchScope scope(ctx, QFX_K_GEMV, bytes, flops);
-      return qfx_launch_gemv_n(ctx, m, k, A2, B2, C2);
-    }
-    if (m == 1 && precision != QFX_PREC_FP32_EXACT) {
-      QfxLaunchScope scope(ctx, QFX_K_GEMV, bytes, flops);
-      // y[n] = sum_k a[k] B[k][n]: transposed GEMV of B (k x n) with x = A.
-      return qfx_launch_gemv_t(ctx, k, n, B2, A2, C2);
-    }
-    if (precision != QFX_PREC_FP32_EXACT && m * n <= 4096 && k >= 1024) {
-      QfxLaunchScope scope(ctx, QFX_K_GEMV, bytes, flops);
-      const uint64_t outs = m * n;
-      uint64_t nchunk = std::max<uint64_t>(1, std::min<uint64_t>(2048 / ((outs + 63) / 64), k / 256));
-      const uint64_t chunk = (k + nchunk - 1) / nchunk;
-      nchunk = (k + chunk - 1) / chunk;
-      void* ws = nullptr;
-      int st = qfx_workspace(ctx, nchunk * outs * sizeof(float2), &ws);
-      if (st != QFX_OK) return st;
-      float2* part = static_cast<float2*>(ws);
-      dim3 g{unsigned(nchunk), unsigned((outs + 63) / 64), 1};
-      cgemm_splitk_partial_kernel<<<g, 256, 0, ctx->stream>>>(A2, B2, part, m, n, k, chunk);
-      sum_partials_kernel<<<cap_grid((outs + 63) / 64), 256, 0, ctx->stream>>>(part, C2, nchunk,
-                                                                            outs);
-      QFX_HIP(hipGetLastError());
-      return QFX_OK;
-    }
+  if (precision != QFX_PREC_FP32_EXACT && (n == 1 || m == 1)) {
+    QfxLaunchScope scope(ctx, QFX_K_GEMV, bytes, flops);
+    // m == 1: y[n] = sum_k a[k] B[k][n], the transposed GEMV of B with x = A
+    return n == 1 ? qfx_launch_gemv_n(ctx, m, k, A2, B2, C2)
+                  : qfx_launch_gemv_t(ctx, k, n, B2, A2, C2);
+  }
+  const bool odd = k % 2 != 0 || n % 2 != 0 || reinterpret_cast<uintptr_t>(A) % 16 != 0 ||
+                   reinterpret_cast<uintptr_t>(B) % 16 != 0;
+  if (f32_route(precision, m, n, k, !odd)) {
+    QfxLaunchScope scope(ctx, QFX_K_CGEMM, bytes, flops);
+    return qfx_launch_f32(ctx, A2, B2, C2, m, n, k, nullptr, false, false, small_output(m, n, k));
+  }
+  if (precision == QFX_PREC_FP32_EXACT || m > 0x7fffffffULL || n > 0x7fffffffULL ||
+      k > 0x7fffffffULL || !split_precision(precision) || m < 64 || n < 16) {
     QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
     cgemm_scalar_kernel<<<cap_grid((m * n + 255) / 256), 256, 0, ctx->stream>>>(A2, B2, C2, m, n,
                                                                                k);
@@ -2234,10 +2020,7 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
   if (grid.y > 65535) return qfx_set_error(QFX_ERR_UNSUPPORTED, "qfx_cgemm_c64: n too large");
   // Large tiles (one block per CU) when there are enough of them to fill
   // the chip; float4 operand loads need even k and n and 16-byte alignment.
-  const bool split = precision != QFX_PREC_FP32 && precision != QFX_PREC_FP8;
-  const bool odd = k % 2 != 0 || n % 2 != 0 || reinterpret_cast<uintptr_t>(A) % 16 != 0 ||
-                   reinterpret_cast<uintptr_t>(B) % 16 != 0;
-  const BigLayout layout = split && !odd && big_operands_fit(m, n, k)
+  const BigLayout layout = !odd && big_operands_fit(m, n, k)
                                ? choose_big_layout(precision, m, n)
                                : kLayoutNone;
   AmaxRef amax{nullptr, 0, nullptr, 0};
@@ -2261,7 +2044,7 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
                                      nullptr, nullptr, wide));
     return QFX_OK;
   }
-  if (split && big_operands_whole(m, n, k)) {
+  if (big_operands_whole(m, n, k)) {
     auto go = [&](auto mode) {
       return launch_split_small<decltype(mode)::value>(ctx->stream, A2, B2, C2, m, n, k, amax,
                                                        odd);
@@ -2277,10 +2060,7 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
     QFX_HIP(hipGetLastError());
     return QFX_OK;
   }
-  // FP8 below its tile sizes runs the FP32 MFMA kernel.
-  if (precision == QFX_PREC_FP32 || precision == QFX_PREC_FP8)
-    cgemm_f32_mfma_kernel<<<grid, 256, 0, ctx->stream>>>(A2, B2, C2, int(m), int(n), int(k));
-  else if (precision == QFX_PREC_SPLIT_BF16)
+  if (precision == QFX_PREC_SPLIT_BF16)
     cgemm_bf16_mfma_kernel<3><<<grid, 256, 0, ctx->stream>>>(A2, B2, C2, int(m), int(n), int(k));
   else
     cgemm_bf16_mfma_kernel<6><<<grid, 256, 0, ctx->stream>>>(A2, B2, C2, int(m), int(n), int(k));
@@ -2423,23 +2203,16 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
     } else if (n <= 16) {
       dim3 g{unsigned((m + 255) / 256), unsigned((n + 15) / 16), 1};
       cgemm_smallk_kernel<16, true><<<g, 256, 0, ctx->stream>>>(
-          A2, B2, C2, m, int(n), int(k), *a_rows, *a_cols, *b_rows, *b_cols, a_mfast, b_nfast, k,
-          nullptr, cmax_for(uint64_t(g.x) * g.y));
+          A2, B2, C2, m, int(n), int(k), *a_rows, *a_cols, *b_rows, *b_cols, a_mfast, b_nfast,
+          cmax_for(uint64_t(g.x) * g.y));
     } else {
       dim3 g{unsigned((m + 63) / 64), unsigned((n + 63) / 64), 1};
       cgemm_smallk_kernel<64, true><<<g, 256, 0, ctx->stream>>>(
-          A2, B2, C2, m, int(n), int(k), *a_rows, *a_cols, *b_rows, *b_cols, a_mfast, b_nfast, k,
-          nullptr, cmax_for(uint64_t(g.x) * g.y));
+          A2, B2, C2, m, int(n), int(k), *a_rows, *a_cols, *b_rows, *b_cols, a_mfast, b_nfast,
+          cmax_for(uint64_t(g.x) * g.y));
     }
     QFX_HIP(hipGetLastError());
     return QFX_OK;
-  }
-  if (precision != QFX_PREC_FP32_EXACT && m > 8 && n > 1 && smallk_splitk_fits(m, n, k)) {
-    QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
-    const qfx_index_map maps[4] = {*a_rows, *a_cols, *b_rows, *b_cols};
-    const bool a_mfast = contiguous(*a_rows, 1) && !contiguous(*a_cols, 3);
-    const bool b_nfast = contiguous(*b_cols, 1) || !contiguous(*b_rows, 1);
-    return launch_smallk_splitk(ctx, A2, B2, C2, m, n, k, true, maps, a_mfast, b_nfast);
   }
   if (precision != QFX_PREC_FP32_EXACT && m <= 8 && n <= 8 && k >= 1024) {
     // Consecutive k go to consecutive lanes: B must be near-contiguous along
@@ -2467,10 +2240,15 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
     const qfx_index_map maps[4] = {*a_rows, *a_cols, *b_rows, *b_cols};
     return qfx_cgemm_fp8(ctx, A2, B2, C2, m, n, k, maps);
   }
-  const bool split = precision == QFX_PREC_SPLIT_FP16 || precision == QFX_PREC_SPLIT_BF16 ||
-                     precision == QFX_PREC_SPLIT_BF16X3;
+  if (precision != QFX_PREC_FP32_EXACT && small_output(m, n, k)) {
+    QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
+    const qfx_index_map maps[4] = {*a_rows, *a_cols, *b_rows, *b_cols};
+    return qfx_launch_f32(ctx, A2, B2, C2, m, n, k, maps,
+                          contiguous(*a_rows, 1) && !contiguous(*a_cols, 3),
+                          contiguous(*b_rows, 1) && !contiguous(*b_cols, 1), true);
+  }
   const BigLayout layout =
-      (split && big_mapped_spans_fit(*a_rows, *a_cols, *b_rows, *b_cols, m, n, k) && k >= 8 &&
+      (split_precision(precision) && big_mapped_spans_fit(*a_rows, *a_cols, *b_rows, *b_cols, m, n, k) && k >= 8 &&
        reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0)
           ? choose_big_layout(precision, m, n)
           : kLayoutNone;
@@ -2643,8 +2421,7 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
     return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: invalid problem list");
   if (precision < QFX_PREC_FP32 || precision > QFX_PREC_FP8)
     return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: unknown precision");
-  const bool split = precision == QFX_PREC_SPLIT_FP16 || precision == QFX_PREC_SPLIT_BF16 ||
-                     precision == QFX_PREC_SPLIT_BF16X3;
+  const bool split = split_precision(precision);
   // Problems for the large tiles go into one launch, and so do those of the
   // row kernel (k, n <= 16, any precision: exact FP32, the kernel
   // qfx_cgemm_c64 runs them on); the others (other precisions, odd sizes,
@@ -2671,7 +2448,7 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
     }
     // the odd products that alone would run split on the matrix cores (the
     // others are exact FP32 alone, and stay so)
-    if (fits && d.m >= 64 && d.n >= 16 && !smallk_splitk_fits(d.m, d.n, d.k)) {
+    if (fits && !f32_route(precision, d.m, d.n, d.k, false)) {
       grouped_odd.push_back(i);
       continue;
     }

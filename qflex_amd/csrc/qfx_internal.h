@@ -162,6 +162,17 @@ int qfx_launch_gemv_n(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
 int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A, const float2* x,
                       float2* y);
 
+// FP32 MFMA products of qfx_f32.hip, any m, n, k that fit (pointers checked by
+// the caller); maps = {a_rows, a_cols, b_rows, b_cols} or null for row-major,
+// a_mfast / b_kfast the operands' contiguous direction.  Products of few
+// outputs are split over k through the workspace; where a sequence being
+// recorded has reserved too little, needs_splits refuses them.
+bool qfx_f32_fits(uint64_t m, uint64_t n, uint64_t k);
+double qfx_f32_time(uint64_t m, uint64_t n, uint64_t k);  // estimate of its kernels, in us
+int qfx_launch_f32(qfx_context* ctx, const float2* A, const float2* B, float2* C, uint64_t m,
+                   uint64_t n, uint64_t k, const qfx_index_map* maps, bool a_mfast,
+                   bool b_kfast, bool needs_splits);
+
 // FP8 (E4M3, per-128x128-tile power-of-two scales) complex GEMM of
 // qfx_fp8.hip: whether the shape is large enough for its tiles, and the
 // launch (maps = {a_rows, a_cols, b_rows, b_cols} or null for row-major).

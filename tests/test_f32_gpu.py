@@ -1,0 +1,120 @@
+"""GPU parity of the FP32 matrix-core products against numpy.
+
+Inputs are small whole numbers, so that every product and sum is exact in
+FP32 (|sum| <= 18 k < 2^24 for k < 2^19): the results must equal numpy's,
+whatever the tile, the stages and the splits over k.
+"""
+import numpy as np
+import pytest
+
+from qflex_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+# Edges and remainders of the tiles (128 x 64, 64 x 32, 128 x 16, 32 x 64,
+# 32 x 16), of their stages (16, 32, 64 k) and of the splits.
+SHAPES = [(2, 2, 17), (9, 17, 64), (33, 15, 65), (31, 65, 100), (32, 64, 1000), (127, 63, 47),
+          (129, 130, 33), (65, 2, 4097), (257, 255, 1001), (20, 707, 18), (1000, 1000, 17),
+          (40000, 3, 40), (33000, 17, 31), (4097, 515, 50), (3, 5000, 129), (64, 64, 100003)]
+
+
+def whole(rng, shape):
+    return (rng.integers(-3, 4, shape) + 1j * rng.integers(-3, 4, shape)).astype(np.complex64)
+
+
+def product(a, b):
+    return (a.astype(np.complex128) @ b.astype(np.complex128)).astype(np.complex64)
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_f32_products_exact_on_whole_numbers(ctx, m, n, k):
+    rng = np.random.default_rng(m * 7 + n * 3 + k)
+    a, b = whole(rng, (m, k)), whole(rng, (k, n))
+    A = ctx.upload(np.concatenate([[0], a.ravel()]).astype(np.complex64))  # 8-byte operands
+    B, C = ctx.upload(b), ctx.alloc((m * n + 1) * 8)
+    ctx.zero(C)
+
+    class At8:
+        ptr = A.ptr + 8
+    ctx.cgemm(capi.FP32, m, n, k, At8, B, C)
+    got = ctx.download(C, np.complex64, (m * n + 1,))
+    assert np.array_equal(got[:-1].reshape(m, n), product(a, b))
+    assert got[-1] == 0  # nothing past the end
+    for buf in (A, B, C):
+        buf.free()
+
+
+def test_f32_products_keep_infinities_in_their_rows_and_columns(ctx):
+    """k that fills no stage: what pads it must not meet an operand's infinity."""
+    m, n, k = 40, 20, 21
+    rng = np.random.default_rng(3)
+    a, b = whole(rng, (m, k)), whole(rng, (k, n))
+    want = product(a, b)
+    a[7, 20] = np.inf
+    b[20, 11] = np.inf
+    A, B, C = ctx.upload(a), ctx.upload(b), ctx.alloc(m * n * 8)
+    ctx.cgemm(capi.FP32, m, n, k, A, B, C)
+    got = ctx.download(C, np.complex64, (m, n))
+    other = np.ones((m, n), bool)
+    other[7], other[:, 11] = False, False
+    assert np.array_equal(got[other], want[other])
+    assert not np.isfinite(got[~other]).any()
+    for buf in (A, B, C):
+        buf.free()
+
+
+# (dims of A, its row axes, its k axes): k contiguous, rows contiguous, and
+# neither; sizes below a tile and a stage and several stages.
+MAPS = [([4, 16, 32], [0, 1], [2]), ([2, 64, 16], [2], [0, 1]), ([16, 2, 32, 8], [1, 3], [0, 2]),
+        ([64, 1024], [0], [1]), ([4096, 16], [1], [0]), ([8, 128, 2, 16], [0, 2], [1, 3])]
+
+
+@pytest.mark.parametrize("n", [2, 16, 32])
+@pytest.mark.parametrize("dims,rows,cols", MAPS)
+def test_f32_small_mapped_products_exact(ctx, dims, rows, cols, n):
+    m, k = (int(np.prod([dims[x] for x in axes])) for axes in (rows, cols))
+    rng = np.random.default_rng(m + n + k)
+    a, b = whole(rng, dims), whole(rng, (n, k))  # B stored along k
+    A, B, C = ctx.upload(a), ctx.upload(b), ctx.alloc(m * n * 8)
+    done = ctx.cgemm_mapped(capi.FP32, A, capi.index_map(dims, rows), capi.index_map(dims, cols), B,
+                            capi.index_map([n, k], [1]), capi.index_map([n, k], [0]), C)
+    assert done
+    want = product(a.transpose(rows + cols).reshape(m, k), b.T)
+    assert np.array_equal(ctx.download(C, np.complex64, (m, n)), want)
+    for buf in (A, B, C):
+        buf.free()
+
+
+def test_f32_rows_beyond_32_bit_offsets(ctx):
+    """32 rows of 2^23 elements are 2 GiB: the 64-bit form."""
+    m, n, k = 9, 2, (1 << 23) + 5
+    rng = np.random.default_rng(1)
+    a, b = np.zeros((m, k), np.complex64), np.zeros((k, n), np.complex64)
+    pick = np.r_[0:1000, k - 1000:k]
+    a[:, pick], b[pick] = whole(rng, (m, 2000)), whole(rng, (2000, n))
+    A, B, C = ctx.upload(a), ctx.upload(b), ctx.alloc(m * n * 8)
+    ctx.cgemm(capi.FP32, m, n, k, A, B, C)
+    assert np.array_equal(ctx.download(C, np.complex64, (m, n)), product(a[:, pick], b[pick]))
+    for buf in (A, B, C):
+        buf.free()
+
+
+def test_f32_map_beyond_32_bit_offsets(ctx):
+    """A digit of A's rows at stride 2^28 elements (2 GiB)."""
+    m, n, k = 16, 8, 64
+    rng = np.random.default_rng(2)
+    a, b = whole(rng, (m, k)), whole(rng, (k, n))
+    A, B, C = ctx.alloc(8 * ((1 << 28) + 8 * k)), ctx.upload(b), ctx.alloc(m * n * 8)
+
+    class At:
+        def __init__(self, offset):
+            self.ptr = A.ptr + offset
+    ctx.upload_async(At(0), a[:8])
+    ctx.upload_async(At(8 << 28), a[8:])
+    rows = capi.index_map([8, k], [0])
+    rows.ndigits, rows.bits[1], rows.shift[1] = 2, 1, 28
+    assert ctx.cgemm_mapped(capi.FP32, A, rows, capi.index_map([8, k], [1]), B,
+                            capi.index_map([k, n], [0]), capi.index_map([k, n], [1]), C)
+    assert np.array_equal(ctx.download(C, np.complex64, (m, n)), product(a, b))
+    for buf in (A, B, C):
+        buf.free()
