@@ -162,9 +162,13 @@ int qfx_cgemm_noalloc_c64(qfx_context* ctx, int precision, uint64_t m, uint64_t 
  * odd k or n or 8-byte aligned operands that qfx_cgemm_c64 would run split
  * share a second such launch, on 128 x 64 tiles (same bits).  Products with k <= 16
  * and n <= 16 (any precision) also share one launch, of the exact-FP32 row
- * kernel qfx_cgemm_c64 runs them on (same bits); the problem list reaches
- * the device through the staged uploads.  All other products run one by
- * one through qfx_cgemm_c64.  The C_i must not overlap each other or
+ * kernel qfx_cgemm_c64 runs them on (same bits), and those with k <= 16 and
+ * n > 16 another (same bits).  The products that are FP32 in the precision
+ * share one launch per tile of the FP32 kernel, not split over k as small
+ * ones are alone (the order of their sums, and so their last bits, may
+ * differ; of 512 or more 128 x 64 tiles: run alone, same bits).  The problem
+ * list reaches the device through the staged uploads.  All other products
+ * run one by one through qfx_cgemm_c64.  The C_i must not overlap each other or
  * any A_j, B_j.  Not allowed while recording a graph.  No counterpart in the
  * reference (one cblas_cgemm per pairwise contraction, src/tensor.cpp:973). */
 typedef struct qfx_gemm_desc {

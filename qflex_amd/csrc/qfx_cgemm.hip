@@ -1033,26 +1033,6 @@ __global__ __launch_bounds__(64 * WM * WN) void cgemm_split_chain_kernel(
       int(L % gy) * 16 * J * WN, L, gridDim.x, ntiles, gy);
 }
 
-// The last of `count` > 0 entries of a grouped launch whose first index (at
-// `first`, stride `bytes`, increasing, 0 at entry 0) is <= t.  Called by whole
-// waves: 64 entries are probed at a time, so 192 entries take two dependent
-// loads, where a binary search takes eight (4 us of each block's life).
-__device__ __forceinline__ int group_entry(const uint64_t* first, size_t bytes, int count,
-                                           uint64_t t) {
-  const int lane = threadIdx.x & 63;
-  int lo = 0, n = count;
-  while (n > 1) {
-    const int step = (n + 63) / 64;
-    const int i = lane * step;
-    const bool le = i < n && *reinterpret_cast<const uint64_t*>(
-                                 reinterpret_cast<const char*>(first) + size_t(lo + i) * bytes) <= t;
-    const int c = __popcll(__ballot(le)) - 1;  // the last probed entry <= t
-    lo += c * step;
-    n = min(step, n - c * step);
-  }
-  return __builtin_amdgcn_readfirstlane(lo);
-}
-
 // One problem of a grouped launch: row-major operands, 256 x 128 tiles.
 struct GroupTile {
   const float2* A;
@@ -1510,10 +1490,11 @@ __device__ __forceinline__ void store_block_max(float v, float* slot) {
 }
 
 template <int BN, bool MAPPED>
-__global__ __launch_bounds__(256) void cgemm_smallk_kernel(
+__device__ __forceinline__ void smallk_tile(
     const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C,
-    uint64_t M, int N, int K, qfx_index_map a_rows, qfx_index_map a_cols, qfx_index_map b_rows,
-    qfx_index_map b_cols, bool a_mfast, bool b_nfast, float* __restrict__ cmax) {
+    uint64_t M, int N, int K, const qfx_index_map& a_rows, const qfx_index_map& a_cols,
+    const qfx_index_map& b_rows, const qfx_index_map& b_cols, bool a_mfast, bool b_nfast,
+    float* __restrict__ cmax, uint64_t tile_m, unsigned tile_n) {
   constexpr int TX = BN / 4;        // column groups
   constexpr int BM = 4 * 256 / TX;  // rows per block
   __shared__ float2 As[BM][kSmallK + 1];
@@ -1521,8 +1502,8 @@ __global__ __launch_bounds__(256) void cgemm_smallk_kernel(
   __shared__ uint64_t arow[MAPPED ? BM : 1], bcol[MAPPED ? BN : 1];
   __shared__ uint64_t acol[MAPPED ? kSmallK : 1], brow[MAPPED ? kSmallK : 1];
   const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-  const uint64_t m0 = uint64_t(blockIdx.x) * BM;
-  const int n0 = blockIdx.y * BN;
+  const uint64_t m0 = tile_m * BM;
+  const int n0 = int(tile_n) * BN;
   if constexpr (MAPPED) {
     for (int i = threadIdx.x; i < BM; i += 256) arow[i] = map_offset(a_rows, m0 + i);
     for (int i = threadIdx.x; i < BN; i += 256) bcol[i] = map_offset(b_cols, uint64_t(n0 + i));
@@ -1532,32 +1513,47 @@ __global__ __launch_bounds__(256) void cgemm_smallk_kernel(
     }
     __syncthreads();
   }
-  // A tile: rows m0.., all K columns
-  for (int e = threadIdx.x; e < BM * K; e += 256) {
+  // A tile: rows m0.., all K columns; B tile alike.  All of a thread's loads
+  // are in flight together: up to 4 of each, over k rounded up to 4, 8 or 16
+  // (k past K is not loaded, and no chain reads it).
+  const int kl = K <= 4 ? 2 : K <= 8 ? 3 : 4;
+  float2 va[BM * kSmallK / 256], vb[BN * kSmallK / 256];
+  auto a_at = [&](int h, int& r, int& c) {  // false (for all threads): past the tile
+    const int e = threadIdx.x + 256 * h;
+    r = MAPPED && a_mfast ? e % BM : e >> kl;
+    c = MAPPED && a_mfast ? e / BM : e & ((1 << kl) - 1);
+    return h * 256 < BM << kl;
+  };
+  auto b_at = [&](int h, int& r, int& c) {
+    const int e = threadIdx.x + 256 * h;
+    r = MAPPED && !b_nfast ? e & ((1 << kl) - 1) : e / BN;
+    c = MAPPED && !b_nfast ? e >> kl : e % BN;
+    return h * 256 < BN << kl;
+  };
+#pragma unroll
+  for (int h = 0; h < BM * kSmallK / 256; ++h) {
     int r, c;
-    if (MAPPED && a_mfast) {
-      c = e / BM;
-      r = e - c * BM;
-    } else {
-      r = e / K;
-      c = e - r * K;
-    }
-    float2 v = make_float2(0.f, 0.f);
-    if (m0 + r < M) v = MAPPED ? A[arow[r] + acol[c]] : A[(m0 + r) * K + c];
-    As[r][c] = v;
+    va[h] = make_float2(0.f, 0.f);
+    if (!a_at(h, r, c)) continue;
+    if (c < K && m0 + r < M) va[h] = MAPPED ? A[arow[r] + acol[c]] : A[(m0 + r) * K + c];
   }
-  for (int e = threadIdx.x; e < K * BN; e += 256) {
+#pragma unroll
+  for (int h = 0; h < BN * kSmallK / 256; ++h) {
     int r, c;
-    if (MAPPED && !b_nfast) {
-      c = e / K;
-      r = e - c * K;
-    } else {
-      r = e / BN;
-      c = e - r * BN;
-    }
-    float2 v = make_float2(0.f, 0.f);
-    if (n0 + c < N) v = MAPPED ? B[brow[r] + bcol[c]] : B[uint64_t(r) * N + n0 + c];
-    Bs[r][c] = v;
+    vb[h] = make_float2(0.f, 0.f);
+    if (!b_at(h, r, c)) continue;
+    if (r < K && n0 + c < N)
+      vb[h] = MAPPED ? B[brow[r] + bcol[c]] : B[uint64_t(r) * N + n0 + c];
+  }
+#pragma unroll
+  for (int h = 0; h < BM * kSmallK / 256; ++h) {
+    int r, c;
+    if (a_at(h, r, c)) As[r][c] = va[h];
+  }
+#pragma unroll
+  for (int h = 0; h < BN * kSmallK / 256; ++h) {
+    int r, c;
+    if (b_at(h, r, c)) Bs[r][c] = vb[h];
   }
   __syncthreads();
   float2 acc[4][4];
@@ -1590,7 +1586,17 @@ __global__ __launch_bounds__(256) void cgemm_smallk_kernel(
       }
     }
   }
-  if (cmax) store_block_max(cm, cmax + blockIdx.x + uint64_t(gridDim.x) * blockIdx.y);
+  if (cmax) store_block_max(cm, cmax);
+}
+
+template <int BN, bool MAPPED>
+__global__ __launch_bounds__(256) void cgemm_smallk_kernel(
+    const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C,
+    uint64_t M, int N, int K, qfx_index_map a_rows, qfx_index_map a_cols, qfx_index_map b_rows,
+    qfx_index_map b_cols, bool a_mfast, bool b_nfast, float* __restrict__ cmax) {
+  smallk_tile<BN, MAPPED>(A, B, C, M, N, K, a_rows, a_cols, b_rows, b_cols, a_mfast, b_nfast,
+                          cmax ? cmax + blockIdx.x + uint64_t(gridDim.x) * blockIdx.y : nullptr,
+                          blockIdx.x, blockIdx.y);
 }
 
 
@@ -1854,6 +1860,18 @@ __global__ __launch_bounds__(256) void cgemm_rows_grouped_kernel(const RowsProb*
   const qfx_index_map none{};
   rows_tile<false, false>(p.A, p.B, p.C, p.M, p.N, p.K, none, none, none, none, nullptr,
                           b - p.first_block);
+}
+
+// The same for k <= 16 and n > 16: tiles of 64 x 64, numbered along n first
+// (150 products of 175 x 126 x 8, one launch each 823 us, 27 us).
+__global__ __launch_bounds__(256) void cgemm_smallk_grouped_kernel(
+    const RowsProb* __restrict__ probs, int count) {
+  const uint64_t b = blockIdx.x;
+  const RowsProb p = probs[group_entry(&probs[0].first_block, sizeof(RowsProb), count, b)];
+  const qfx_index_map none{};
+  const uint64_t t = b - p.first_block, tiles_n = uint64_t((p.N + 63) / 64);
+  smallk_tile<64, false>(p.A, p.B, p.C, p.M, p.N, p.K, none, none, none, none, false, true,
+                         nullptr, t / tiles_n, unsigned(t % tiles_n));
 }
 
 unsigned cap_grid(uint64_t g) { return unsigned(std::max<uint64_t>(1, std::min<uint64_t>(g, 65535))); }
@@ -2296,7 +2314,7 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
 // A grouped launch's problem list to the device, through the staged uploads
 // and launched at once: in pieces of one 16-byte load per thread of an
 // upload's block, so that the whole list takes one trip over the bus.
-static int upload_problems(qfx_context* ctx, void* dev, const void* host, size_t bytes) {
+int qfx_upload_problems(qfx_context* ctx, void* dev, const void* host, size_t bytes) {
   for (size_t at = 0; at < bytes; at += 4096) {
     const int st = qfx_copy_h2d_async(ctx, static_cast<char*>(dev) + at,
                                       static_cast<const char*>(host) + at,
@@ -2306,11 +2324,12 @@ static int upload_problems(qfx_context* ctx, void* dev, const void* host, size_t
   return qfx_flush_uploads(ctx);
 }
 
-// The row-kernel problems of a grouped call in one launch.  The problem
+// The k <= 16 problems of a grouped call in one launch: those of the row
+// kernel (n <= 16), or those of 64 x 64 tiles.  The problem
 // list goes to the device through the staged uploads (flushed right before
 // the launch) into the workspace.
-static int launch_rows_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
-                               const std::vector<int>& rows) {
+static int launch_smallk_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
+                                 const std::vector<int>& rows, bool narrow) {
   std::vector<RowsProb> probs(rows.size());
   uint64_t blocks = 0;
   double flops = 0, bytes = 0;
@@ -2318,7 +2337,7 @@ static int launch_rows_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
     const qfx_gemm_desc& d = descs[rows[r]];
     probs[r] = RowsProb{reinterpret_cast<const float2*>(d.A), reinterpret_cast<const float2*>(d.B),
                         reinterpret_cast<float2*>(d.C), d.m, int(d.n), int(d.k), blocks};
-    blocks += (d.m + 255) / 256;
+    blocks += narrow ? (d.m + 255) / 256 : (d.m + 63) / 64 * ((d.n + 63) / 64);
     flops += 8.0 * double(d.m) * double(d.n) * double(d.k);
     bytes += 8.0 * (double(d.m) * d.k + double(d.k) * d.n + double(d.m) * d.n);
   }
@@ -2327,10 +2346,11 @@ static int launch_rows_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
   void* ws = nullptr;
   int st = qfx_workspace(ctx, probs.size() * sizeof(RowsProb), &ws);
   if (st != QFX_OK) return st;
-  st = upload_problems(ctx, ws, probs.data(), probs.size() * sizeof(RowsProb));
+  st = qfx_upload_problems(ctx, ws, probs.data(), probs.size() * sizeof(RowsProb));
   if (st != QFX_OK) return st;
   QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
-  cgemm_rows_grouped_kernel<<<unsigned(blocks), 256, 0, ctx->stream>>>(
+  (narrow ? cgemm_rows_grouped_kernel
+          : cgemm_smallk_grouped_kernel)<<<unsigned(blocks), 256, 0, ctx->stream>>>(
       static_cast<const RowsProb*>(ws), int(probs.size()));
   QFX_HIP(hipGetLastError());
   return QFX_OK;
@@ -2384,7 +2404,7 @@ static int launch_split_grouped(qfx_context* ctx, int precision, const qfx_gemm_
     t.amax = AmaxRef{part + off, ba, part + off + ba, bb};
     off += uint64_t(ba + bb);
   }
-  st = upload_problems(ctx, dev, host.data(), desc_bytes);
+  st = qfx_upload_problems(ctx, dev, host.data(), desc_bytes);
   if (st != QFX_OK) return st;
   if (nparts > 0)
     amax_grouped_kernel<<<unsigned(nparts), 256, 0, ctx->stream>>>(dev, int(host.size()), part);
@@ -2422,23 +2442,21 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
   if (precision < QFX_PREC_FP32 || precision > QFX_PREC_FP8)
     return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: unknown precision");
   const bool split = split_precision(precision);
-  // Problems for the large tiles go into one launch, and so do those of the
-  // row kernel (k, n <= 16, any precision: exact FP32, the kernel
-  // qfx_cgemm_c64 runs them on); the others (other precisions, odd sizes,
-  // unaligned or too large operands) run one by one exactly as
-  // qfx_cgemm_c64 would run them.
-  std::vector<int> grouped, grouped_odd, rows;
+  // One launch each for the problems of the large tiles, of the odd ones, of
+  // the row kernel (k, n <= 16), of the other k <= 16 ones (both exact FP32 in
+  // any precision) and per tile of the FP32 kernel.  What is left (exact
+  // FP32 beyond k = 16, vectors, very large operands, FP8) runs one by one.
+  std::vector<int> grouped, grouped_odd, rows, smallk, f32;
   for (int i = 0; i < count; ++i) {
     const qfx_gemm_desc& d = descs[i];
-    if (d.m > 0 && d.n > 0 && d.k > 0 && d.k <= uint64_t(kSmallK) && d.n <= 16 && d.A && d.B &&
-        d.C && (d.m + 255) / 256 <= 0x7fffffffULL) {
+    const bool full = d.m > 0 && d.n > 0 && d.k > 0 && d.A && d.B && d.C;
+    if (full && d.k <= uint64_t(kSmallK) && d.n <= 16 && (d.m + 255) / 256 <= 0x7fffffffULL) {
       rows.push_back(i);
       continue;
     }
-    const bool fits = split && d.m > 0 && d.n > 0 && d.k > uint64_t(kSmallK) && d.A && d.B &&
-                      d.C && big_operands_fit(d.m, d.n, d.k) &&
-                      big_operands_whole(d.m, d.n, d.k) && d.m <= 0x7fffffffULL &&
-                      d.n <= 0x7fffffffULL;
+    const bool fits = split && full && d.k > uint64_t(kSmallK) &&
+                      big_operands_fit(d.m, d.n, d.k) && big_operands_whole(d.m, d.n, d.k) &&
+                      d.m <= 0x7fffffffULL && d.n <= 0x7fffffffULL;
     const bool even = d.k % 2 == 0 && d.n % 2 == 0 &&
                       reinterpret_cast<uintptr_t>(d.A) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(d.B) % 16 == 0;
@@ -2447,16 +2465,36 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
       continue;
     }
     // the odd products that alone would run split on the matrix cores (the
-    // others are exact FP32 alone, and stay so)
+    // others are FP32 alone, and stay so)
     if (fits && !f32_route(precision, d.m, d.n, d.k, false)) {
       grouped_odd.push_back(i);
+      continue;
+    }
+    const bool small = d.k <= uint64_t(kSmallK) && d.n <= 65535ULL * 64 &&
+                       d.m <= 0x7fffffffULL;
+    const bool matrix = d.k > uint64_t(kSmallK) && d.m > 1 && d.n > 1 &&
+                        (d.m > 8 || d.n > 8 || d.k < 1024) && precision != QFX_PREC_FP8 &&
+                        f32_route(precision, d.m, d.n, d.k, false);
+    if (full && (small || matrix)) {
+      QFX_EXTENT(ctx, d.A, 8.0 * double(d.m) * double(d.k), "qfx_cgemm_grouped_c64: A");
+      QFX_EXTENT(ctx, d.B, 8.0 * double(d.k) * double(d.n), "qfx_cgemm_grouped_c64: B");
+      QFX_EXTENT(ctx, d.C, 8.0 * double(d.m) * double(d.n), "qfx_cgemm_grouped_c64: C");
+      (small ? smallk : f32).push_back(i);
       continue;
     }
     const int st = qfx_cgemm_c64(ctx, precision, d.m, d.n, d.k, d.A, d.B, d.C);
     if (st != QFX_OK) return st;
   }
   if (!rows.empty()) {
-    const int st = launch_rows_grouped(ctx, descs, rows);
+    const int st = launch_smallk_grouped(ctx, descs, rows, true);
+    if (st != QFX_OK) return st;
+  }
+  if (!smallk.empty()) {
+    const int st = launch_smallk_grouped(ctx, descs, smallk, false);
+    if (st != QFX_OK) return st;
+  }
+  if (!f32.empty()) {
+    const int st = qfx_launch_f32_grouped(ctx, descs, f32);
     if (st != QFX_OK) return st;
   }
   if (!grouped.empty()) {

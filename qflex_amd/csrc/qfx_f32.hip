@@ -26,6 +26,7 @@
 // tiles add their sums up once per stage): 57 x 104 x 3384 1e-6 -> 1e-7.
 #include <algorithm>
 #include <type_traits>
+#include <vector>
 
 #include "qfx_internal.h"
 
@@ -293,6 +294,31 @@ __global__ __launch_bounds__(256, 2) void cgemm_f32_kernel(
                     min(s0 + stages_per, stages), lds);
 }
 
+// One problem of a grouped launch (row-major operands).
+struct F32Prob {
+  const float2* A;
+  const float2* B;
+  float2* C;
+  int64_t K;
+  int M, N, tiles_n, stages;
+  uint64_t first_tile;  // index of its first tile in the launch
+};
+
+// A block per tile of all problems that take this tile; one launch each took
+// 5 to 10 us (100 products of 512 x 64 x 64: 1045 -> 38 us, 250 of 64 x 5 x 100
+// 6534 -> 41, most of the last the caller's list).
+template <class T>
+__global__ __launch_bounds__(256, 2) void cgemm_f32_grouped_kernel(
+    const F32Prob* __restrict__ probs, int count) {
+  __shared__ __align__(16) float2 lds[T::kLds];
+  const uint64_t t = xcd_tile(blockIdx.x, gridDim.x);
+  const F32Prob p = probs[group_entry(&probs[0].first_tile, sizeof(F32Prob), count, t)];
+  const int local = int(t - p.first_tile);
+  const int tm = __builtin_amdgcn_readfirstlane(local / p.tiles_n);
+  f32_tile<T, kRowMajor>(p.A, p.B, p.C, p.M, p.N, p.K, Maps{}, false, false, false, tm * T::TM,
+                         (local - tm * p.tiles_n) * T::TN, 0, p.stages, lds);
+}
+
 // C[c] = sum_s part[s][c]: four groups of 64 lanes, eight loads in flight.
 __global__ __launch_bounds__(256) void f32_sum_kernel(const float2* __restrict__ part,
                                                       float2* __restrict__ C, int nsplit,
@@ -344,8 +370,9 @@ int stage_of(F32Tile t) {
 // CU, and for splits the sum's launch and its traffic.  Within 10% of the best
 // measured choice on 30 shapes but for 12-20% on three below 13 us.  Only
 // products of up to 2^16 outputs are split (16 MiB of partial sums at most).
+constexpr double kStageUs[] = {2.0, 1.2, 0.6, 0.6, 0.9};  // per tile, every CU busy
+constexpr double kAlone = 1.35;                           // of a CU with one block
 F32Plan f32_plan(uint64_t m, uint64_t n, uint64_t k) {
-  static const double us[] = {2.0, 1.2, 0.6, 0.6, 0.9};  // per stage
   F32Plan best{kTileC, 1, 1e30};
   for (int t = kTileA; t <= kTileC; ++t) {
     const uint64_t tiles = tiles_of(F32Tile(t), m, n), kb = stage_of(F32Tile(t));
@@ -356,7 +383,7 @@ F32Plan f32_plan(uint64_t m, uint64_t n, uint64_t k) {
         break;
       const uint64_t per = (stages + s - 1) / s, splits = (stages + per - 1) / per;
       const uint64_t rounds = (tiles * splits + 255) / 256;
-      double time = us[t] * double(per) * (rounds == 1 ? 1.35 : double(rounds));
+      double time = kStageUs[t] * double(per) * (rounds == 1 ? kAlone : double(rounds));
       if (splits > 1) time += 2.5 + double(splits * m * n) * 4e-6;
       if (time < best.us) best = F32Plan{F32Tile(t), int(splits), time};
     }
@@ -405,7 +432,7 @@ double qfx_f32_time(uint64_t m, uint64_t n, uint64_t k) { return f32_plan(m, n, 
 
 bool qfx_f32_fits(uint64_t m, uint64_t n, uint64_t k) {
   return m <= 0x7fffff00ULL && n <= 0x7fffff00ULL && k <= (1ULL << 34) &&
-         tiles_of(f32_plan(m, n, k).tile, m, n) <= 0x7fffffffULL;
+         tiles_of(kTileC, m, n) <= 0x7fffffffULL;  // (the smallest tile)
 }
 
 int qfx_launch_f32(qfx_context* ctx, const float2* A, const float2* B, float2* C, uint64_t m,
@@ -433,6 +460,89 @@ int qfx_launch_f32(qfx_context* ctx, const float2* A, const float2* B, float2* C
                              : go(TileC{}));
   if (p.splits > 1)
     f32_sum_kernel<<<unsigned((m * n + 63) / 64), 256, 0, ctx->stream>>>(out, C, p.splits, m * n);
+  QFX_HIP(hipGetLastError());
+  return QFX_OK;
+}
+
+int qfx_launch_f32_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
+                           const std::vector<int>& which) {
+  // Each product takes the tile that would be the fastest if all were like it.
+  // Those that fill the chip alone run as qfx_cgemm_c64 runs them, and so do
+  // all of a few where that is estimated faster (long k, split alone).
+  std::vector<std::vector<int>> by_tile(kTileC + 1);
+  double alone_us = 0, group_us = 6, longest = 0;
+  auto alone = [&](const qfx_gemm_desc& d) {
+    return qfx_launch_f32(ctx, reinterpret_cast<const float2*>(d.A),
+                          reinterpret_cast<const float2*>(d.B), reinterpret_cast<float2*>(d.C),
+                          d.m, d.n, d.k, nullptr, false, false, false);
+  };
+  for (int i : which) {
+    const qfx_gemm_desc& d = descs[i];
+    const bool reach = 128 * d.k + 64 < (1ULL << 28) && 64 * d.n + 64 < (1ULL << 28) &&
+                       tiles_of(kTileC, d.m, d.n) < (1ULL << 24);
+    if (!reach || tiles_of(kTileA, d.m, d.n) >= 512) {
+      const int st = alone(d);
+      if (st != QFX_OK) return st;
+      continue;
+    }
+    int best = -1;
+    double best_us = 1e30, best_work = 0, best_chain = 0;
+    for (int t = kTileA; t <= kTileC; ++t) {
+      const uint64_t kb = stage_of(F32Tile(t));
+      const double chain = kStageUs[t] * double((d.k + kb - 1) / kb);
+      const double work = chain * double(tiles_of(F32Tile(t), d.m, d.n)) / 256;
+      const double us = work * double(which.size()) + kAlone * chain;
+      if (us < best_us) best = t, best_us = us, best_work = work, best_chain = chain;
+    }
+    by_tile[best].push_back(i);
+    alone_us += which.size() > 16 ? 1e9 : f32_plan(d.m, d.n, d.k).us + 4;
+    group_us += best_work;
+    longest = std::max(longest, kAlone * best_chain);
+  }
+  std::vector<F32Prob> probs;
+  uint64_t tiles[kTileC + 1] = {};
+  for (int t = kTileA; t <= kTileC; ++t)
+    for (int i : by_tile[t]) {
+      const qfx_gemm_desc& d = descs[i];
+      if (alone_us < group_us + longest) {
+        const int st = alone(d);
+        if (st != QFX_OK) return st;
+        continue;
+      }
+      static const int tn[] = {64, 32, 16, 64, 16};
+      probs.push_back(F32Prob{reinterpret_cast<const float2*>(d.A),
+                              reinterpret_cast<const float2*>(d.B), reinterpret_cast<float2*>(d.C),
+                              int64_t(d.k), int(d.m), int(d.n), int((d.n + tn[t] - 1) / tn[t]),
+                              int((d.k + stage_of(F32Tile(t)) - 1) / stage_of(F32Tile(t))),
+                              tiles[t]});
+      tiles[t] += tiles_of(F32Tile(t), d.m, d.n);
+      if (tiles[t] > 0x7fffffffULL)
+        return qfx_set_error(QFX_ERR_UNSUPPORTED, "qfx_cgemm_grouped_c64: too many tiles");
+    }
+  if (probs.empty()) return QFX_OK;
+  void* ws = nullptr;
+  int st = qfx_workspace(ctx, probs.size() * sizeof(F32Prob), &ws);
+  if (st != QFX_OK) return st;
+  st = qfx_upload_problems(ctx, ws, probs.data(), probs.size() * sizeof(F32Prob));
+  if (st != QFX_OK) return st;
+  double flops = 0, bytes = 0;
+  for (const F32Prob& p : probs) {
+    flops += 8.0 * p.M * p.N * double(p.K);
+    bytes += 8.0 * (double(p.M) * p.K + double(p.K) * p.N + double(p.M) * p.N);
+  }
+  QfxLaunchScope scope(ctx, QFX_K_CGEMM, bytes, flops);
+  const F32Prob* dev = static_cast<const F32Prob*>(ws);
+  auto go = [&](auto tile, int t) {
+    const int n = int(by_tile[t].size());
+    if (n == 0) return;
+    cgemm_f32_grouped_kernel<decltype(tile)><<<unsigned(tiles[t]), 256, 0, ctx->stream>>>(dev, n);
+    dev += n;
+  };
+  go(TileA{}, kTileA);
+  go(TileF{}, kTileF);
+  go(TileD{}, kTileD);
+  go(TileE{}, kTileE);
+  go(TileC{}, kTileC);
   QFX_HIP(hipGetLastError());
   return QFX_OK;
 }

@@ -154,6 +154,26 @@ __device__ __forceinline__ uint64_t map_offset(const qfx_index_map& d, uint64_t 
   return off;
 }
 
+// The last of `count` > 0 entries of a grouped launch whose first index (at
+// `first`, stride `bytes`, increasing, 0 at entry 0) is <= t.  Called by whole
+// waves: 64 entries are probed at a time, so 192 entries take two dependent
+// loads, where a binary search takes eight (4 us of each block's life).
+__device__ __forceinline__ int group_entry(const uint64_t* first, size_t bytes, int count,
+                                           uint64_t t) {
+  const int lane = threadIdx.x & 63;
+  int lo = 0, n = count;
+  while (n > 1) {
+    const int step = (n + 63) / 64;
+    const int i = lane * step;
+    const bool le = i < n && *reinterpret_cast<const uint64_t*>(
+                                 reinterpret_cast<const char*>(first) + size_t(lo + i) * bytes) <= t;
+    const int c = __popcll(__ballot(le)) - 1;  // the last probed entry <= t
+    lo += c * step;
+    n = min(step, n - c * step);
+  }
+  return __builtin_amdgcn_readfirstlane(lo);
+}
+
 // Matrix-vector products of qfx_gemv.hip (pointers checked by the caller,
 // m, k > 0): y[m] = A[m x k] . x, without device scratch, and y[k] =
 // sum_r x[r] A[r][.].
@@ -168,6 +188,12 @@ int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
 // outputs are split over k through the workspace; where a sequence being
 // recorded has reserved too little, needs_splits refuses them.
 bool qfx_f32_fits(uint64_t m, uint64_t n, uint64_t k);
+// The products of a grouped call that would run there, `which` of them, in one
+// launch per tile (row-major operands, pointers checked).
+int qfx_launch_f32_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
+                           const std::vector<int>& which);
+// A grouped launch's problem list to the device, through the staged uploads.
+int qfx_upload_problems(qfx_context* ctx, void* dev, const void* host, size_t bytes);
 double qfx_f32_time(uint64_t m, uint64_t n, uint64_t k);  // estimate of its kernels, in us
 int qfx_launch_f32(qfx_context* ctx, const float2* A, const float2* B, float2* C, uint64_t m,
                    uint64_t n, uint64_t k, const qfx_index_map* maps, bool a_mfast,
