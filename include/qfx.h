@@ -166,8 +166,9 @@ int qfx_cgemm_noalloc_c64(qfx_context* ctx, int precision, uint64_t m, uint64_t 
  * n > 16 another (same bits).  The products that are FP32 in the precision
  * share one launch per tile of the FP32 kernel, not split over k as small
  * ones are alone (the order of their sums, and so their last bits, may
- * differ; of 512 or more 128 x 64 tiles: run alone, same bits).  The problem
- * list reaches the device through the staged uploads.  All other products
+ * differ; of 512 or more 128 x 64 tiles: run alone, same bits).  A
+ * launch's problem list goes up as a kernel argument (up to 32) or through the
+ * staged uploads.  All other products
  * run one by one through qfx_cgemm_c64.  The C_i must not overlap each other or
  * any A_j, B_j.  Not allowed while recording a graph.  No counterpart in the
  * reference (one cblas_cgemm per pairwise contraction, src/tensor.cpp:973). */

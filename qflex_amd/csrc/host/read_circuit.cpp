@@ -296,6 +296,82 @@ void circuit_data_to_tensor_network(
   }
 }
 
+namespace {
+
+// The indices of a site tensor while bonds are bundled: each is a run of the
+// axes the tensor is stored with, so that any number of reorders and bundles
+// cost one permutation of the data.
+struct SiteIndices {
+  std::vector<std::string> names;
+  std::vector<std::vector<std::size_t>> axes;  // of each index, in order
+
+  explicit SiteIndices(const Tensor& t) : names(t.get_indices()) {
+    for (std::size_t a = 0; a < names.size(); ++a) axes.push_back({a});
+  }
+
+  // As Tensor::reorder; false where `order` is no reordering of the indices.
+  bool reorder(const std::vector<std::string>& order) {
+    if (order.size() != names.size()) return false;
+    std::vector<std::vector<std::size_t>> moved;
+    for (const auto& x : order) {
+      const auto it = std::find(names.begin(), names.end(), x);
+      if (it == names.end()) return false;
+      moved.push_back(axes[std::size_t(it - names.begin())]);
+    }
+    std::size_t total = 0;  // (an index named twice would repeat axes)
+    for (const auto& x : names) total += std::size_t(_string_in_vector(x, order));
+    if (total != names.size()) return false;
+    names = order;
+    axes = std::move(moved);
+    return true;
+  }
+
+  // The `count` indices from `at` on as one.
+  void bundle(std::size_t at, std::size_t count, const std::string& name) {
+    std::vector<std::size_t> run;
+    for (std::size_t x = at; x < at + count; ++x)
+      run.insert(run.end(), axes[x].begin(), axes[x].end());
+    names.erase(names.begin() + at, names.begin() + at + count);
+    axes.erase(axes.begin() + at, axes.begin() + at + count);
+    names.insert(names.begin() + at, name);
+    axes.insert(axes.begin() + at, std::move(run));
+  }
+
+  // The tensor these indices were made of, permuted to `order`.
+  void apply(Tensor& t, const std::vector<std::string>& order, s_type* scratch) {
+    const bool valid = reorder(order);
+    const std::vector<std::string> stored = t.get_indices();
+    const std::vector<std::size_t> stored_dims = t.get_dimensions();
+    std::vector<std::string> flat;
+    std::vector<std::size_t> dims;
+    for (const auto& run : axes) {
+      std::size_t d = 1;
+      for (std::size_t a : run) {
+        flat.push_back(stored[a]);
+        d *= stored_dims[a];
+      }
+      dims.push_back(d);
+    }
+    if (!flat.empty()) t.reorder(flat, scratch);
+    t.set_indices_and_dimensions(names, dims);
+    if (!valid || flat.empty()) t.reorder(order, scratch);  // its message or warning
+  }
+};
+
+// bundle_between on the index lists of two sites.
+void bundle_indices(SiteIndices& A, SiteIndices& B, const std::string& name) {
+  const auto left = _vector_subtraction(A.names, B.names);
+  const auto right = _vector_subtraction(B.names, A.names);
+  const auto common = _vector_intersection(A.names, B.names);
+  A.reorder(_vector_union(left, common));
+  B.reorder(_vector_union(common, right));
+  // (sites without a common gate: a bond of dimension 1, first in both)
+  A.bundle(common.empty() ? 0 : left.size(), common.size(), name);
+  B.bundle(0, common.size(), name);
+}
+
+}  // namespace
+
 void flatten_grid_of_tensors(
     std::vector<std::vector<std::vector<Tensor>>>& grid_of_tensors,
     std::vector<std::vector<Tensor>>& grid_of_tensors_2D,
@@ -306,10 +382,12 @@ void flatten_grid_of_tensors(
   const std::size_t I = grid_of_tensors.size();
   // 1. Contract each qubit's time line into one site tensor, one gate layer
   //    at a time over all sites (the reference runs each site's line to the
-  //    end; the products are the same): the matrix products of a layer go
-  //    out as one grouped launch, products with a vector operand one by one.
+  //    end; the products are the same).  The products of a layer go out as
+  //    one grouped launch, those of vectors over up to 16 values (gates of
+  //    one qubit on the initial state, 56 of the 180 launches of a 4 x 4
+  //    circuit of depth 16) among them.
   std::vector<std::array<std::size_t, 2>> sites;
-  std::vector<Tensor> line_product;
+  std::vector<Tensor*> line_product;  // the line's first tensor, then `product`
   std::size_t depth = 0;
   for (std::size_t i = 0; i < I; ++i) {
     const std::size_t J = grid_of_tensors[i].size();
@@ -317,11 +395,11 @@ void flatten_grid_of_tensors(
       if (find_grid_coord_in_list(off, i, j)) continue;
       if (grid_of_tensors[i][j].empty()) throw ERROR_MSG("Time-direction cannot be empty");
       sites.push_back({i, j});
-      line_product.push_back(grid_of_tensors[i][j][0]);
+      line_product.push_back(&grid_of_tensors[i][j][0]);
       depth = std::max(depth, grid_of_tensors[i][j].size());
     }
   }
-  std::vector<Tensor> next(sites.size());
+  std::vector<Tensor> product(sites.size()), next(sites.size());
   std::vector<qfx_gemm_desc> layer;
   for (std::size_t k = 1; k < depth; ++k) {
     layer.clear();
@@ -329,12 +407,12 @@ void flatten_grid_of_tensors(
     for (std::size_t s = 0; s < sites.size(); ++s) {
       auto& line = grid_of_tensors[sites[s][0]][sites[s][1]];
       if (k >= line.size()) continue;
-      Tensor& A = line_product[s];
+      Tensor& A = *line_product[s];
       Tensor& B = line[k];
       Tensor C({""}, {result_size(A, B)}, Tensor::for_overwrite);  // written whole below
       try {
         const ProductShape p = prepare_multiply(A, B, C, scratch);
-        if (p.has_left && p.has_right) {
+        if ((p.has_left && p.has_right) || p.common_dim <= 16) {
           layer.push_back(qfx_gemm_desc{p.left_dim, p.right_dim, p.common_dim,
                                         reinterpret_cast<const qfx_c64*>(A.data()),
                                         reinterpret_cast<const qfx_c64*>(B.data()),
@@ -352,11 +430,23 @@ void flatten_grid_of_tensors(
     if (!layer.empty())
       qfx_check(qfx_cgemm_grouped_c64(device(), global::precision, int(layer.size()), layer.data()),
                 "qfx_cgemm_grouped_c64");
-    for (std::size_t s : stepped) line_product[s] = std::move(next[s]);
+    for (std::size_t s : stepped) {
+      product[s] = std::move(next[s]);
+      line_product[s] = &product[s];
+    }
   }
-  for (std::size_t s = 0; s < sites.size(); ++s)
-    grid_of_tensors_2D[sites[s][0]][sites[s][1]] = std::move(line_product[s]);
-  // 2. Bundle the virtual indices shared by neighbouring sites into one bond.
+  for (std::size_t s = 0; s < sites.size(); ++s) {
+    Tensor& site = grid_of_tensors_2D[sites[s][0]][sites[s][1]];
+    if (line_product[s] == &product[s])
+      site = std::move(product[s]);
+    else
+      site = Tensor(*line_product[s]);
+  }
+  // 2. Bundle the virtual indices shared by neighbouring sites into one bond:
+  //    on the sites' index lists only, the data moves once, below.
+  std::vector<std::vector<SiteIndices>> site_indices(I);
+  for (std::size_t i = 0; i < I; ++i)
+    for (const auto& t : grid_of_tensors_2D[i]) site_indices[i].emplace_back(t);
   for (std::size_t i = 0; i < I; ++i) {
     const std::size_t J = grid_of_tensors[i].size();
     for (std::size_t j = 0; j < J; ++j) {
@@ -365,8 +455,8 @@ void flatten_grid_of_tensors(
       if (i < I - 1 && !find_grid_coord_in_list(off, i + 1, j)) pairs.push_back({i + 1, j});
       if (j < J - 1 && !find_grid_coord_in_list(off, i, j + 1)) pairs.push_back({i, j + 1});
       for (const auto& pair : pairs)
-        bundle_between(grid_of_tensors_2D[i][j], grid_of_tensors_2D[pair[0]][pair[1]],
-                       index_name({i, j}, pair), scratch);
+        bundle_indices(site_indices[i][j], site_indices[pair[0]][pair[1]],
+                       index_name({i, j}, pair));
     }
   }
   // 3. Put each site's indices in the order the contraction consumes them.
@@ -401,7 +491,7 @@ void flatten_grid_of_tensors(
           order.push_back(index_name(local, pair));
       }
       try {
-        grid_of_tensors_2D[i][j].reorder(order, scratch);
+        site_indices[i][j].apply(grid_of_tensors_2D[i][j], order, scratch);
       } catch (const std::string& err_msg) {
         throw ERROR_MSG("Failed to call reorder(). Error:\n\t[", err_msg, "]");
       }

@@ -1853,25 +1853,39 @@ struct RowsProb {
 
 // Grouped row kernel: block b runs block b - first_block of the last
 // problem whose first block is <= b.
-__global__ __launch_bounds__(256) void cgemm_rows_grouped_kernel(const RowsProb* __restrict__ probs,
-                                                                 int count) {
+__device__ __forceinline__ void rows_grouped_block(const RowsProb* probs, int count) {
   const uint64_t b = blockIdx.x;
   const RowsProb p = probs[group_entry(&probs[0].first_block, sizeof(RowsProb), count, b)];
   const qfx_index_map none{};
   rows_tile<false, false>(p.A, p.B, p.C, p.M, p.N, p.K, none, none, none, none, nullptr,
                           b - p.first_block);
 }
+__global__ __launch_bounds__(256) void cgemm_rows_grouped_kernel(const RowsProb* __restrict__ probs,
+                                                                 int count) {
+  rows_grouped_block(probs, count);
+}
+__global__ __launch_bounds__(256) void cgemm_rows_grouped_args_kernel(ArgList<RowsProb> list,
+                                                                      int count) {
+  rows_grouped_block(list.p, count);
+}
 
 // The same for k <= 16 and n > 16: tiles of 64 x 64, numbered along n first
 // (150 products of 175 x 126 x 8, one launch each 823 us, 27 us).
-__global__ __launch_bounds__(256) void cgemm_smallk_grouped_kernel(
-    const RowsProb* __restrict__ probs, int count) {
+__device__ __forceinline__ void smallk_grouped_block(const RowsProb* probs, int count) {
   const uint64_t b = blockIdx.x;
   const RowsProb p = probs[group_entry(&probs[0].first_block, sizeof(RowsProb), count, b)];
   const qfx_index_map none{};
   const uint64_t t = b - p.first_block, tiles_n = uint64_t((p.N + 63) / 64);
   smallk_tile<64, false>(p.A, p.B, p.C, p.M, p.N, p.K, none, none, none, none, false, true,
                          nullptr, t / tiles_n, unsigned(t % tiles_n));
+}
+__global__ __launch_bounds__(256) void cgemm_smallk_grouped_kernel(
+    const RowsProb* __restrict__ probs, int count) {
+  smallk_grouped_block(probs, count);
+}
+__global__ __launch_bounds__(256) void cgemm_smallk_grouped_args_kernel(ArgList<RowsProb> list,
+                                                                        int count) {
+  smallk_grouped_block(list.p, count);
 }
 
 unsigned cap_grid(uint64_t g) { return unsigned(std::max<uint64_t>(1, std::min<uint64_t>(g, 65535))); }
@@ -2325,7 +2339,7 @@ int qfx_upload_problems(qfx_context* ctx, void* dev, const void* host, size_t by
 }
 
 // The k <= 16 problems of a grouped call in one launch: those of the row
-// kernel (n <= 16), or those of 64 x 64 tiles.  The problem
+// kernel (n <= 16), or those of 64 x 64 tiles.  A longer problem
 // list goes to the device through the staged uploads (flushed right before
 // the launch) into the workspace.
 static int launch_smallk_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
@@ -2343,6 +2357,16 @@ static int launch_smallk_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
   }
   if (blocks > 0x7fffffffULL)
     return qfx_set_error(QFX_ERR_UNSUPPORTED, "qfx_cgemm_grouped_c64: too many row blocks");
+  if (probs.size() <= size_t(kArgProblems)) {
+    ArgList<RowsProb> list{};
+    std::copy(probs.begin(), probs.end(), list.p);
+    QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
+    (narrow ? cgemm_rows_grouped_args_kernel
+            : cgemm_smallk_grouped_args_kernel)<<<unsigned(blocks), 256, 0, ctx->stream>>>(
+        list, int(probs.size()));
+    QFX_HIP(hipGetLastError());
+    return QFX_OK;
+  }
   void* ws = nullptr;
   int st = qfx_workspace(ctx, probs.size() * sizeof(RowsProb), &ws);
   if (st != QFX_OK) return st;

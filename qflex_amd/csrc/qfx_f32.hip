@@ -308,15 +308,25 @@ struct F32Prob {
 // 5 to 10 us (100 products of 512 x 64 x 64: 1045 -> 38 us, 250 of 64 x 5 x 100
 // 6534 -> 41, most of the last the caller's list).
 template <class T>
-__global__ __launch_bounds__(256, 2) void cgemm_f32_grouped_kernel(
-    const F32Prob* __restrict__ probs, int count) {
-  __shared__ __align__(16) float2 lds[T::kLds];
+__device__ __forceinline__ void f32_grouped_block(const F32Prob* probs, int count, float2* lds) {
   const uint64_t t = xcd_tile(blockIdx.x, gridDim.x);
   const F32Prob p = probs[group_entry(&probs[0].first_tile, sizeof(F32Prob), count, t)];
   const int local = int(t - p.first_tile);
   const int tm = __builtin_amdgcn_readfirstlane(local / p.tiles_n);
   f32_tile<T, kRowMajor>(p.A, p.B, p.C, p.M, p.N, p.K, Maps{}, false, false, false, tm * T::TM,
                          (local - tm * p.tiles_n) * T::TN, 0, p.stages, lds);
+}
+template <class T>
+__global__ __launch_bounds__(256, 2) void cgemm_f32_grouped_kernel(
+    const F32Prob* __restrict__ probs, int count) {
+  __shared__ __align__(16) float2 lds[T::kLds];
+  f32_grouped_block<T>(probs, count, lds);
+}
+template <class T>
+__global__ __launch_bounds__(256, 2) void cgemm_f32_grouped_args_kernel(ArgList<F32Prob> list,
+                                                                        int count) {
+  __shared__ __align__(16) float2 lds[T::kLds];
+  f32_grouped_block<T>(list.p, count, lds);
 }
 
 // C[c] = sum_s part[s][c]: four groups of 64 lanes, eight loads in flight.
@@ -520,11 +530,14 @@ int qfx_launch_f32_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
         return qfx_set_error(QFX_ERR_UNSUPPORTED, "qfx_cgemm_grouped_c64: too many tiles");
     }
   if (probs.empty()) return QFX_OK;
+  const bool args = probs.size() <= size_t(kArgProblems);
   void* ws = nullptr;
-  int st = qfx_workspace(ctx, probs.size() * sizeof(F32Prob), &ws);
-  if (st != QFX_OK) return st;
-  st = qfx_upload_problems(ctx, ws, probs.data(), probs.size() * sizeof(F32Prob));
-  if (st != QFX_OK) return st;
+  if (!args) {
+    int st = qfx_workspace(ctx, probs.size() * sizeof(F32Prob), &ws);
+    if (st != QFX_OK) return st;
+    st = qfx_upload_problems(ctx, ws, probs.data(), probs.size() * sizeof(F32Prob));
+    if (st != QFX_OK) return st;
+  }
   double flops = 0, bytes = 0;
   for (const F32Prob& p : probs) {
     flops += 8.0 * p.M * p.N * double(p.K);
@@ -532,11 +545,20 @@ int qfx_launch_f32_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
   }
   QfxLaunchScope scope(ctx, QFX_K_CGEMM, bytes, flops);
   const F32Prob* dev = static_cast<const F32Prob*>(ws);
+  const F32Prob* host = probs.data();
   auto go = [&](auto tile, int t) {
     const int n = int(by_tile[t].size());
     if (n == 0) return;
-    cgemm_f32_grouped_kernel<decltype(tile)><<<unsigned(tiles[t]), 256, 0, ctx->stream>>>(dev, n);
-    dev += n;
+    if (args) {
+      ArgList<F32Prob> list{};
+      std::copy(host, host + n, list.p);
+      cgemm_f32_grouped_args_kernel<decltype(tile)>
+          <<<unsigned(tiles[t]), 256, 0, ctx->stream>>>(list, n);
+    } else {
+      cgemm_f32_grouped_kernel<decltype(tile)><<<unsigned(tiles[t]), 256, 0, ctx->stream>>>(dev, n);
+      dev += n;
+    }
+    host += n;
   };
   go(TileA{}, kTileA);
   go(TileF{}, kTileF);

@@ -174,6 +174,14 @@ __device__ __forceinline__ int group_entry(const uint64_t* first, size_t bytes, 
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
+// A short problem list as a kernel argument: no workspace and no upload launch
+// before the grouped one (5 us of a call).
+constexpr int kArgProblems = 32;
+template <class P>
+struct ArgList {
+  P p[kArgProblems];
+};
+
 // Matrix-vector products of qfx_gemv.hip (pointers checked by the caller,
 // m, k > 0): y[m] = A[m x k] . x, without device scratch, and y[k] =
 // sum_r x[r] A[r][.].

@@ -120,11 +120,13 @@ def test_f32_map_beyond_32_bit_offsets(ctx):
         buf.free()
 
 
+@pytest.mark.parametrize("times", [1, 8])
 @pytest.mark.parametrize("prec", [capi.FP32, capi.SPLIT_FP16, capi.SPLIT_BF16X3])
-def test_grouped_products_off_the_large_tiles_exact(ctx, prec):
+def test_grouped_products_off_the_large_tiles_exact(ctx, prec, times):
     """Every route of a grouped call that is FP32 in this precision, several
     products per tile and some alone, operands at 8-byte addresses: k <= 16
-    with n above and below 16, and the FP32 kernel's tiles."""
+    with n above and below 16, and the FP32 kernel's tiles; problem lists as
+    kernel arguments and uploaded."""
     shapes = [(5, 3, 1), (300, 16, 16), (70, 17, 5), (64, 64, 16), (129, 200, 11), (1, 40, 9),
               (33, 7, 35), (513, 9, 100), (20, 300, 33), (40, 15, 1025), (63, 90, 49),
               (9, 4, 4097), (32, 64, 17), (1000, 2, 19), (17, 130, 300)]
@@ -132,7 +134,7 @@ def test_grouped_products_off_the_large_tiles_exact(ctx, prec):
         shapes += [(100, 100, 100), (513, 65, 33), (1300, 700, 20), (129, 129, 1000)]
     rng = np.random.default_rng(prec)
     problems, want, bufs = [], [], []
-    for m, n, k in shapes * 2:
+    for m, n, k in shapes * times:
         a, b = whole(rng, (m, k)), whole(rng, (k, n))
         A = ctx.upload(np.concatenate([[0], a.ravel()]).astype(np.complex64))
         B, C = ctx.upload(b), ctx.alloc((m * n + 1) * 8)
