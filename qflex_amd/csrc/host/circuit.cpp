@@ -187,7 +187,7 @@ void QflexCircuit::load(std::istream&& istream) {
       if (!integer_token(words[w], &q)) throw fail("Qubit must be a valid number.");
       gate.qubits.push_back(std::size_t(q));
     }
-    gates.push_back(gate);
+    gates.push_back(std::move(gate));
     for (auto q : gates.back().qubits)
       if (!busy.insert(q).second) throw fail("Qubits can only used once per cycle.");
   }

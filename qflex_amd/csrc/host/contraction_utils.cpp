@@ -79,9 +79,10 @@ std::vector<std::size_t> get_qubit_coords(std::size_t q, std::size_t J) {
 
 bool find_grid_coord_in_list(const std::optional<std::vector<std::vector<std::size_t>>>& coord_list,
                              const std::size_t i, const std::size_t j) {
-  return coord_list.has_value() &&
-         std::find(coord_list.value().begin(), coord_list.value().end(),
-                   std::vector<std::size_t>({i, j})) != coord_list.value().end();
+  if (!coord_list.has_value()) return false;
+  for (const auto& at : coord_list.value())
+    if (at.size() == 2 && at[0] == i && at[1] == j) return true;
+  return false;
 }
 
 // ------------------------------------------------------------ parsing

@@ -3,7 +3,7 @@
 #include <cctype>
 #include <cmath>
 #include <ctime>
-#include <regex>
+#include <cstring>
 
 #include "device.h"
 #include "errors.h"
@@ -18,9 +18,14 @@ std::string get_date_time() {
 }
 
 std::size_t from_readable_memory_string(std::string memory) {
-  memory = std::regex_replace(memory, std::regex("[^)(\\s\\ta-zA-Z0-9_.,-]"), "");
+  // white space and what no memory size has in it are dropped
   memory.erase(std::remove_if(memory.begin(), memory.end(),
-                              [](unsigned char c) { return std::isspace(c); }),
+                              [](unsigned char c) {
+                                const bool kept = (c >= 'a' && c <= 'z') || (c >= 'A' && c <= 'Z') ||
+                                                  (c >= '0' && c <= '9') ||
+                                                  (c != 0 && std::strchr(")(_.,-", c));
+                                return !kept;
+                              }),
                memory.end());
   for (auto& c : memory) c = char(std::toupper(static_cast<unsigned char>(c)));
   const std::size_t digits_end = std::min(memory.find_first_not_of("0123456789"), memory.size());

@@ -60,6 +60,25 @@ std::string get_output_states(const QflexInput* input,
 
 namespace {
 
+// Size of the tensor that a time line's product leaves: the indices that
+// only one tensor of the line has.
+std::size_t open_size(const std::vector<Tensor>& line) {
+  std::vector<std::pair<const std::string*, std::size_t>> open;
+  for (const auto& t : line)
+    for (std::size_t a = 0; a < t.get_indices().size(); ++a) {
+      const std::string& index = t.get_indices()[a];
+      auto it = std::find_if(open.begin(), open.end(), [&](const auto& o) { return *o.first == index; });
+      if (it != open.end())
+        open.erase(it);
+      else
+        open.emplace_back(&index, t.get_dimensions()[a]);
+    }
+  std::size_t size = 1;
+  for (const auto& o : open) size *= o.second;
+  return size;
+}
+
+
 // Ordering, output strings and the flattened 2D grid of an input (the part
 // of EvaluateCircuit before ContractGrid).
 void build_network(QflexInput* input, std::list<ContractionOperation>* ordering,
@@ -109,17 +128,7 @@ void build_network(QflexInput* input, std::list<ContractionOperation>* ordering,
     std::size_t max_size = 1;
     for (auto& row : tensor_grid_3D)
       for (auto& line : row) {
-        std::unordered_map<std::string, std::size_t> index_dim;
-        for (const auto& t : line)
-          for (const auto& [index, dim] : t.get_index_to_dimension()) {
-            if (index_dim.count(index))
-              index_dim.erase(index);
-            else
-              index_dim[index] = dim;
-          }
-        std::size_t s = 1;
-        for (const auto& p : index_dim) s *= p.second;
-        max_size = std::max(max_size, s);
+        max_size = std::max(max_size, open_size(line));
         // intermediate products along the time line can be larger
         std::size_t run = 1;
         for (const auto& t : line) run = std::max(run, t.size());
@@ -258,17 +267,7 @@ std::vector<std::pair<std::string, std::complex<double>>> EvaluateCircuitStates(
     std::size_t site_max = 1;
     for (auto& row : grid3D)
       for (auto& line : row) {
-        std::unordered_map<std::string, std::size_t> index_dim;
-        for (const auto& t : line)
-          for (const auto& [index, dim] : t.get_index_to_dimension()) {
-            if (index_dim.count(index))
-              index_dim.erase(index);
-            else
-              index_dim[index] = dim;
-          }
-        std::size_t sz = 1;
-        for (const auto& kv : index_dim) sz *= kv.second;
-        site_max = std::max(site_max, sz);
+        site_max = std::max(site_max, open_size(line));
       }
     s_type* scratch_2D = device_alloc(std::max(max_size, site_max) * 2);
     try {

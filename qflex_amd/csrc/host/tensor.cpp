@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <iostream>
+#include <mutex>
 #include <numeric>
 
 #include "device.h"
@@ -39,9 +40,18 @@ void Tensor::_init(const std::vector<std::string>& indices,
   }
   _indices = indices;
   _dimensions = dimensions;
+  generate_index_to_dimension();
+}
+
+void Tensor::_make_map() const {
+  if (!_map_pending.load(std::memory_order_acquire)) return;
+  static std::mutex several_readers;
+  const std::lock_guard<std::mutex> lock(several_readers);
+  if (!_map_pending.load(std::memory_order_relaxed)) return;
   _index_to_dimension.clear();
-  for (std::size_t i = 0; i < _dimensions.size(); ++i)
-    _index_to_dimension[indices[i]] = dimensions[i];
+  for (std::size_t i = 0; i < _indices.size(); ++i)
+    _index_to_dimension[_indices[i]] = _dimensions[i];
+  _map_pending.store(false, std::memory_order_release);
 }
 
 void Tensor::_clear() {
@@ -78,6 +88,7 @@ void Tensor::_move(Tensor&& other) noexcept {
   _indices = std::move(other._indices);
   _dimensions = std::move(other._dimensions);
   _index_to_dimension = std::move(other._index_to_dimension);
+  _map_pending = other._map_pending.load();
   _data = other._data;
   _capacity = other._capacity;
   other._data = nullptr;
@@ -151,7 +162,10 @@ const Tensor& Tensor::operator=(Tensor&& other) {
 
 const std::vector<std::string>& Tensor::get_indices() const { return _indices; }
 
-void Tensor::set_indices(const std::vector<std::string>& indices) { _indices = indices; }
+void Tensor::set_indices(const std::vector<std::string>& indices) {
+  _make_map();  // (the map stays that of the old indices)
+  _indices = indices;
+}
 
 const std::vector<std::size_t>& Tensor::get_dimensions() const { return _dimensions; }
 
@@ -165,16 +179,19 @@ void Tensor::set_dimensions(const std::vector<std::size_t>& dimensions) {
                       ".");
     }
   }
+  _make_map();
   _dimensions = dimensions;
 }
 
 void Tensor::set_indices_and_dimensions(const std::vector<std::string>& indices,
                                         const std::vector<std::size_t>& dimensions) {
-  try {
-    set_dimensions(dimensions);
-  } catch (const std::string& err_msg) {
-    throw ERROR_MSG("Failed to call set_dimensions(). Error:\n\t[", err_msg, "]");
-  }
+  std::size_t total_dim = 1;
+  for (auto d : dimensions) total_dim *= d;
+  if (indices.size() != dimensions.size() || (_data && capacity() < total_dim)) try {
+      set_dimensions(dimensions);
+    } catch (const std::string& err_msg) {
+      throw ERROR_MSG("Failed to call set_dimensions(). Error:\n\t[", err_msg, "]");
+    }
   try {
     _init(indices, dimensions);
   } catch (const std::string& err_msg) {
@@ -183,13 +200,14 @@ void Tensor::set_indices_and_dimensions(const std::vector<std::string>& indices,
 }
 
 const std::unordered_map<std::string, std::size_t>& Tensor::get_index_to_dimension() const {
+  _make_map();
   return _index_to_dimension;
 }
 
-void Tensor::generate_index_to_dimension() {
-  _index_to_dimension.clear();
-  for (std::size_t i = 0; i < _indices.size(); ++i)
-    _index_to_dimension[_indices[i]] = _dimensions[i];
+void Tensor::generate_index_to_dimension() { _map_pending = true; }
+
+std::size_t Tensor::index_dimension(std::size_t position) const {
+  return _map_pending ? _dimensions[position] : _index_to_dimension.at(_indices[position]);
 }
 
 std::size_t Tensor::size() const {
@@ -252,6 +270,7 @@ void Tensor::rename_index(std::string old_name, std::string new_name) {
   if (it == _indices.end()) throw ERROR_MSG("old_name: ", old_name, ", has to be a valid index.");
   if (std::find(_indices.begin(), _indices.end(), new_name) != _indices.end())
     throw ERROR_MSG("new_name: ", new_name, ", cannot be an existing index.");
+  _make_map();
   *it = new_name;
   _index_to_dimension[new_name] = _index_to_dimension[old_name];
   _index_to_dimension.erase(old_name);
@@ -270,6 +289,7 @@ void Tensor::bundle(std::vector<std::string> indices_to_bundle, std::string bund
                     " must be in its original order: ", _string_vector_to_string(original_order),
                     ".");
   }
+  _make_map();
   std::size_t bundled_dim = 1;
   for (const auto& idx : indices_to_bundle) {
     bundled_dim *= _index_to_dimension[idx];
@@ -320,6 +340,7 @@ void Tensor::reorder(std::vector<std::string> new_ordering, s_type* scratch_copy
               << std::endl;
     return;
   }
+  if (new_ordering == _indices) return;
   if (!_vector_s_in_vector_s(new_ordering, _indices) ||
       !_vector_s_in_vector_s(_indices, new_ordering) ||
       new_ordering.size() != _indices.size()) {
@@ -327,11 +348,11 @@ void Tensor::reorder(std::vector<std::string> new_ordering, s_type* scratch_copy
                     " must be a reordering of current indices: ",
                     _string_vector_to_string(_indices), ".");
   }
-  if (new_ordering == _indices) return;
   // The permutation goes into a fresh arena buffer of the same capacity,
   // which replaces _data (the reference permutes into scratch_copy and
   // copies back; the copy is saved here).  The old buffer returns to the
   // arena; work on the stream that reads it is ordered before any reuse.
+  _make_map();
   s_type* fresh = device_alloc(_capacity);
   device_reorder(_data, fresh, _indices, _dimensions, new_ordering);
   device_free(_data);
@@ -410,15 +431,32 @@ ProductShape prepare_multiply(Tensor& A, Tensor& B, Tensor& C, s_type* scratch_c
   if (B.data() == C.data())
     throw ERROR_MSG("B and C cannot be the same tensor: ", C.tensor_to_string());
 
-  std::vector<std::string> left = _vector_subtraction(A.get_indices(), B.get_indices());
-  std::vector<std::string> right = _vector_subtraction(B.get_indices(), A.get_indices());
-  std::vector<std::string> common = _vector_intersection(A.get_indices(), B.get_indices());
+  // Positions, not copies of the names: of A's left and common indices, and
+  // of B's common (in A's order) and right ones.
+  const auto& ai = A.get_indices();
+  const auto& bi = B.get_indices();
+  std::vector<std::size_t> a_order, a_common, b_order, right;
+  std::vector<char> b_shared(bi.size(), 0);
+  for (auto* v : {&a_order, &a_common, &b_order, &right}) v->reserve(ai.size() + bi.size());
+  for (std::size_t i = 0; i < ai.size(); ++i) {
+    const std::size_t j = std::size_t(std::find(bi.begin(), bi.end(), ai[i]) - bi.begin());
+    if (j == bi.size()) {
+      a_order.push_back(i);
+    } else {
+      a_common.push_back(i);
+      b_order.push_back(j);
+      b_shared[j] = 1;
+    }
+  }
+  const std::size_t n_left = a_order.size();
+  for (std::size_t j = 0; j < bi.size(); ++j)
+    if (!b_shared[j]) right.push_back(j);
   ProductShape p;
-  for (const auto& i : left) p.left_dim *= A.get_index_to_dimension().at(i);
-  for (const auto& i : right) p.right_dim *= B.get_index_to_dimension().at(i);
-  for (std::size_t i = 0; i < common.size(); ++i) {
-    std::size_t a_dim = A.get_index_to_dimension().at(common[i]);
-    std::size_t b_dim = B.get_index_to_dimension().at(common[i]);
+  for (std::size_t i : a_order) p.left_dim *= A.index_dimension(i);
+  for (std::size_t j : right) p.right_dim *= B.index_dimension(j);
+  for (std::size_t i = 0; i < a_common.size(); ++i) {
+    const std::size_t a_dim = A.index_dimension(a_common[i]);
+    const std::size_t b_dim = B.index_dimension(b_order[i]);
     if (a_dim != b_dim) {
       throw ERROR_MSG("Common indices must have matching dimensions, but at index: ", i,
                       ", the dimensions are A: ", a_dim, ", B: ", b_dim, ".");
@@ -429,32 +467,37 @@ ProductShape prepare_multiply(Tensor& A, Tensor& B, Tensor& C, s_type* scratch_c
     throw ERROR_MSG("C: ", C.capacity(), " doesn't have enough space for the product of A*B: ",
                     (p.left_dim * p.right_dim), ".");
   }
-  try {
-    A.reorder(_vector_union(left, common), scratch_copy);
-  } catch (const std::string& err_msg) {
-    throw ERROR_MSG("Failed to call reorder(). Error:\n\t[", err_msg, "]");
+  std::vector<std::string> C_indices;
+  std::vector<std::size_t> C_dimensions;
+  C_indices.reserve(n_left + right.size());
+  C_dimensions.reserve(n_left + right.size());
+  for (std::size_t i : a_order) {
+    C_indices.push_back(ai[i]);
+    C_dimensions.push_back(A.index_dimension(i));
   }
-  try {
-    B.reorder(_vector_union(common, right), scratch_copy);
-  } catch (const std::string& err_msg) {
-    throw ERROR_MSG("Failed to call reorder(). Error:\n\t[", err_msg, "]");
+  for (std::size_t j : right) {
+    C_indices.push_back(bi[j]);
+    C_dimensions.push_back(B.index_dimension(j));
   }
-  p.has_left = !left.empty();
+  a_order.insert(a_order.end(), a_common.begin(), a_common.end());
+  b_order.insert(b_order.end(), right.begin(), right.end());
+  for (auto [t, order] : {std::make_pair(&A, &a_order), std::make_pair(&B, &b_order)}) {
+    if (!order->empty() && std::is_sorted(order->begin(), order->end())) continue;
+    std::vector<std::string> names;
+    for (std::size_t i : *order) names.push_back(t->get_indices()[i]);
+    try {
+      t->reorder(names, scratch_copy);
+    } catch (const std::string& err_msg) {
+      throw ERROR_MSG("Failed to call reorder(). Error:\n\t[", err_msg, "]");
+    }
+  }
+  p.has_left = n_left > 0;
   p.has_right = !right.empty();
-
-  std::vector<std::string> C_indices = _vector_union(left, right);
-  std::vector<std::size_t> C_dimensions(C_indices.size());
-  for (std::size_t i = 0; i < left.size(); ++i)
-    C_dimensions[i] = A.get_index_to_dimension().at(left[i]);
-  for (std::size_t i = 0; i < right.size(); ++i)
-    C_dimensions[i + left.size()] = B.get_index_to_dimension().at(right[i]);
-  C.set_indices(C_indices);
   try {
-    C.set_dimensions(C_dimensions);
+    C.set_indices_and_dimensions(C_indices, C_dimensions);
   } catch (const std::string& err_msg) {
     throw ERROR_MSG("Failed to call set_dimensions(). Error:\n\t[", err_msg, "]");
   }
-  C.generate_index_to_dimension();
   return p;
 }
 
@@ -465,12 +508,14 @@ void multiply(Tensor& A, Tensor& B, Tensor& C, s_type* scratch_copy) {
 }
 
 std::size_t result_size(Tensor& A, Tensor& B) {
-  std::size_t left_dim = 1, right_dim = 1;
-  for (const auto& i : _vector_subtraction(A.get_indices(), B.get_indices()))
-    left_dim *= A.get_index_to_dimension().at(i);
-  for (const auto& i : _vector_subtraction(B.get_indices(), A.get_indices()))
-    right_dim *= B.get_index_to_dimension().at(i);
-  return left_dim * right_dim;
+  std::size_t size = 1;
+  auto others = [&size](const Tensor& x, const Tensor& y) {
+    for (std::size_t i = 0; i < x.get_indices().size(); ++i)
+      if (!_string_in_vector(x.get_indices()[i], y.get_indices())) size *= x.index_dimension(i);
+  };
+  others(A, B);
+  others(B, A);
+  return size;
 }
 
 void bundle_between(Tensor& A, Tensor& B, std::string bundled_index, s_type* scratch_copy) {

@@ -11,6 +11,7 @@
 #ifndef QFLEX_AMD_TENSOR_H_
 #define QFLEX_AMD_TENSOR_H_
 
+#include <atomic>
 #include <complex>
 #include <string>
 #include <unordered_map>
@@ -53,6 +54,8 @@ class Tensor {
                                   const std::vector<std::size_t>& dimensions);
   const std::unordered_map<std::string, std::size_t>& get_index_to_dimension() const;
   void generate_index_to_dimension();
+  // get_index_to_dimension().at(get_indices()[position]), without making the map.
+  std::size_t index_dimension(std::size_t position) const;
   std::size_t size() const;
   std::size_t capacity() const;
 
@@ -77,11 +80,15 @@ class Tensor {
  private:
   std::vector<std::string> _indices;
   std::vector<std::size_t> _dimensions;
-  std::unordered_map<std::string, std::size_t> _index_to_dimension;
+  // Made when it is first asked for (_map_pending), of the indices and
+  // dimensions that generate_index_to_dimension() saw; most tensors never are.
+  mutable std::unordered_map<std::string, std::size_t> _index_to_dimension;
+  mutable std::atomic<bool> _map_pending{false};
   s_type* _data{nullptr};
   std::size_t _capacity{0};
 
   void _init(const std::vector<std::string>& indices, const std::vector<std::size_t>& dimensions);
+  void _make_map() const;
   void _clear();
   void _copy(const Tensor& other);
   void _move(Tensor&& other) noexcept;

@@ -5,21 +5,34 @@
 
 #include <sstream>
 #include <string>
+#include <string_view>
+#include <type_traits>
 
 namespace qflex::utils {
 
+// x as an output stream writes it, behind `out` (no stream for strings and
+// whole numbers: index names are made of them, hundreds per circuit).
 template <typename T>
-std::string concat(const T& x) {
-  std::stringstream ss;
-  ss << x;
-  return ss.str();
+void append(std::string& out, const T& x) {
+  if constexpr (std::is_same_v<T, char> || std::is_same_v<T, signed char> ||
+                std::is_same_v<T, unsigned char>) {
+    out.push_back(char(x));
+  } else if constexpr (std::is_convertible_v<const T&, std::string_view>) {
+    out.append(std::string_view(x));
+  } else if constexpr (std::is_integral_v<T>) {
+    out += std::to_string(x);
+  } else {
+    std::ostringstream ss;
+    ss << x;
+    out += ss.str();
+  }
 }
 
-template <typename T, typename... Q>
-std::string concat(const T& x, const Q&... y) {
-  std::stringstream ss;
-  ss << x;
-  return ss.str() + concat(y...);
+template <typename... T>
+std::string concat(const T&... x) {
+  std::string out;
+  (append(out, x), ...);
+  return out;
 }
 
 // "Thu Aug 23 14:55:02 2001"
