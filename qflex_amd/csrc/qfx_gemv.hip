@@ -8,8 +8,8 @@
 // Reductions run in a fixed order (no atomics): results are deterministic.
 // Measured against one wave per row (N) and against blocks that walked all
 // columns of 4 to 16 rows, 64 at a time (T), a plain copy running at 5.0 TB/s:
-//   T 4096 x 4096 (134 MB)   144 -> 32.5 us     N 4096 x 4096    36.7 -> 24.4 us
-//   T 227 x 37463 (68 MB)    842 -> 18.6 us     N 81 x 12430     51 -> 4.3 us
+//   T 4096 x 4096 (134 MB)   144 -> 23.0 us     N 4096 x 4096    36.7 -> 24.4 us
+//   T 227 x 37463 (68 MB)    842 -> 16.2 us     N 81 x 12430     51 -> 4.3 us
 //   T 16384 x 256 (34 MB)    74 -> 12.2 us      N 1000000 x 4    122 -> 7.8 us
 //   T 1000000 x 4 (32 MB)    141 -> 12.6 us     N 20000 x 2048   73.4 -> 62.1 us
 #include <algorithm>
@@ -159,13 +159,16 @@ __global__ __launch_bounds__(1024) void gemv_n_block_kernel(const float2* __rest
 }
 
 // Sum over the groups of a block of one value per thread, in a fixed tree:
-// thread t belongs to group t / CL (CL threads each, G = 256 / CL groups; the
-// threads past G * CL take no part).  The result is in group 0.
+// thread t belongs to group t / CL (CL threads each, G = T / CL groups of the
+// block's T; the threads past G * CL take no part).  The result is in group 0.
+template <int T = 256>
 __device__ __forceinline__ float2 group_sum(float2 v, float2* red, int CL, int G) {
   const int t = threadIdx.x;
   red[t] = v;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {  // group g takes over group g + w
+  int w = T / 2;
+  while (w >= G && w > 1) w >>= 1;
+  for (; w > 0; w >>= 1) {  // group g takes over group g + w
     if (t < w * CL && t + w * CL < G * CL) red[t] = cadd(red[t], red[t + w * CL]);
     __syncthreads();
   }
@@ -175,18 +178,18 @@ __device__ __forceinline__ float2 group_sum(float2 v, float2* red, int CL, int G
 }
 
 // y[c] = sum_r x[r] A[r][c] (A is m x k, row-major).  Block (x, y): the
-// columns V * (CL x + lane) of the rows [rows_per * y, ...); its 256 threads
-// are G = 256 / CL row groups of CL column lanes, four rows in flight each.
+// columns V * (CL x + lane) of the rows [rows_per * y, ...); its T threads
+// are G = T / CL row groups of CL column lanes, four rows in flight each.
 // A narrow matrix takes all its columns as the lanes (CL = k / V), so that
 // the block reads whole rows one after the other.  One split over the rows
 // writes y itself, several write part[split][c].
-template <int V>
-__global__ __launch_bounds__(256) void gemv_t_kernel(const float2* __restrict__ A,
+template <int V, int T>
+__global__ __launch_bounds__(T) void gemv_t_kernel(const float2* __restrict__ A,
                                                      const float2* __restrict__ x,
                                                      float2* __restrict__ out, uint64_t M,
                                                      uint64_t K, uint64_t rows_per, int CL) {
-  __shared__ float2 red[256];
-  const int G = 256 / CL;
+  __shared__ float2 red[T];
+  const int G = T / CL;
   const int rg = threadIdx.x / CL, cl = threadIdx.x - rg * CL;
   const uint64_t c = (uint64_t(blockIdx.x) * CL + cl) * V;
   const uint64_t r0 = blockIdx.y * rows_per;
@@ -220,7 +223,7 @@ __global__ __launch_bounds__(256) void gemv_t_kernel(const float2* __restrict__ 
   }
 #pragma unroll
   for (int v = 0; v < V; ++v) {
-    const float2 t = group_sum(cadd(cadd(acc[0][v], acc[1][v]), cadd(acc[2][v], acc[3][v])), red,
+    const float2 t = group_sum<T>(cadd(cadd(acc[0][v], acc[1][v]), cadd(acc[2][v], acc[3][v])), red,
                                CL, G);
     if (rg == 0 && in) out[blockIdx.y * K + c + v] = t;
   }
@@ -332,6 +335,25 @@ int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
   const uint64_t rows_per = (m + nsplit - 1) / nsplit;
   nsplit = (m + rows_per - 1) / rows_per;
   if (tiles > 0x7fffffffULL) return qfx_set_error(QFX_ERR_UNSUPPORTED, "gemv: too many columns");
+  // Blocks of 1024 threads that take all rows of fewer columns save the
+  // partials and their launch.  Taken with at most 32 rows per thread in at
+  // least 128 blocks (4096 x 4096: 28.2 -> 23.0 us, 5.8 TB/s; 1024 x 65536 98.2 ->
+  // 87.6; 227 x 37463 18.8 -> 16.2; with 63 blocks 1000 x 4000 took 13.0 instead
+  // of 8.7) and otherwise with at most 8 (100 x 100: 6.3 -> 5.2; with 23,
+  // 1409 x 17 took 8.1 instead of 6.2).  8-byte loads of many rows want the
+  // widest blocks (2047 x 8191: 37.8 with 16 columns, 27.6 split).
+  for (uint64_t cl = units <= 64 ? units : 64; nsplit > 1 && cl > 0; cl /= 2) {
+    const uint64_t cols = (units + cl - 1) / cl, rows = (m * cl + 1023) / 1024;
+    const bool few = rows <= 8 && (cl == units || cl * V >= 16);
+    const bool many = rows <= 32 && cols >= 128 && cl >= (V == 2 ? 8 : 64);
+    if (m > 65536 || (!few && !many)) continue;
+    if (V == 2)
+      gemv_t_kernel<2, 1024><<<unsigned(cols), 1024, 0, ctx->stream>>>(A, x, y, m, k, m, int(cl));
+    else
+      gemv_t_kernel<1, 1024><<<unsigned(cols), 1024, 0, ctx->stream>>>(A, x, y, m, k, m, int(cl));
+    QFX_HIP(hipGetLastError());
+    return QFX_OK;
+  }
   float2* out = y;
   if (nsplit > 1) {
     void* ws = nullptr;
@@ -341,9 +363,9 @@ int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
   }
   const dim3 g{unsigned(tiles), unsigned(nsplit), 1};
   if (V == 2)
-    gemv_t_kernel<2><<<g, 256, 0, ctx->stream>>>(A, x, out, m, k, rows_per, CL);
+    gemv_t_kernel<2, 256><<<g, 256, 0, ctx->stream>>>(A, x, out, m, k, rows_per, CL);
   else
-    gemv_t_kernel<1><<<g, 256, 0, ctx->stream>>>(A, x, out, m, k, rows_per, CL);
+    gemv_t_kernel<1, 256><<<g, 256, 0, ctx->stream>>>(A, x, out, m, k, rows_per, CL);
   if (nsplit > 1) launch_sum(ctx->stream, out, y, nsplit, k);
   QFX_HIP(hipGetLastError());
   return QFX_OK;

@@ -447,3 +447,28 @@ def test_staged_upload_into_freed_block_then_reused(ctx):
     ctx.zero(c)
     assert np.all(ctx.download(c, np.uint64, (256,)) == 0)
     c.free()
+
+
+# x A in blocks of 1024 threads that take all rows: edges of the rows per
+# thread (8, 32), of the column lanes and of the 128 blocks, odd k and 8-byte
+# operands.  Whole numbers: every order of the sums is exact.
+@pytest.mark.parametrize("m,k,off", [(33, 100, 0), (100, 101, 0), (300, 50, 8), (1024, 16, 0),
+                                     (1025, 16, 0), (127, 1000, 0), (1000, 1000, 0),
+                                     (512, 16384, 0), (513, 16382, 0), (500, 8193, 0),
+                                     (2048, 4096, 0), (4097, 4096, 0), (260, 33000, 8)])
+def test_cgemv_t_all_rows_in_a_block_exact(ctx, m, k, off):
+    rng = np.random.default_rng(m + k)
+    a = (rng.integers(-3, 4, (m, k)) + 1j * rng.integers(-3, 4, (m, k))).astype(np.complex64)
+    x = (rng.integers(-3, 4, m) + 1j * rng.integers(-3, 4, m)).astype(np.complex64)
+    A = ctx.upload(np.concatenate([np.zeros(off // 8), a.ravel()]).astype(np.complex64))
+    X, Y = ctx.upload(x), ctx.alloc((k + 1) * 8)
+    ctx.zero(Y)
+
+    class At:
+        ptr = A.ptr + off
+    ctx.cgemv(1, m, k, At, X, Y)
+    got = ctx.download(Y, np.complex64, (k + 1,))
+    want = x.astype(np.complex128) @ a.astype(np.complex128)
+    assert np.array_equal(got[:-1], want.astype(np.complex64)) and got[-1] == 0
+    for buf in (A, X, Y):
+        buf.free()
