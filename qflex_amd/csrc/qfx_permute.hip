@@ -170,8 +170,10 @@ __global__ __launch_bounds__(BLOCK) void permute_pairs_kernel(const float2* __re
 // 29 M of 5 x 7 x 16 x 3 x 7 x 2 x 11 x 7 x 16 282, now 153.
 constexpr int kBoxAxes = 24;
 constexpr int kBoxMax = 2048;  // elements of a box
-// Below, one thread per element is faster, it has more to run at once: 0.63
-// and 0.74 M elements 5.6 and 6.3 us against 7.4 and 8.5; 1.4 M: 14 us with boxes, 20 without.
+// Below, two elements per thread without boxes is faster, it has more to run at
+// once; from 1.07 to 1.8 M elements either is, by up to twice, as the gathered
+// loads share lines or not (8 x 5 x 16 x 16 x 2 x 8 x 8: 8.1 us with boxes, 16.7
+// without; 8 x 7 x 16 x 4 x 7 x 7 x 8: 10.7 and 6.9).
 constexpr uint64_t kBoxesFrom = uint64_t(1) << 20;
 struct BoxParams {
   int size;
@@ -306,22 +308,57 @@ struct GenericParams {
   uint64_t in_stride_of_out[kMaxRank];  // input stride of output axis k
 };
 
-// T: an integer type that holds every element index (32 bits divide faster).
-template <typename T>
+// 2^31 elements and more.
 __global__ void permute_generic_kernel(const float2* __restrict__ src, float2* __restrict__ dst,
                                        GenericParams p) {
   uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
   for (; i < p.total; i += stride) {
-    T rem = T(i), off = 0;
+    uint64_t rem = i, off = 0;
     for (int k = p.rank - 1; k >= 0; --k) {
-      const T d = T(p.out_dims[k]);
-      const T q = rem / d;
-      off += (rem - q * d) * T(p.in_stride_of_out[k]);
+      const uint64_t d = p.out_dims[k], q = rem / d;
+      off += (rem - q * d) * p.in_stride_of_out[k];
       rem = q;
     }
     dst[i] = src[off];
   }
+}
+
+// Fewer than kBoxesFrom elements (at most 2^21), whose digits single precision
+// divides exactly: e + 1/2 is exact, 1 / d and the product are off by 2^-24 each,
+// together by less than 1 / (4 d), and (e + 1/2) / d is at least 1 / (2 d) from a
+// whole number.  Two elements per thread.  The integer divisions bounded it:
+// 0.74 M elements of 16 x 2 x 4 x 11 x 3 x 5 x 7 x 5 11.0 -> 8.5 us, 0.79 M of
+// 8 x 16 x 7 x 11 x 5 x 4 x 4 9.2 -> 7.3; below 2^19 a call is bound by its launch.
+static_assert(kBoxesFrom <= (uint64_t(1) << 21), "exact digits");
+struct SmallParams {
+  int rank;
+  uint32_t total;
+  uint32_t dim[kMaxRank], step[kMaxRank];  // from the innermost output axis; input strides
+  float inv[kMaxRank];
+};
+__global__ __launch_bounds__(256) void permute_small_kernel(const float2* __restrict__ src,
+                                                            float2* __restrict__ dst,
+                                                            SmallParams p) {
+  const uint32_t i = blockIdx.x * 512 + threadIdx.x;
+  uint32_t rem[2] = {i, i + 256}, off[2] = {0, 0};
+  for (int k = 0; k + 1 < p.rank; ++k) {
+    const uint32_t d = p.dim[k], step = p.step[k];
+    const float inv = p.inv[k];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const uint32_t q = uint32_t((float(rem[u]) + 0.5f) * inv);
+      off[u] += (rem[u] - q * d) * step;
+      rem[u] = q;
+    }
+  }
+  float2 v[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+    if (i + 256 * u < p.total) v[u] = src[off[u] + rem[u] * p.step[p.rank - 1]];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+    if (i + 256 * u < p.total) dst[i + 256 * u] = v[u];
 }
 
 // The box of a permutation of fused axes: dims in input order, perm[k] the
@@ -581,6 +618,20 @@ extern "C" int qfx_reorder_c64(qfx_context* ctx, const qfx_c64* src, qfx_c64* ds
       case 7: launch_boxes<7>(p, s2, d2, ctx->stream); break;
       default: launch_boxes<8>(p, s2, d2, ctx->stream); break;
     }
+  } else if (total < kBoxesFrom && r <= kMaxRank) {
+    SmallParams p{};
+    p.rank = r;
+    p.total = uint32_t(total);
+    std::vector<uint32_t> in_stride(r);
+    uint32_t st = 1;
+    for (int a = r - 1; a >= 0; st *= uint32_t(fdims[a]), --a) in_stride[a] = st;
+    for (int k = 0; k < r; ++k) {
+      const int a = fperm[r - 1 - k];
+      p.dim[k] = uint32_t(fdims[a]);
+      p.step[k] = in_stride[a];
+      p.inv[k] = 1.f / float(fdims[a]);
+    }
+    permute_small_kernel<<<unsigned((total + 511) / 512), 256, 0, ctx->stream>>>(s2, d2, p);
   } else {
     if (r > kMaxRank) return qfx_set_error(QFX_ERR_UNSUPPORTED, "rank too large");
     GenericParams p{};
@@ -597,10 +648,7 @@ extern "C" int qfx_reorder_c64(qfx_context* ctx, const qfx_c64* src, qfx_c64* ds
       p.in_stride_of_out[k] = in_stride[fperm[k]];
     }
     uint64_t g = std::min<uint64_t>((total + 255) / 256, 65536);
-    if (total < (uint64_t(1) << 31))
-      permute_generic_kernel<uint32_t><<<unsigned(g), 256, 0, ctx->stream>>>(s2, d2, p);
-    else
-      permute_generic_kernel<uint64_t><<<unsigned(g), 256, 0, ctx->stream>>>(s2, d2, p);
+    permute_generic_kernel<<<unsigned(g), 256, 0, ctx->stream>>>(s2, d2, p);
   }
   QFX_HIP(hipGetLastError());
   return QFX_OK;

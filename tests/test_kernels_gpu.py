@@ -472,3 +472,23 @@ def test_cgemv_t_all_rows_in_a_block_exact(ctx, m, k, off):
     assert np.array_equal(got[:-1], want.astype(np.complex64)) and got[-1] == 0
     for buf in (A, X, Y):
         buf.free()
+
+
+# One element per position: every index is its own value.  Edges of the two
+# elements per thread (512 per block), large and small divisors, the largest
+# size of the kernel and the first one past it.
+@pytest.mark.parametrize("dims,perm", [([3, 2], [1, 0]), ([7, 73], [1, 0]), ([3, 171], [1, 0]),
+                                       ([5, 11, 3, 31], [2, 0, 3, 1]), ([255, 4111], [1, 0]),
+                                       ([349525, 3], [1, 0]), ([3, 349525], [1, 0]),
+                                       ([3, 5, 7, 11, 13, 67], [5, 2, 4, 0, 3, 1]),
+                                       ([1025, 1023], [1, 0]), ([1023, 1027], [1, 0]),
+                                       ([3] * 12, [11, 0, 9, 2, 7, 4, 5, 6, 3, 8, 1, 10])])
+def test_reorder_small_odd_tensors_bit_exact(ctx, dims, perm):
+    x = np.arange(np.prod(dims), dtype=np.uint64).reshape(dims)
+    src, dst = ctx.upload(x), ctx.alloc(x.nbytes + 8)
+    ctx.zero(dst)
+    ctx.reorder(src, dst, dims, perm)
+    got = ctx.download(dst, np.uint64, (x.size + 1,))
+    assert np.array_equal(got[:-1], x.transpose(perm).ravel()) and got[-1] == 0
+    src.free()
+    dst.free()
