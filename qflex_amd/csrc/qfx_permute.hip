@@ -170,11 +170,14 @@ __global__ __launch_bounds__(BLOCK) void permute_pairs_kernel(const float2* __re
 // 29 M of 5 x 7 x 16 x 3 x 7 x 2 x 11 x 7 x 16 282, now 153.
 constexpr int kBoxAxes = 24;
 constexpr int kBoxMax = 2048;  // elements of a box
-// Below, two elements per thread without boxes is faster, it has more to run at
-// once; from 1.07 to 1.8 M elements either is, by up to twice, as the gathered
-// loads share lines or not (8 x 5 x 16 x 16 x 2 x 8 x 8: 8.1 us with boxes, 16.7
-// without; 8 x 7 x 16 x 4 x 7 x 7 x 8: 10.7 and 6.9).
-constexpr uint64_t kBoxesFrom = uint64_t(1) << 20;
+// Below kBoxesFrom, two elements per thread without boxes is faster, it has more
+// to run at once.  From there to kSmallUpTo it is where a wave's 64 gathered loads
+// share lines: of 40 tensors of 1.1 to 1.9 M elements, the ones that touch 6 to 18
+// lines were 1.0 to 1.6 times faster without boxes (8 x 7 x 16 x 4 x 7 x 7 x 8:
+// 10.7 -> 6.9 us), two with 28 lines 1.65 and 0.73 times, those with 32 to 64
+// lines 0.47 to 0.97 times.
+constexpr uint64_t kBoxesFrom = uint64_t(1) << 20, kSmallUpTo = uint64_t(1) << 21;
+constexpr int kSmallLines = 20;
 struct BoxParams {
   int size;
   int naxes;  // axes with more than one coordinate in a box
@@ -324,13 +327,12 @@ __global__ void permute_generic_kernel(const float2* __restrict__ src, float2* _
   }
 }
 
-// Fewer than kBoxesFrom elements (at most 2^21), whose digits single precision
+// At most kSmallUpTo = 2^21 elements, whose digits single precision
 // divides exactly: e + 1/2 is exact, 1 / d and the product are off by 2^-24 each,
 // together by less than 1 / (4 d), and (e + 1/2) / d is at least 1 / (2 d) from a
 // whole number.  Two elements per thread.  The integer divisions bounded it:
 // 0.74 M elements of 16 x 2 x 4 x 11 x 3 x 5 x 7 x 5 11.0 -> 8.5 us, 0.79 M of
 // 8 x 16 x 7 x 11 x 5 x 4 x 4 9.2 -> 7.3; below 2^19 a call is bound by its launch.
-static_assert(kBoxesFrom <= (uint64_t(1) << 21), "exact digits");
 struct SmallParams {
   int rank;
   uint32_t total;
@@ -394,6 +396,27 @@ void choose_box(const std::vector<uint64_t>& dims, const std::vector<int>& perm,
     block = b;
     if (size >= enough) break;
   }
+}
+
+// Lines of 128 bytes that 64 consecutive output elements, from the middle of
+// the tensor on, are read from.
+int lines_of_a_wave(const std::vector<uint64_t>& dims, const std::vector<int>& perm,
+                    uint64_t total) {
+  const int r = int(dims.size());
+  std::vector<uint64_t> stride(r);
+  uint64_t st = 1;
+  for (int a = r - 1; a >= 0; st *= dims[a], --a) stride[a] = st;
+  uint64_t line[64];
+  for (int i = 0; i < 64; ++i) {
+    uint64_t e = total / 2 / 64 * 64 + i, off = 0;
+    for (int k = r - 1; k >= 0 && e > 0; --k) {
+      off += e % dims[perm[k]] * stride[perm[k]];
+      e /= dims[perm[k]];
+    }
+    line[i] = off / 16;
+  }
+  std::sort(line, line + 64);
+  return int(std::unique(line, line + 64) - line);
 }
 
 template <int PER>
@@ -556,7 +579,8 @@ extern "C" int qfx_reorder_c64(qfx_context* ctx, const qfx_c64* src, qfx_c64* ds
       case 2: launch_bits<2, 4>(p, s2, d2, ctx->stream); break;
       default: launch_bits<1, 2>(p, s2, d2, ctx->stream); break;
     }
-  } else if (total >= kBoxesFrom && total < (uint64_t(1) << 31) && r <= kBoxAxes) {
+  } else if (total >= kBoxesFrom && total < (uint64_t(1) << 31) && r <= kBoxAxes &&
+             (total > kSmallUpTo || lines_of_a_wave(fdims, fperm, total) > kSmallLines)) {
     std::vector<uint64_t> block(r, 1), in_stride(r), out_stride(r);
     choose_box(fdims, fperm, total, block);
     uint64_t st = 1;
@@ -618,7 +642,7 @@ extern "C" int qfx_reorder_c64(qfx_context* ctx, const qfx_c64* src, qfx_c64* ds
       case 7: launch_boxes<7>(p, s2, d2, ctx->stream); break;
       default: launch_boxes<8>(p, s2, d2, ctx->stream); break;
     }
-  } else if (total < kBoxesFrom && r <= kMaxRank) {
+  } else if (total <= kSmallUpTo && r <= kMaxRank) {
     SmallParams p{};
     p.rank = r;
     p.total = uint32_t(total);

@@ -482,6 +482,9 @@ def test_cgemv_t_all_rows_in_a_block_exact(ctx, m, k, off):
                                        ([349525, 3], [1, 0]), ([3, 349525], [1, 0]),
                                        ([3, 5, 7, 11, 13, 67], [5, 2, 4, 0, 3, 1]),
                                        ([1025, 1023], [1, 0]), ([1023, 1027], [1, 0]),
+                                       ([2, 3, 349525], [1, 0, 2]), ([3, 699050], [1, 0]),
+                                       ([149797, 2, 7], [1, 0, 2]), ([7, 2, 149797], [1, 2, 0]),
+                                       ([3, 5, 139810], [1, 0, 2]),
                                        ([3] * 12, [11, 0, 9, 2, 7, 4, 5, 6, 3, 8, 1, 10])])
 def test_reorder_small_odd_tensors_bit_exact(ctx, dims, perm):
     x = np.arange(np.prod(dims), dtype=np.uint64).reshape(dims)
