@@ -1011,7 +1011,14 @@ __global__ __launch_bounds__(64 * WM * WN) void cgemm_split_big_kernel(
   // Column tiles vary fastest in dispatch order (the grid's x counts row
   // tiles): 2-4% faster than row tiles fastest on the 65536-131072 x 256-512
   // products, the same on 4096^3; the tile computation is unchanged.
-  const unsigned L = blockIdx.x + gridDim.x * blockIdx.y;
+  // The 128 x 64 tile, and the odd large ones of up to 8 columns of tiles, give
+  // each XCD a contiguous range of them, so that an L2 fetches a row panel of A
+  // once (26201 x 225 x 53 52.1 -> 50.6 us, 9001 x 701 x 2001 366 -> 356, 6145 x 515 x
+  // 333 52.4 -> 51.5; 3000 x 3001 x 1000 288 -> 290); the even large tile gained
+  // nothing (65536 x 256 x 256 BF16x3 183 -> 186).
+  const unsigned at = blockIdx.x + gridDim.x * blockIdx.y;
+  const unsigned L =
+      WM * WN == 4 || (ODD && gridDim.y <= 8) ? unsigned(xcd_tile(at, gridDim.x * gridDim.y)) : at;
   const unsigned tn = L % gridDim.y, tm = L / gridDim.y;
   split_big_tile<MODE, WM, WN, J, AM, I, WIDE, false, ODD>(
       A, B, C, M, N, K, amax, a_rows, a_cols, b_rows, b_cols, cmax ? cmax + L : nullptr,
@@ -1027,7 +1034,10 @@ __global__ __launch_bounds__(64 * WM * WN) void cgemm_split_chain_kernel(
     int N, int K, AmaxRef amax, qfx_index_map a_rows, qfx_index_map a_cols,
     qfx_index_map b_rows, qfx_index_map b_cols, float* __restrict__ cmax, unsigned ntiles,
     unsigned gy) {
-  const unsigned L = blockIdx.x;
+  // Up to 8 column tiles: an XCD's blocks take neighbouring tiles at a time, the
+  // ones that share a row panel of A (131072 x 256 x 256 262 -> 256 us, 262144 x 64
+  // x 64 89.4 -> 85.6; with 16 column tiles 8192 x 4096 x 128 took 133 instead of 131).
+  const unsigned L = gy <= 8 ? unsigned(xcd_tile(blockIdx.x, gridDim.x)) : blockIdx.x;
   split_big_tile<MODE, WM, WN, J, AM, I, false, true>(
       A, B, C, M, N, K, amax, a_rows, a_cols, b_rows, b_cols, cmax, int(L / gy) * 32 * I * WM,
       int(L % gy) * 16 * J * WN, L, gridDim.x, ntiles, gy);

@@ -272,14 +272,6 @@ __device__ __forceinline__ void f32_tile(const float2* __restrict__ A,
   }
 }
 
-// Tile of block b of `tiles`: each of the 8 XCDs (which take blocks in turn)
-// gets a contiguous range of them, so that the column tiles that share rows
-// of A read them through one L2.
-__device__ __forceinline__ uint64_t xcd_tile(uint64_t b, uint64_t tiles) {
-  const uint64_t q = tiles / 8, r = tiles % 8, x = b % 8;
-  return x * q + (x < r ? x : r) + b / 8;
-}
-
 template <class T, int LOAD>
 __global__ __launch_bounds__(256, 2) void cgemm_f32_kernel(
     const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C, int M,

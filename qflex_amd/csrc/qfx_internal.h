@@ -174,6 +174,14 @@ __device__ __forceinline__ int group_entry(const uint64_t* first, size_t bytes, 
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
+// Tile of block b of `tiles`: each of the 8 XCDs (which take blocks in turn)
+// gets a contiguous range of them, so that the column tiles that share rows
+// of A read them through one L2.
+__device__ __forceinline__ uint64_t xcd_tile(uint64_t b, uint64_t tiles) {
+  const uint64_t q = tiles / 8, r = tiles % 8, x = b % 8;
+  return x * q + (x < r ? x : r) + b / 8;
+}
+
 // A short problem list as a kernel argument: no workspace and no upload launch
 // before the grouped one (5 us of a call).
 constexpr int kArgProblems = 32;
