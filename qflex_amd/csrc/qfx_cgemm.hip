@@ -1072,12 +1072,14 @@ __global__ __launch_bounds__(256) void amax_grouped_kernel(const GroupTile* __re
 
 // Persistent grouped launch: the blocks walk the tiles of all problems
 // (problems of any shape, tiles numbered problem by problem), each block
-// taking every gridDim.x-th tile.
+// taking every gridDim.x-th tile; the blocks of an XCD take neighbouring ones,
+// which share B or A in its L2 (192 products of 512 x 128 x 64 48.6 -> 45.6 us, 150
+// of 300 x 99 x 101 57.8 -> 52.0, 200 of 700 x 250 x 32 143 -> 132).
 template <int MODE, int WM, int WN, int J, bool ODD>
 __global__ __launch_bounds__(64 * WM * WN) void cgemm_split_grouped_kernel(const GroupTile* __restrict__ probs,
                                                                   int count, uint64_t total) {
   const qfx_index_map none{};
-  for (uint64_t t = blockIdx.x; t < total; t += gridDim.x) {
+  for (uint64_t t = xcd_tile(blockIdx.x, gridDim.x); t < total; t += gridDim.x) {
     const GroupTile g =
         probs[group_entry(&probs[0].first_tile, sizeof(GroupTile), count, t)];
     const uint64_t local = t - g.first_tile;
