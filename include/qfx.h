@@ -55,9 +55,10 @@ enum qfx_precision {
                                 split into FP16 hi + lo; hi*hi + hi*lo + lo*hi, FP32 acc */
   QFX_PREC_FP8 = 5           /* low fidelity: A and the real 2x2 expansion of B as OCP
                                 E4M3, one power-of-two scale per 128x128 tile (max scaled
-                                value < 256), FP32 acc.  Small products run as in the other
-                                precisions (exact FP32 for k <= 16 or m*n <= 2^16); the
-                                rest below m 128, n 64, k 64 run as QFX_PREC_FP32 */
+                                value < 256), FP32 acc.  Small products run in FP32 as in the
+                                other precisions (k <= 16; m*n <= 2^16 with k a multiple of 16
+                                up to 4096; m, n <= 8 with k >= 1024); the rest below m 128,
+                                n 64, k 64 run as QFX_PREC_FP32 */
 };
 
 /* Kernel classes reported by qfx_profile_read. */

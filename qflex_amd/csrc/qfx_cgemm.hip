@@ -2062,7 +2062,8 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
     QFX_HIP(hipGetLastError());
     return QFX_OK;
   }
-  if (precision == QFX_PREC_FP8 && qfx_fp8_applies(m, n, k)) {
+  // (small outputs are FP32 in every precision)
+  if (precision == QFX_PREC_FP8 && !small_output(m, n, k) && qfx_fp8_applies(m, n, k)) {
     QfxLaunchScope scope(ctx, QFX_K_CGEMM, bytes, flops);
     return qfx_cgemm_fp8(ctx, A2, B2, C2, m, n, k, nullptr);
   }
@@ -2303,6 +2304,13 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
     QFX_HIP(hipGetLastError());
     return QFX_OK;
   }
+  if (precision != QFX_PREC_FP32_EXACT && small_output(m, n, k)) {
+    QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
+    const qfx_index_map maps[4] = {*a_rows, *a_cols, *b_rows, *b_cols};
+    return qfx_launch_f32(ctx, A2, B2, C2, m, n, k, maps,
+                          contiguous(*a_rows, 1) && !contiguous(*a_cols, 3),
+                          contiguous(*b_rows, 1) && !contiguous(*b_cols, 1), true);
+  }
   if (precision == QFX_PREC_FP8) {
     // The quantize kernels read the operands through the maps: every form.
     if (!qfx_fp8_applies(m, n, k))
@@ -2310,13 +2318,6 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
     QfxLaunchScope scope(ctx, QFX_K_CGEMM, bytes, flops);
     const qfx_index_map maps[4] = {*a_rows, *a_cols, *b_rows, *b_cols};
     return qfx_cgemm_fp8(ctx, A2, B2, C2, m, n, k, maps);
-  }
-  if (precision != QFX_PREC_FP32_EXACT && small_output(m, n, k)) {
-    QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
-    const qfx_index_map maps[4] = {*a_rows, *a_cols, *b_rows, *b_cols};
-    return qfx_launch_f32(ctx, A2, B2, C2, m, n, k, maps,
-                          contiguous(*a_rows, 1) && !contiguous(*a_cols, 3),
-                          contiguous(*b_rows, 1) && !contiguous(*b_cols, 1), true);
   }
   const BigLayout layout =
       (split_precision(precision) && big_mapped_spans_fit(*a_rows, *a_cols, *b_rows, *b_cols, m, n, k) && k >= 8 &&

@@ -158,3 +158,43 @@ def test_fp8_mapped_declines_small_k(ctx):
     assert not ctx.cgemm_mapped(capi.FP8, A, maps[0], maps[1], B, maps[2], maps[3], C)
     for buf in (A, B, C):
         buf.free()
+
+
+# At most 2^16 outputs over 16 < k <= 4096, k a multiple of 16: FP32, also
+# where the shape would fill the FP8 tiles.  An FP32 sum of 2 k products is
+# off by less than 2^-24 sqrt(2 k) in the norm; E4M3 costs a few 1e-2.
+def fp32_sum_bound(k):
+    return 2.0 ** -24 * np.sqrt(2.0 * k)
+
+
+@pytest.mark.parametrize("shape", [(256, 256, 128), (128, 64, 64), (1024, 64, 80), (128, 512, 4096),
+                                   (128, 70, 4096), (655, 100, 64)])
+def test_fp8_small_outputs_run_as_fp32(ctx, shape):
+    m, n, k = shape
+    rng = np.random.default_rng(m + n + k)
+    a, b = rand_c(rng, (m, k)), rand_c(rng, (k, n))
+    exact = a.astype(np.complex128) @ b.astype(np.complex128)
+    assert relerr(gpu_cgemm(ctx, a, b), exact) < fp32_sum_bound(k)
+
+
+# The first two fill the FP8 tiles, the others are below them.
+@pytest.mark.parametrize("left,common,right", [([16, 16], [16, 8], [16, 16]), ([8, 16], [4, 16], [4, 16]),
+                                               ([4, 16], [2, 16], [4, 16]), ([4, 16], [4, 16], [16, 16]),
+                                               ([16, 16], [16, 16], [2, 16])])
+@pytest.mark.parametrize("inner", ["left", "common"])
+def test_fp8_mapped_small_outputs_run_as_fp32(ctx, left, common, right, inner):
+    a_dims, a_left, a_common, b_dims, b_common, b_right = make_case(left, common, right, inner,
+                                                                    "right", seed=3)
+    rng = np.random.default_rng(4)
+    a, b = rand_c(rng, a_dims), rand_c(rng, b_dims)
+    m, k, n = (int(np.prod(x)) for x in (left, common, right))
+    A, B, C = ctx.upload(a), ctx.upload(b), ctx.alloc(m * n * 8)
+    assert ctx.cgemm_mapped(capi.FP8, A, capi.index_map(a_dims, a_left),
+                            capi.index_map(a_dims, a_common), B, capi.index_map(b_dims, b_common),
+                            capi.index_map(b_dims, b_right), C)
+    got = ctx.download(C, np.complex64, (m, n))
+    exact = (a.transpose(a_left + a_common).reshape(m, k).astype(np.complex128)
+             @ b.transpose(b_common + b_right).reshape(k, n).astype(np.complex128))
+    assert relerr(got, exact) < fp32_sum_bound(k)
+    for buf in (A, B, C):
+        buf.free()
