@@ -2505,6 +2505,14 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
     return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: invalid problem list");
   if (precision < QFX_PREC_FP32 || precision > QFX_PREC_FP8)
     return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: unknown precision");
+  // Every route's operands are checked here, before the first launch.
+  for (int i = 0; i < count; ++i) {
+    const qfx_gemm_desc& d = descs[i];
+    if (d.m == 0 || d.n == 0 || d.k == 0 || !d.A || !d.B || !d.C) continue;  // qfx_cgemm_c64's cases
+    QFX_EXTENT(ctx, d.A, 8.0 * double(d.m) * double(d.k), "qfx_cgemm_grouped_c64: A");
+    QFX_EXTENT(ctx, d.B, 8.0 * double(d.k) * double(d.n), "qfx_cgemm_grouped_c64: B");
+    QFX_EXTENT(ctx, d.C, 8.0 * double(d.m) * double(d.n), "qfx_cgemm_grouped_c64: C");
+  }
   const bool split = split_precision(precision);
   // One launch each for the problems of the large tiles, of the odd ones, of
   // the row kernel (k, n <= 16), of the other k <= 16 ones (both exact FP32 in
@@ -2540,9 +2548,6 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
                         (d.m > 8 || d.n > 8 || d.k < 1024) && precision != QFX_PREC_FP8 &&
                         f32_route(precision, d.m, d.n, d.k, false);
     if (full && (small || matrix)) {
-      QFX_EXTENT(ctx, d.A, 8.0 * double(d.m) * double(d.k), "qfx_cgemm_grouped_c64: A");
-      QFX_EXTENT(ctx, d.B, 8.0 * double(d.k) * double(d.n), "qfx_cgemm_grouped_c64: B");
-      QFX_EXTENT(ctx, d.C, 8.0 * double(d.m) * double(d.n), "qfx_cgemm_grouped_c64: C");
       (small ? smallk : f32).push_back(i);
       continue;
     }

@@ -214,3 +214,46 @@ def test_chained_mapped_tiles_bit_identical_to_single_tiles(ctx, a_inner, left, 
     assert np.array_equal(got.view(np.uint64), want.view(np.uint64)), a_inner
     for buf in (A, B, C, Am, Bm, G):
         buf.free()
+
+
+class At:
+    def __init__(self, buf, byte):
+        self.ptr = buf.ptr + byte
+
+
+# A product of every route: row kernel (a vector among them), k <= 16, FP32
+# tiles, FP32 alone, split, split of odd sizes, one by one.
+@pytest.mark.parametrize("operand", [0, 1, 2])
+@pytest.mark.parametrize("prec,shape", [(capi.FP32, (300, 16, 16)), (capi.SPLIT_FP16, (1, 8, 4)),
+                                        (capi.FP32, (64, 64, 16)), (capi.FP32, (33, 7, 35)),
+                                        (capi.FP32, (57, 104, 3384)),
+                                        (capi.SPLIT_FP16, (256, 128, 64)),
+                                        (capi.SPLIT_BF16X3, (256, 130, 66)),
+                                        (capi.SPLIT_FP16, (129, 65, 33)),
+                                        (capi.SPLIT_BF16, (200, 100, 35)),
+                                        (capi.FP32_EXACT, (20, 20, 20))])
+def test_grouped_refuses_operands_past_their_block(ctx, prec, shape, operand):
+    """An operand that ends 16 bytes past its arena block is refused by the
+    host, with nothing launched: a good product of the same call stays unrun."""
+    m, n, k = shape
+    rng = np.random.default_rng(sum(shape))
+    a = (rng.integers(-3, 4, (m, k)) + 1j * rng.integers(-3, 4, (m, k))).astype(np.complex64)
+    b = (rng.integers(-3, 4, (k, n)) + 1j * rng.integers(-3, 4, (k, n))).astype(np.complex64)
+    sizes = [8 * m * k, 8 * k * n, 8 * m * n]
+    # blocks of a power of two bytes are handed out as they are asked for
+    blocks = [ctx.alloc(max(256, 1 << (s - 1).bit_length())) for s in sizes]
+    ends = [At(buf, buf.nbytes - s) for buf, s in zip(blocks, sizes)]
+    ctx.upload_async(ends[0], a)
+    ctx.upload_async(ends[1], b)
+    ctx.zero(blocks[2])
+    ctx.cgemm_grouped(prec, [(m, n, k, *ends)])  # up to the last byte
+    want = (a.astype(np.complex128) @ b.astype(np.complex128)).astype(np.complex64)
+    assert np.array_equal(ctx.download(ends[2], np.complex64, (m, n)), want)
+    ctx.zero(blocks[2])
+    past = list(ends)
+    past[operand] = At(blocks[operand], blocks[operand].nbytes - sizes[operand] + 16)
+    with pytest.raises(capi.QfxError, match="qfx_cgemm_grouped_c64: " + "ABC"[operand]):
+        ctx.cgemm_grouped(prec, [(m, n, k, *ends), (m, n, k, *past)])
+    assert not ctx.download(blocks[2], np.uint8, (blocks[2].nbytes,)).any()
+    for buf in blocks:
+        buf.free()
