@@ -474,6 +474,9 @@ int qfx_launch_f32_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
   std::vector<std::vector<int>> by_tile(kTileC + 1);
   double alone_us = 0, group_us = 6, longest = 0;
   auto alone = [&](const qfx_gemm_desc& d) {
+    QfxLaunchScope scope(ctx, QFX_K_CGEMM,
+                         8.0 * (double(d.m) * d.k + double(d.k) * d.n + double(d.m) * d.n),
+                         8.0 * double(d.m) * double(d.n) * double(d.k));
     return qfx_launch_f32(ctx, reinterpret_cast<const float2*>(d.A),
                           reinterpret_cast<const float2*>(d.B), reinterpret_cast<float2*>(d.C),
                           d.m, d.n, d.k, nullptr, false, false, false);

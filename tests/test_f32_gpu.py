@@ -152,3 +152,22 @@ def test_grouped_products_off_the_large_tiles_exact(ctx, prec, times):
         assert got[-1] == 0, (m, n, k)
     for buf in bufs:
         buf.free()
+
+
+def test_grouped_products_run_alone_are_profiled(ctx):
+    """Products of a grouped call that the FP32 kernel takes one by one (long
+    k, or 512 tiles and more) count in the profile as single calls do."""
+    rng = np.random.default_rng(8)
+    shapes = [(57, 104, 3384), (40, 30, 20000), (8192, 1024, 32)]
+    problems = [(m, n, k, ctx.upload(whole(rng, (m, k))), ctx.upload(whole(rng, (k, n))),
+                 ctx.alloc(m * n * 8)) for m, n, k in shapes]
+    ctx.profile(True)
+    ctx.profile_reset()
+    ctx.cgemm_grouped(capi.FP32, problems)
+    got = ctx.profile_read()["cgemm"]
+    ctx.profile(False)
+    assert got["flops"] == sum(8.0 * m * n * k for m, n, k in shapes)
+    assert got["bytes"] == sum(8.0 * (m * k + k * n + m * n) for m, n, k in shapes)
+    for problem in problems:
+        for buf in problem[3:]:
+            buf.free()
