@@ -2305,7 +2305,7 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
     return QFX_OK;
   }
   if (precision != QFX_PREC_FP32_EXACT && small_output(m, n, k)) {
-    QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
+    QfxLaunchScope scope(ctx, QFX_K_CGEMM, bytes, flops);
     const qfx_index_map maps[4] = {*a_rows, *a_cols, *b_rows, *b_cols};
     return qfx_launch_f32(ctx, A2, B2, C2, m, n, k, maps,
                           contiguous(*a_rows, 1) && !contiguous(*a_cols, 3),

@@ -171,3 +171,20 @@ def test_grouped_products_run_alone_are_profiled(ctx):
     for problem in problems:
         for buf in problem[3:]:
             buf.free()
+
+
+def test_small_outputs_are_one_class_in_the_profile(ctx):
+    """The same matrix-core kernel reads them row-major and through index maps."""
+    m, n, k = 128, 64, 256
+    rng = np.random.default_rng(9)
+    A, B, C = ctx.upload(whole(rng, (m, k))), ctx.upload(whole(rng, (k, n))), ctx.alloc(m * n * 8)
+    maps = [capi.index_map(dims, [axis]) for dims in ([m, k], [k, n]) for axis in (0, 1)]
+    ctx.profile(True)
+    ctx.profile_reset()
+    ctx.cgemm(capi.FP32, m, n, k, A, B, C)
+    assert ctx.cgemm_mapped(capi.FP32, A, maps[0], maps[1], B, maps[2], maps[3], C)
+    prof = ctx.profile_read()
+    ctx.profile(False)
+    assert prof["cgemm"]["launches"] == 2 and prof["cgemm_small"]["launches"] == 0
+    for buf in (A, B, C):
+        buf.free()
