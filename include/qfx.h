@@ -276,8 +276,10 @@ int qfx_accumulate_batched_c128(qfx_context* ctx, const qfx_c64* src, uint64_t n
  * sequence with one launch, on the same buffers.  Meant for a sequence that
  * repeats with the same pointers, such as the contraction after the cuts of
  * one slice.  The device workspace is reserved at `workspace_bytes` before
- * recording and may not grow while recording; calls that synchronize or
- * allocate device memory from HIP (copies to or from the host,
+ * recording and may not grow while recording; the first qfx_graph_begin also
+ * takes 16 MiB of the arena, for the partial sums of FP32 products that need
+ * no reservation (recorded results have the eager calls' bits).  Calls that
+ * synchronize or allocate device memory from HIP (copies to or from the host,
  * qfx_synchronize, qfx_profile_*, an arena that must grow) fail while
  * recording, the tile autotuner times nothing, and profiling is off.  Zero
  * fills are kernels (no memset nodes).  No counterpart in the reference. */

@@ -439,17 +439,20 @@ bool qfx_f32_fits(uint64_t m, uint64_t n, uint64_t k) {
 
 int qfx_launch_f32(qfx_context* ctx, const float2* A, const float2* B, float2* C, uint64_t m,
                    uint64_t n, uint64_t k, const qfx_index_map* maps, bool a_mfast,
-                   bool b_kfast, bool needs_splits) {
-  F32Plan p = f32_plan(m, n, k);
-  const size_t bytes = p.splits > 1 ? size_t(p.splits) * m * n * sizeof(float2) : 0;
-  // A sequence being recorded cannot grow the workspace: one split then, or
-  // the refusal.
-  if (!needs_splits && ctx->capturing && !ctx->use_fixed_scratch && bytes > ctx->work_bytes) p.splits = 1;
+                   bool b_kfast, bool needs_reservation) {
+  const F32Plan p = f32_plan(m, n, k);
   float2* out = C;
   if (p.splits > 1) {
+    const size_t bytes = size_t(p.splits) * m * n * sizeof(float2);  // <= kFixedScratchBytes
     void* ws = nullptr;
-    const int st = qfx_workspace(ctx, bytes, &ws);
-    if (st != QFX_OK) return st;
+    // A sequence being recorded cannot grow the workspace: the partial sums
+    // go into the context's own scratch for it, or the product is refused.
+    if (ctx->capturing && !ctx->use_fixed_scratch && bytes > ctx->work_bytes && !needs_reservation) {
+      ws = ctx->record_scratch;
+    } else {
+      const int st = qfx_workspace(ctx, bytes, &ws);
+      if (st != QFX_OK) return st;
+    }
     out = static_cast<float2*>(ws);
   }
   auto go = [&](auto tile) {

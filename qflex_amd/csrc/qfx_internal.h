@@ -34,6 +34,10 @@ struct qfx_context {
   // Device workspace for split reductions (grows on demand).
   void* work = nullptr;
   size_t work_bytes = 0;
+  // Partial sums of recorded FP32 products that the reserved workspace does
+  // not hold: kFixedScratchBytes of the arena, from the first qfx_graph_begin
+  // on (a replay may come at any time after it).
+  void* record_scratch = nullptr;
   // Profiling.
   bool profiling = false;
   std::vector<QfxProfRec> pending;
@@ -201,8 +205,10 @@ int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
 // FP32 MFMA products of qfx_f32.hip, any m, n, k that fit (pointers checked by
 // the caller); maps = {a_rows, a_cols, b_rows, b_cols} or null for row-major,
 // a_mfast / b_kfast the operands' contiguous direction.  Products of few
-// outputs are split over k through the workspace; where a sequence being
-// recorded has reserved too little, needs_splits refuses them.
+// outputs are split over k through the workspace, at most kFixedScratchBytes
+// of it.  Where a sequence being recorded has reserved too little they take
+// the context's record_scratch, or are refused with needs_reservation.  The
+// splits depend on m, n and k alone, so recorded and eager bits are equal.
 bool qfx_f32_fits(uint64_t m, uint64_t n, uint64_t k);
 // The products of a grouped call that would run there, `which` of them, in one
 // launch per tile (row-major operands, pointers checked).
@@ -213,7 +219,7 @@ int qfx_upload_problems(qfx_context* ctx, void* dev, const void* host, size_t by
 double qfx_f32_time(uint64_t m, uint64_t n, uint64_t k);  // estimate of its kernels, in us
 int qfx_launch_f32(qfx_context* ctx, const float2* A, const float2* B, float2* C, uint64_t m,
                    uint64_t n, uint64_t k, const qfx_index_map* maps, bool a_mfast,
-                   bool b_kfast, bool needs_splits);
+                   bool b_kfast, bool needs_reservation);
 
 // FP8 (E4M3, per-128x128-tile power-of-two scales) complex GEMM of
 // qfx_fp8.hip: whether the shape is large enough for its tiles, and the

@@ -609,6 +609,10 @@ extern "C" int qfx_graph_begin(qfx_context* ctx, size_t workspace_bytes) {
     int st = qfx_workspace(ctx, workspace_bytes, &ws);
     if (st != QFX_OK) return st;
   }
+  if (!ctx->record_scratch) {
+    const int st = qfx_alloc(ctx, kFixedScratchBytes, &ctx->record_scratch);
+    if (st != QFX_OK) return st;
+  }
   QFX_HIP(hipStreamSynchronize(ctx->stream));
   QFX_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
   ctx->capturing = true;

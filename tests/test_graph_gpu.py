@@ -103,3 +103,33 @@ def test_workspace_must_be_reserved_before_recording():
         c.sync()
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("prec", [capi.FP32, capi.SPLIT_FP16])
+@pytest.mark.parametrize("workspace", [0, 64 << 20])
+def test_recorded_products_of_few_outputs_match_eager(prec, workspace):
+    """Products the FP32 kernel splits over k, at a small and a large
+    reservation: the recorded ones give the eager bits."""
+    rng = np.random.default_rng(6)
+    for m, n, k in [(57, 104, 3384), (200, 14, 1000), (3, 2000, 700)]:
+        c = capi.Context(0)  # its workspace has not grown yet
+        try:
+            A, B = c.upload(rand_c(rng, (m, k))), c.upload(rand_c(rng, (k, n)))
+            C = c.alloc(m * n * 8)
+            c.graph_begin(workspace_bytes=workspace)
+            try:
+                c.cgemm(prec, m, n, k, A, B, C)
+            finally:
+                graph = c.graph_end()
+            got = []
+            for _ in range(3):
+                c.zero(C)
+                graph.launch()
+                got.append(c.download(C, np.complex64, (m, n)))
+            graph.destroy()
+            c.zero(C)
+            c.cgemm(prec, m, n, k, A, B, C)
+            want = c.download(C, np.complex64, (m, n))
+            assert all(np.array_equal(g, want) for g in got), (m, n, k)
+        finally:
+            c.close()
