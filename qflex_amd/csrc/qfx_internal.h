@@ -34,6 +34,12 @@ struct qfx_context {
   // Device workspace for split reductions (grows on demand).
   void* work = nullptr;
   size_t work_bytes = 0;
+  // Recorded graphs replay with the workspace's address: one that a recorded
+  // call took stays out of the arena when it is outgrown, until no graph of
+  // the context is left.
+  int graphs = 0;                  // recorded and not destroyed
+  bool work_recorded = false;      // a recorded call took `work`
+  std::vector<void*> kept_works;   // outgrown ones
   // Partial sums of recorded FP32 products that the reserved workspace does
   // not hold: kFixedScratchBytes of the arena, from the first qfx_graph_begin
   // on (a replay may come at any time after it).

@@ -215,7 +215,9 @@ int qfx_workspace(qfx_context* ctx, size_t bytes, void** out) {
       // The stream may still read the old workspace; it is not freed to HIP,
       // only returned to the arena after the stream drains.
       QFX_HIP(hipStreamSynchronize(ctx->stream));
-      qfx_free(ctx, ctx->work);
+      if (ctx->work_recorded) ctx->kept_works.push_back(ctx->work);
+      else qfx_free(ctx, ctx->work);
+      ctx->work_recorded = false;
       ctx->work = nullptr;
       ctx->work_bytes = 0;  // a failed allocation below leaves no workspace
     }
@@ -224,6 +226,7 @@ int qfx_workspace(qfx_context* ctx, size_t bytes, void** out) {
     if (st != QFX_OK) return st;
     ctx->work_bytes = sz;
   }
+  if (ctx->capturing) ctx->work_recorded = true;
   *out = ctx->work;
   return QFX_OK;
 }
@@ -601,6 +604,15 @@ extern "C" int qfx_accumulate_batched_c128(qfx_context* ctx, const qfx_c64* src,
 
 // ---------------------------------------------------------------- graphs
 
+// No graph of the context is left, and none is being recorded: nothing
+// replays into an earlier workspace any more.
+static void release_recorded_works(qfx_context* ctx) {
+  if (ctx->graphs > 0 || ctx->capturing) return;
+  for (void* w : ctx->kept_works) qfx_free(ctx, w);
+  ctx->kept_works.clear();
+  ctx->work_recorded = false;
+}
+
 extern "C" int qfx_graph_begin(qfx_context* ctx, size_t workspace_bytes) {
   QFX_CHECK_CTX(ctx);
   QFX_NOT_CAPTURING(ctx, "qfx_graph_begin");
@@ -627,18 +639,21 @@ extern "C" int qfx_graph_end(qfx_context* ctx, qfx_graph** out) {
   QFX_HIP(hipStreamEndCapture(ctx->stream, &graph));
   if (!out) {
     hipGraphDestroy(graph);
+    release_recorded_works(ctx);
     return qfx_set_error(QFX_ERR_INVALID, "qfx_graph_end: null output");
   }
   hipGraphExec_t exec = nullptr;
   hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
   if (e != hipSuccess) {
     hipGraphDestroy(graph);
+    release_recorded_works(ctx);
     return qfx_hip_error(e, "hipGraphInstantiate");
   }
   qfx_graph* g = new qfx_graph;
   g->graph = graph;
   g->exec = exec;
   g->ctx = ctx;
+  ++ctx->graphs;
   *out = g;
   return QFX_OK;
 }
@@ -657,6 +672,10 @@ extern "C" int qfx_graph_destroy(qfx_graph* graph) {
   if (graph->ctx) hipStreamSynchronize(graph->ctx->stream);
   if (graph->exec) hipGraphExecDestroy(graph->exec);
   if (graph->graph) hipGraphDestroy(graph->graph);
+  if (graph->ctx) {
+    --graph->ctx->graphs;
+    release_recorded_works(graph->ctx);
+  }
   delete graph;
   return QFX_OK;
 }

@@ -133,3 +133,38 @@ def test_recorded_products_of_few_outputs_match_eager(prec, workspace):
             assert all(np.array_equal(g, want) for g in got), (m, n, k)
         finally:
             c.close()
+
+
+def test_outgrown_workspace_of_a_graph_is_not_handed_out():
+    """An eager product grows the workspace that a recorded one uses: the old
+    one must not become another buffer's memory while the graph can be
+    replayed, and goes back to the arena once the graph is destroyed."""
+    rng = np.random.default_rng(12)
+    m, n, k = 57, 104, 3384
+    reserve = 4 << 20
+    c = capi.Context(0)
+    try:
+        A, B, C = c.upload(rand_c(rng, (m, k))), c.upload(rand_c(rng, (k, n))), c.alloc(m * n * 8)
+        c.cgemm(capi.FP32, m, n, k, A, B, C)
+        want = c.download(C, np.complex64, (m, n))
+        c.graph_begin(workspace_bytes=reserve)
+        try:
+            c.cgemm(capi.FP32, m, n, k, A, B, C)
+        finally:
+            graph = c.graph_end()
+        # partial sums of 16384 chunks of 8 x 8 outputs, 8 MiB: more than the reservation
+        X, Z = c.alloc(8 * 8 * (1 << 25)), c.alloc(8 * 64)
+        c.zero(X)
+        c.cgemm(capi.FP32, 8, 8, 1 << 25, X, X, Z)
+        others = [c.upload(np.full(reserve // 8, i + 1, np.uint64)) for i in range(4)]
+        for _ in range(2):
+            c.zero(C)
+            graph.launch()
+            assert np.array_equal(c.download(C, np.complex64, (m, n)), want)
+        for i, buf in enumerate(others):
+            assert (c.download(buf, np.uint64, (reserve // 8,)) == i + 1).all(), i
+        held = c.arena_stats()[1]
+        graph.destroy()
+        assert held - c.arena_stats()[1] >= reserve
+    finally:
+        c.close()
