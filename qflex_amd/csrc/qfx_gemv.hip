@@ -177,8 +177,9 @@ __device__ __forceinline__ float2 group_sum(float2 v, float2* red, int CL, int G
   return r;
 }
 
-// y[c] = sum_r x[r] A[r][c] (A is m x k, row-major).  Block (x, y): the
-// columns V * (CL x + lane) of the rows [rows_per * y, ...); its T threads
+// y[c] = sum_r x[r] A[r][c] (A is m x k, row-major).  Block (x, y, z): column
+// tile t = x + z gridDim.x, the columns V * (CL t + lane), of the rows
+// [rows_per * y, ...); its T threads
 // are G = T / CL row groups of CL column lanes, four rows in flight each.
 // A narrow matrix takes all its columns as the lanes (CL = k / V), so that
 // the block reads whole rows one after the other.  One split over the rows
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(T) void gemv_t_kernel(const float2* __restrict__ A,
   __shared__ float2 red[T];
   const int G = T / CL;
   const int rg = threadIdx.x / CL, cl = threadIdx.x - rg * CL;
-  const uint64_t c = (uint64_t(blockIdx.x) * CL + cl) * V;
+  const uint64_t c = ((uint64_t(blockIdx.z) * gridDim.x + blockIdx.x) * CL + cl) * V;
   const uint64_t r0 = blockIdx.y * rows_per;
   const uint64_t r1 = r0 + rows_per < M ? r0 + rows_per : M;
   const bool in = rg < G && c < K;  // (V divides K)
@@ -334,7 +335,10 @@ int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
   nsplit = std::max<uint64_t>(nsplit, 1);
   const uint64_t rows_per = (m + nsplit - 1) / nsplit;
   nsplit = (m + rows_per - 1) / rows_per;
-  if (tiles > 0x7fffffffULL) return qfx_set_error(QFX_ERR_UNSUPPORTED, "gemv: too many columns");
+  // 2^23 tiles along x (2^31 threads of the 2^32 that a grid dimension can
+  // hold), from 2^29 columns on several of those along z
+  const uint64_t tiles_x = std::min(tiles, uint64_t(1) << 23);
+  if (tiles > tiles_x * 65535) return qfx_set_error(QFX_ERR_UNSUPPORTED, "gemv: too many columns");
   // Blocks of 1024 threads that take all rows of fewer columns save the
   // partials and their launch.  Taken with at most 32 rows per thread in at
   // least 128 blocks (4096 x 4096: 28.2 -> 23.0 us, 5.8 TB/s; 1024 x 65536 98.2 ->
@@ -361,7 +365,7 @@ int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
     if (st != QFX_OK) return st;
     out = static_cast<float2*>(ws);
   }
-  const dim3 g{unsigned(tiles), unsigned(nsplit), 1};
+  const dim3 g{unsigned(tiles_x), unsigned(nsplit), unsigned((tiles + tiles_x - 1) / tiles_x)};
   if (V == 2)
     gemv_t_kernel<2, 256><<<g, 256, 0, ctx->stream>>>(A, x, out, m, k, rows_per, CL);
   else

@@ -495,3 +495,27 @@ def test_reorder_small_odd_tensors_bit_exact(ctx, dims, perm):
     assert np.array_equal(got[:-1], x.transpose(perm).ravel()) and got[-1] == 0
     src.free()
     dst.free()
+
+
+def test_cgemv_t_more_than_2_30_columns():
+    """Column tiles beyond what one grid dimension holds (2^32 threads)."""
+    ctx = capi.Context(0)  # 20 GiB that closing it gives back
+    k = (1 << 30) + 1
+    A, Y, X = ctx.alloc(8 * k), ctx.alloc(8 * (k + 1)), ctx.upload(np.array([2 - 1j], np.complex64))
+    ctx.zero(A)
+    ctx.zero(Y)
+    rng = np.random.default_rng(30)
+
+    class At:
+        def __init__(self, buf, element):
+            self.ptr = buf.ptr + 8 * element
+    spots = [0, (1 << 29) - 500, k - 1000]
+    parts = [(rng.integers(-9, 10, 1000) + 1j * rng.integers(-9, 10, 1000)).astype(np.complex64)
+             for _ in spots]
+    for spot, part in zip(spots, parts):
+        ctx.upload_async(At(A, spot), part)
+    ctx.cgemv(1, 1, k, A, X, Y)
+    for spot, part in zip(spots, parts):
+        assert np.array_equal(ctx.download(At(Y, spot), np.complex64, (1000,)), (2 - 1j) * part), spot
+    assert ctx.download(At(Y, k), np.complex64, (1,))[0] == 0
+    ctx.close()
