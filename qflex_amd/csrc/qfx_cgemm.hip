@@ -2378,45 +2378,56 @@ int qfx_upload_problems(qfx_context* ctx, void* dev, const void* host, size_t by
   return qfx_flush_uploads(ctx);
 }
 
-// The k <= 16 problems of a grouped call in one launch: those of the row
-// kernel (n <= 16), or those of 64 x 64 tiles.  A longer problem
+// Blocks of a k <= 16 problem: of the row kernel (narrow), or tiles of 64 x 64.
+static uint64_t smallk_blocks(const qfx_gemm_desc& d, bool narrow) {
+  return narrow ? (d.m + 255) / 256 : (d.m + 63) / 64 * ((d.n + 63) / 64);
+}
+
+// The k <= 16 problems of a grouped call: those of the row kernel (n <= 16),
+// or those of 64 x 64 tiles, in one launch (more only where one grid does not
+// hold their blocks; one problem's it does).  A longer problem
 // list goes to the device through the staged uploads (flushed right before
 // the launch) into the workspace.
 static int launch_smallk_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
                                  const std::vector<int>& rows, bool narrow) {
-  std::vector<RowsProb> probs(rows.size());
-  uint64_t blocks = 0;
-  double flops = 0, bytes = 0;
-  for (size_t r = 0; r < rows.size(); ++r) {
-    const qfx_gemm_desc& d = descs[rows[r]];
-    probs[r] = RowsProb{reinterpret_cast<const float2*>(d.A), reinterpret_cast<const float2*>(d.B),
-                        reinterpret_cast<float2*>(d.C), d.m, int(d.n), int(d.k), blocks};
-    blocks += narrow ? (d.m + 255) / 256 : (d.m + 63) / 64 * ((d.n + 63) / 64);
-    flops += 8.0 * double(d.m) * double(d.n) * double(d.k);
-    bytes += 8.0 * (double(d.m) * d.k + double(d.k) * d.n + double(d.m) * d.n);
-  }
-  if (blocks > 0x7fffffffULL)
-    return qfx_set_error(QFX_ERR_UNSUPPORTED, "qfx_cgemm_grouped_c64: too many row blocks");
-  if (probs.size() <= size_t(kArgProblems)) {
-    ArgList<RowsProb> list{};
-    std::copy(probs.begin(), probs.end(), list.p);
+  std::vector<RowsProb> probs;
+  probs.reserve(rows.size());
+  for (size_t at = 0; at < rows.size();) {
+    probs.clear();
+    uint64_t blocks = 0;
+    double flops = 0, bytes = 0;
+    for (; at < rows.size(); ++at) {
+      const qfx_gemm_desc& d = descs[rows[at]];
+      const uint64_t more = smallk_blocks(d, narrow);
+      if (blocks + more > kMaxBlocks) break;
+      probs.push_back(RowsProb{reinterpret_cast<const float2*>(d.A),
+                               reinterpret_cast<const float2*>(d.B),
+                               reinterpret_cast<float2*>(d.C), d.m, int(d.n), int(d.k), blocks});
+      blocks += more;
+      flops += 8.0 * double(d.m) * double(d.n) * double(d.k);
+      bytes += 8.0 * (double(d.m) * d.k + double(d.k) * d.n + double(d.m) * d.n);
+    }
+    if (probs.size() <= size_t(kArgProblems)) {
+      ArgList<RowsProb> list{};
+      std::copy(probs.begin(), probs.end(), list.p);
+      QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
+      (narrow ? cgemm_rows_grouped_args_kernel
+              : cgemm_smallk_grouped_args_kernel)<<<unsigned(blocks), 256, 0, ctx->stream>>>(
+          list, int(probs.size()));
+      QFX_HIP(hipGetLastError());
+      continue;
+    }
+    void* ws = nullptr;
+    int st = qfx_workspace(ctx, probs.size() * sizeof(RowsProb), &ws);
+    if (st != QFX_OK) return st;
+    st = qfx_upload_problems(ctx, ws, probs.data(), probs.size() * sizeof(RowsProb));
+    if (st != QFX_OK) return st;
     QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
-    (narrow ? cgemm_rows_grouped_args_kernel
-            : cgemm_smallk_grouped_args_kernel)<<<unsigned(blocks), 256, 0, ctx->stream>>>(
-        list, int(probs.size()));
+    (narrow ? cgemm_rows_grouped_kernel
+            : cgemm_smallk_grouped_kernel)<<<unsigned(blocks), 256, 0, ctx->stream>>>(
+        static_cast<const RowsProb*>(ws), int(probs.size()));
     QFX_HIP(hipGetLastError());
-    return QFX_OK;
   }
-  void* ws = nullptr;
-  int st = qfx_workspace(ctx, probs.size() * sizeof(RowsProb), &ws);
-  if (st != QFX_OK) return st;
-  st = qfx_upload_problems(ctx, ws, probs.data(), probs.size() * sizeof(RowsProb));
-  if (st != QFX_OK) return st;
-  QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
-  (narrow ? cgemm_rows_grouped_kernel
-          : cgemm_smallk_grouped_kernel)<<<unsigned(blocks), 256, 0, ctx->stream>>>(
-      static_cast<const RowsProb*>(ws), int(probs.size()));
-  QFX_HIP(hipGetLastError());
   return QFX_OK;
 }
 
@@ -2522,7 +2533,7 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
   for (int i = 0; i < count; ++i) {
     const qfx_gemm_desc& d = descs[i];
     const bool full = d.m > 0 && d.n > 0 && d.k > 0 && d.A && d.B && d.C;
-    if (full && d.k <= uint64_t(kSmallK) && d.n <= 16 && (d.m + 255) / 256 <= 0x7fffffffULL) {
+    if (full && d.k <= uint64_t(kSmallK) && d.n <= 16 && smallk_blocks(d, true) <= kMaxBlocks) {
       rows.push_back(i);
       continue;
     }
@@ -2542,8 +2553,8 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
       grouped_odd.push_back(i);
       continue;
     }
-    const bool small = d.k <= uint64_t(kSmallK) && d.n <= 65535ULL * 64 &&
-                       d.m <= 0x7fffffffULL;
+    const bool small = d.k <= uint64_t(kSmallK) && d.n > 16 && d.n <= 65535ULL * 64 &&
+                       d.m <= 0x7fffffffULL && smallk_blocks(d, false) <= kMaxBlocks;
     const bool matrix = d.k > uint64_t(kSmallK) && d.m > 1 && d.n > 1 &&
                         (d.m > 8 || d.n > 8 || d.k < 1024) && precision != QFX_PREC_FP8 &&
                         f32_route(precision, d.m, d.n, d.k, false);

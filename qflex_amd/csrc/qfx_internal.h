@@ -192,6 +192,10 @@ __device__ __forceinline__ uint64_t xcd_tile(uint64_t b, uint64_t tiles) {
   return x * q + (x < r ? x : r) + b / 8;
 }
 
+// Blocks of 256 threads along one dimension of a launch: a grid dimension
+// holds less than 2^32 threads, and a launch of more is cut without an error.
+constexpr uint64_t kMaxBlocks = (uint64_t(1) << 24) - 1;
+
 // A short problem list as a kernel argument: no workspace and no upload launch
 // before the grouped one (5 us of a call).
 constexpr int kArgProblems = 32;

@@ -257,3 +257,18 @@ def test_grouped_refuses_operands_past_their_block(ctx, prec, shape, operand):
     assert not ctx.download(blocks[2], np.uint8, (blocks[2].nbytes,)).any()
     for buf in blocks:
         buf.free()
+
+
+def test_grouped_small_k_products_beyond_one_grid():
+    """257 products of 65535 blocks each, more than 2^32 threads together."""
+    ctx = capi.Context(0)  # 10 GiB that closing it gives back
+    m, n, k, count = 1, 65535 * 64, 2, 257
+    rng = np.random.default_rng(21)
+    a = (rng.integers(-9, 10, (m, k)) + 1j * rng.integers(-9, 10, (m, k))).astype(np.complex64)
+    b = (rng.integers(-9, 10, (k, n)) + 1j * rng.integers(-9, 10, (k, n))).astype(np.complex64)
+    A, B, C = ctx.upload(a), ctx.upload(b), ctx.alloc(count * n * 8)
+    ctx.zero(C)
+    ctx.cgemm_grouped(capi.FP32, [(m, n, k, A, B, At(C, 8 * n * i)) for i in range(count)])
+    for i in (0, 1, count - 2, count - 1):
+        assert np.array_equal(ctx.download(At(C, 8 * n * i), np.complex64, (m, n)), a @ b), i
+    ctx.close()
