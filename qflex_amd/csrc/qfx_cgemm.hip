@@ -1055,12 +1055,13 @@ struct GroupTile {
 };
 
 // The operand maxima of all problems of a grouped launch: block b runs its
-// block of A or B of the problem whose partial maxima b is among.  (One
-// launch per problem cost 3 us each.)
+// block of A or B of the problem whose partial maxima `first` + b is among.
+// (One launch per problem cost 3 us each.)
 __global__ __launch_bounds__(256) void amax_grouped_kernel(const GroupTile* __restrict__ probs,
-                                                           int count, float* __restrict__ part) {
+                                                           int count, float* __restrict__ part,
+                                                           uint64_t first) {
   __shared__ float red[4];
-  const uint64_t t = blockIdx.x;
+  const uint64_t t = first + blockIdx.x;
   const GroupTile& g =
       probs[group_entry(&probs[0].first_part, sizeof(GroupTile), count, t)];
   const int b = int(t - g.first_part);
@@ -2451,8 +2452,6 @@ static int launch_split_grouped(qfx_context* ctx, int precision, const qfx_gemm_
     }
   }
   QfxLaunchScope scope(ctx, QFX_K_CGEMM, bytes, flops);
-  if (nparts > 0x7fffffffULL)
-    return qfx_set_error(QFX_ERR_UNSUPPORTED, "qfx_cgemm_grouped_c64: too many operand blocks");
   const size_t part_bytes = (nparts * sizeof(float) + 255) / 256 * 256;
   const size_t desc_bytes = grouped.size() * sizeof(GroupTile);
   void* ws = nullptr;
@@ -2481,8 +2480,9 @@ static int launch_split_grouped(qfx_context* ctx, int precision, const qfx_gemm_
   }
   st = qfx_upload_problems(ctx, dev, host.data(), desc_bytes);
   if (st != QFX_OK) return st;
-  if (nparts > 0)
-    amax_grouped_kernel<<<unsigned(nparts), 256, 0, ctx->stream>>>(dev, int(host.size()), part);
+  for (uint64_t at = 0; at < nparts; at += kMaxBlocks)
+    amax_grouped_kernel<<<unsigned(std::min<uint64_t>(kMaxBlocks, nparts - at)), 256, 0,
+                          ctx->stream>>>(dev, int(host.size()), part, at);
   QFX_HIP(hipGetLastError());
   if (ctx->cus <= 0) {
     int cus = 0;

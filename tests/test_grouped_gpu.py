@@ -272,3 +272,23 @@ def test_grouped_small_k_products_beyond_one_grid():
     for i in (0, 1, count - 2, count - 1):
         assert np.array_equal(ctx.download(At(C, 8 * n * i), np.complex64, (m, n)), a @ b), i
     ctx.close()
+
+
+def test_grouped_maxima_beyond_one_grid(ctx):
+    """33000 split-FP16 products of 512 blocks of maxima each, of values that
+    without their scale vanish in FP16."""
+    m, n, k, count = 64, 64, 16384, 33000
+    rng = np.random.default_rng(22)
+    # whole numbers times 2^-40: exact in the scaled planes and in every sum (18 k < 2^24)
+    a = (rng.integers(-3, 4, (m, k)) + 1j * rng.integers(-3, 4, (m, k))).astype(np.complex64)
+    b = (rng.integers(-3, 4, (k, n)) + 1j * rng.integers(-3, 4, (k, n))).astype(np.complex64)
+    a, b = a * np.float32(2.0 ** -40), b * np.float32(2.0 ** -40)
+    A, B, C = ctx.upload(a), ctx.upload(b), ctx.alloc(count * m * n * 8)
+    ctx.zero(C)
+    ctx.cgemm_grouped(capi.SPLIT_FP16,
+                      [(m, n, k, A, B, At(C, 8 * m * n * i)) for i in range(count)])
+    got = ctx.download(C, np.complex64, (count, m, n))
+    want = (a.astype(np.complex128) @ b.astype(np.complex128)).astype(np.complex64)
+    assert (got == want).all()
+    for buf in (A, B, C):
+        buf.free()
