@@ -473,7 +473,8 @@ int qfx_launch_f32_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
                            const std::vector<int>& which) {
   // Each product takes the tile that would be the fastest if all were like it.
   // Those that fill the chip alone run as qfx_cgemm_c64 runs them, and so do
-  // all of a few where that is estimated faster (long k, split alone).
+  // all of a few where that is estimated faster (long k, split alone) and
+  // what is beyond one grid.
   std::vector<std::vector<int>> by_tile(kTileC + 1);
   double alone_us = 0, group_us = 6, longest = 0;
   auto alone = [&](const qfx_gemm_desc& d) {
@@ -509,10 +510,12 @@ int qfx_launch_f32_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
   }
   std::vector<F32Prob> probs;
   uint64_t tiles[kTileC + 1] = {};
+  int counts[kTileC + 1] = {};
   for (int t = kTileA; t <= kTileC; ++t)
     for (int i : by_tile[t]) {
       const qfx_gemm_desc& d = descs[i];
-      if (alone_us < group_us + longest) {
+      const uint64_t more = tiles_of(F32Tile(t), d.m, d.n);
+      if (alone_us < group_us + longest || tiles[t] + more > kMaxBlocks) {
         const int st = alone(d);
         if (st != QFX_OK) return st;
         continue;
@@ -523,9 +526,8 @@ int qfx_launch_f32_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
                               int64_t(d.k), int(d.m), int(d.n), int((d.n + tn[t] - 1) / tn[t]),
                               int((d.k + stage_of(F32Tile(t)) - 1) / stage_of(F32Tile(t))),
                               tiles[t]});
-      tiles[t] += tiles_of(F32Tile(t), d.m, d.n);
-      if (tiles[t] > 0x7fffffffULL)
-        return qfx_set_error(QFX_ERR_UNSUPPORTED, "qfx_cgemm_grouped_c64: too many tiles");
+      tiles[t] += more;
+      ++counts[t];
     }
   if (probs.empty()) return QFX_OK;
   const bool args = probs.size() <= size_t(kArgProblems);
@@ -545,7 +547,7 @@ int qfx_launch_f32_grouped(qfx_context* ctx, const qfx_gemm_desc* descs,
   const F32Prob* dev = static_cast<const F32Prob*>(ws);
   const F32Prob* host = probs.data();
   auto go = [&](auto tile, int t) {
-    const int n = int(by_tile[t].size());
+    const int n = counts[t];
     if (n == 0) return;
     if (args) {
       ArgList<F32Prob> list{};

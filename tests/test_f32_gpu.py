@@ -188,3 +188,24 @@ def test_small_outputs_are_one_class_in_the_profile(ctx):
     assert prof["cgemm"]["launches"] == 2 and prof["cgemm_small"]["launches"] == 0
     for buf in (A, B, C):
         buf.free()
+
+
+def test_grouped_f32_products_beyond_one_grid():
+    """33000 products of 511 tiles each: more blocks than a launch can hold."""
+    m, n, k, count = 65408, 2, 17, 33000
+    ctx = capi.Context(0)  # 40 GiB that closing it gives back
+    rng = np.random.default_rng(11)
+    a, b = whole(rng, (m, k)), whole(rng, (k, n))
+    A, B, C = ctx.upload(a), ctx.upload(b), ctx.alloc(8 * m * n * count)
+
+    class At:
+        def __init__(self, i):
+            self.ptr, self.nbytes = C.ptr + 8 * m * n * i, 8 * m * n
+    spots = [0, 1, count // 3, count - 200, count - 2, count - 1]
+    for i in spots:
+        ctx.zero(At(i))
+    ctx.cgemm_grouped(capi.FP32, [(m, n, k, A, B, At(i)) for i in range(count)])
+    want = product(a, b)
+    for i in spots:
+        assert np.array_equal(ctx.download(At(i), np.complex64, (m, n)), want), i
+    ctx.close()
