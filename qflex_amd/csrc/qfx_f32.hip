@@ -434,7 +434,8 @@ double qfx_f32_time(uint64_t m, uint64_t n, uint64_t k) { return f32_plan(m, n, 
 
 bool qfx_f32_fits(uint64_t m, uint64_t n, uint64_t k) {
   return m <= 0x7fffff00ULL && n <= 0x7fffff00ULL && k <= (1ULL << 34) &&
-         tiles_of(kTileC, m, n) <= 0x7fffffffULL;  // (the smallest tile)
+         (tiles_of(kTileC, m, n) <= kMaxBlocks ||  // (the smallest tile)
+          tiles_of(f32_plan(m, n, k).tile, m, n) <= kMaxBlocks);
 }
 
 int qfx_launch_f32(qfx_context* ctx, const float2* A, const float2* B, float2* C, uint64_t m,
