@@ -1484,9 +1484,9 @@ __global__ __launch_bounds__(256) void cgemm_tiny_mn_partial_kernel(
 
 // Small common dimension (k <= 16): exact FP32 on the vector ALUs, one
 // fmaf chain per output in increasing k (the same operation order as
-// cgemm_scalar_kernel, hence bit-identical to it).  Block tile BM x BN
-// (BM = 4096 / BN), each thread 4 rows x 4 columns; A and B tiles staged
-// through LDS with coalesced loads.
+// cgemm_scalar_kernel, hence bit-identical to it).  Block tile 64 x 64, each
+// thread 4 rows x 4 columns; A and B tiles staged through LDS with coalesced
+// loads.  (n <= 16 takes the row kernels below.)
 constexpr int kSmallK = 16;
 // MAPPED: operands through digit maps (offset tables in LDS); A is read
 // along m when a_mfast (a_rows digit 0 at stride 1), else along k; B along
@@ -1502,14 +1502,16 @@ __device__ __forceinline__ void store_block_max(float v, float* slot) {
   if (threadIdx.x == 0) *slot = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-template <int BN, bool MAPPED>
+template <bool MAPPED>
 __device__ __forceinline__ void smallk_tile(
     const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C,
     uint64_t M, int N, int K, const qfx_index_map& a_rows, const qfx_index_map& a_cols,
     const qfx_index_map& b_rows, const qfx_index_map& b_cols, bool a_mfast, bool b_nfast,
     float* __restrict__ cmax, uint64_t tile_m, unsigned tile_n) {
-  constexpr int TX = BN / 4;        // column groups
-  constexpr int BM = 4 * 256 / TX;  // rows per block
+  constexpr int BM = 64, BN = 64;
+  constexpr int TX = BN / 4;  // column groups
+  static_assert(BM * 4 % 256 == 0 && BN * 4 % 256 == 0,
+                "a_at and b_at bound whole steps of the block's 256 threads");
   __shared__ float2 As[BM][kSmallK + 1];
   __shared__ float2 Bs[kSmallK][BN];
   __shared__ uint64_t arow[MAPPED ? BM : 1], bcol[MAPPED ? BN : 1];
@@ -1602,12 +1604,12 @@ __device__ __forceinline__ void smallk_tile(
   if (cmax) store_block_max(cm, cmax);
 }
 
-template <int BN, bool MAPPED>
+template <bool MAPPED>
 __global__ __launch_bounds__(256) void cgemm_smallk_kernel(
     const float2* __restrict__ A, const float2* __restrict__ B, float2* __restrict__ C,
     uint64_t M, int N, int K, qfx_index_map a_rows, qfx_index_map a_cols, qfx_index_map b_rows,
     qfx_index_map b_cols, bool a_mfast, bool b_nfast, float* __restrict__ cmax) {
-  smallk_tile<BN, MAPPED>(A, B, C, M, N, K, a_rows, a_cols, b_rows, b_cols, a_mfast, b_nfast,
+  smallk_tile<MAPPED>(A, B, C, M, N, K, a_rows, a_cols, b_rows, b_cols, a_mfast, b_nfast,
                           cmax ? cmax + blockIdx.x + uint64_t(gridDim.x) * blockIdx.y : nullptr,
                           blockIdx.x, blockIdx.y);
 }
@@ -1916,7 +1918,7 @@ __device__ __forceinline__ void smallk_grouped_block(const RowsProb* probs, int 
   const RowsProb p = probs[group_entry(&probs[0].first_block, sizeof(RowsProb), count, b)];
   const qfx_index_map none{};
   const uint64_t t = b - p.first_block, tiles_n = uint64_t((p.N + 63) / 64);
-  smallk_tile<64, false>(p.A, p.B, p.C, p.M, p.N, p.K, none, none, none, none, false, true,
+  smallk_tile<false>(p.A, p.B, p.C, p.M, p.N, p.K, none, none, none, none, false, true,
                          nullptr, t / tiles_n, unsigned(t % tiles_n));
 }
 __global__ __launch_bounds__(256) void cgemm_smallk_grouped_kernel(
@@ -2027,7 +2029,7 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
     // Small common dimension: exact FP32 on the vector ALUs for every
     // precision (bit-identical to the defined-order scalar kernel).
     QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
-    if (n <= 16 && (m + 255) / 256 <= 0x7fffffffULL) {
+    if (n <= 16) {
       const unsigned blocks = unsigned((m + 255) / 256);
       if (k % 2 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0)
         cgemm_rows_kernel<false, true><<<blocks, 256, 0, ctx->stream>>>(
@@ -2038,14 +2040,10 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
       else
         cgemm_rows_kernel<false, false><<<blocks, 256, 0, ctx->stream>>>(
             A2, B2, C2, m, int(n), int(k), {}, {}, {}, {}, nullptr);
-    } else if (n <= 16) {
-      dim3 g{unsigned((m + 255) / 256), unsigned((n + 15) / 16), 1};
-      cgemm_smallk_kernel<16, false><<<g, 256, 0, ctx->stream>>>(A2, B2, C2, m, int(n), int(k),
-                                                                 {}, {}, {}, {}, false, true, nullptr);
     } else {
       dim3 g{unsigned((m + 63) / 64), unsigned((n + 63) / 64), 1};
-      cgemm_smallk_kernel<64, false><<<g, 256, 0, ctx->stream>>>(A2, B2, C2, m, int(n), int(k),
-                                                                 {}, {}, {}, {}, false, true, nullptr);
+      cgemm_smallk_kernel<false><<<g, 256, 0, ctx->stream>>>(A2, B2, C2, m, int(n), int(k), {}, {},
+                                                             {}, {}, false, true, nullptr);
     }
     QFX_HIP(hipGetLastError());
     return QFX_OK;
@@ -2258,7 +2256,7 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
       io->c_max_n = int(blocks);
       return io->c_max;
     };
-    if (n <= 16 && (m + 255) / 256 <= 0x7fffffffULL) {
+    if (n <= 16) {
       const uint64_t blocks = (m + 255) / 256;
       // rows of A contiguous along k (A's k digits in order from stride 1)
       // and starting at even offsets (16-byte aligned)
@@ -2273,14 +2271,9 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
       else
         cgemm_rows_kernel<true, false><<<unsigned(blocks), 256, 0, ctx->stream>>>(
             A2, B2, C2, m, int(n), int(k), *a_rows, *a_cols, *b_rows, *b_cols, cmax_for(blocks));
-    } else if (n <= 16) {
-      dim3 g{unsigned((m + 255) / 256), unsigned((n + 15) / 16), 1};
-      cgemm_smallk_kernel<16, true><<<g, 256, 0, ctx->stream>>>(
-          A2, B2, C2, m, int(n), int(k), *a_rows, *a_cols, *b_rows, *b_cols, a_mfast, b_nfast,
-          cmax_for(uint64_t(g.x) * g.y));
     } else {
       dim3 g{unsigned((m + 63) / 64), unsigned((n + 63) / 64), 1};
-      cgemm_smallk_kernel<64, true><<<g, 256, 0, ctx->stream>>>(
+      cgemm_smallk_kernel<true><<<g, 256, 0, ctx->stream>>>(
           A2, B2, C2, m, int(n), int(k), *a_rows, *a_cols, *b_rows, *b_cols, a_mfast, b_nfast,
           cmax_for(uint64_t(g.x) * g.y));
     }
