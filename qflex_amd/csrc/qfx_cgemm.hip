@@ -2030,20 +2030,23 @@ extern "C" int qfx_cgemm_c64(qfx_context* ctx, int precision, uint64_t m, uint64
     // precision (bit-identical to the defined-order scalar kernel).
     QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
     if (n <= 16) {
-      const unsigned blocks = unsigned((m + 255) / 256);
-      if (k % 2 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0)
-        cgemm_rows_kernel<false, true><<<blocks, 256, 0, ctx->stream>>>(
+      const uint64_t blocks = (m + 255) / 256;
+      if (k % 2 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 && blocks <= kMaxBlocks)
+        cgemm_rows_kernel<false, true><<<unsigned(blocks), 256, 0, ctx->stream>>>(
             A2, B2, C2, m, int(n), int(k), {}, {}, {}, {}, nullptr);
       else if (blocks >= 2 * kRowsStreamBlocks)
         cgemm_rows_stream_kernel<false><<<kRowsStreamBlocks, 256, 0, ctx->stream>>>(
             A2, B2, C2, m, int(n), int(k), {}, {}, {}, {}, nullptr, blocks);
       else
-        cgemm_rows_kernel<false, false><<<blocks, 256, 0, ctx->stream>>>(
+        cgemm_rows_kernel<false, false><<<unsigned(blocks), 256, 0, ctx->stream>>>(
             A2, B2, C2, m, int(n), int(k), {}, {}, {}, {}, nullptr);
     } else {
-      dim3 g{unsigned((m + 63) / 64), unsigned((n + 63) / 64), 1};
-      cgemm_smallk_kernel<false><<<g, 256, 0, ctx->stream>>>(A2, B2, C2, m, int(n), int(k), {}, {},
-                                                             {}, {}, false, true, nullptr);
+      for (uint64_t r = 0; r < m; r += 64 * kMaxBlocks) {  // (one launch below 2^30 rows)
+        const uint64_t rows = std::min(64 * kMaxBlocks, m - r);
+        dim3 g{unsigned((rows + 63) / 64), unsigned((n + 63) / 64), 1};
+        cgemm_smallk_kernel<false><<<g, 256, 0, ctx->stream>>>(
+            A2 + r * k, B2, C2 + r * n, rows, int(n), int(k), {}, {}, {}, {}, false, true, nullptr);
+      }
     }
     QFX_HIP(hipGetLastError());
     return QFX_OK;
@@ -2245,6 +2248,8 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
   const double bytes = 8.0 * (double(m) * k + double(k) * n + double(m) * n);
 
   if (k <= uint64_t(kSmallK) && n <= 65535ULL * 64) {
+    if (n > 16 && (m + 63) / 64 > kMaxBlocks)
+      return qfx_set_error(QFX_ERR_UNSUPPORTED, "qfx_cgemm_mapped_c64: too many rows");
     QfxLaunchScope scope(ctx, QFX_K_CGEMM_SMALL, bytes, flops);
     const bool a_mfast = contiguous(*a_rows, 1) && !contiguous(*a_cols, 3);
     const bool b_nfast = contiguous(*b_cols, 1) || !contiguous(*b_rows, 1);
@@ -2261,7 +2266,7 @@ extern "C" int qfx_cgemm_mapped_ex_c64(qfx_context* ctx, int precision, const qf
       // rows of A contiguous along k (A's k digits in order from stride 1)
       // and starting at even offsets (16-byte aligned)
       if (k % 2 == 0 && identity_map(*a_cols) && !has_digit_at(*a_rows, 0) &&
-          reinterpret_cast<uintptr_t>(A) % 16 == 0)
+          reinterpret_cast<uintptr_t>(A) % 16 == 0 && blocks <= kMaxBlocks)
         cgemm_rows_kernel<true, true><<<unsigned(blocks), 256, 0, ctx->stream>>>(
             A2, B2, C2, m, int(n), int(k), *a_rows, *a_cols, *b_rows, *b_cols, cmax_for(blocks));
       else if (blocks >= 2 * kRowsStreamBlocks)

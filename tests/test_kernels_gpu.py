@@ -519,3 +519,27 @@ def test_cgemv_t_more_than_2_30_columns():
         assert np.array_equal(ctx.download(At(Y, spot), np.complex64, (1000,)), (2 - 1j) * part), spot
     assert ctx.download(At(Y, k), np.complex64, (1,))[0] == 0
     ctx.close()
+
+
+# 2^24 row tiles and more: 2^32 rows of the row kernel, 2^30 of the 64 x 64 tile.
+@pytest.mark.parametrize("m,n,k", [((1 << 32) + 300, 1, 2), ((1 << 30) + 70, 17, 1)])
+def test_small_k_products_beyond_one_grid(m, n, k):
+    ctx = capi.Context(0)  # up to 180 GiB that closing it gives back
+    rng = np.random.default_rng(32)
+    whole = lambda *s: (rng.integers(-9, 10, s) + 1j * rng.integers(-9, 10, s)).astype(np.complex64)
+    b = whole(k, n)
+    A, B, C = ctx.alloc(8 * m * k), ctx.upload(b), ctx.alloc(8 * m * n)
+
+    class At:
+        def __init__(self, buf, row, width):
+            self.ptr, self.nbytes = buf.ptr + 8 * row * width, 8 * 1000 * width
+    spots = [0, m // 2, m - 1000]
+    parts = [whole(1000, k) for _ in spots]
+    for spot, part in zip(spots, parts):
+        ctx.upload_async(At(A, spot, k), part)
+        ctx.zero(At(C, spot, n))
+    ctx.cgemm(capi.FP32, m, n, k, A, B, C)
+    for spot, part in zip(spots, parts):
+        got = ctx.download(At(C, spot, n), np.complex64, (1000, n))
+        assert np.array_equal(got, (part.astype(np.complex128) @ b).astype(np.complex64)), spot
+    ctx.close()
