@@ -209,3 +209,29 @@ def test_grouped_f32_products_beyond_one_grid():
     for i in spots:
         assert np.array_equal(ctx.download(At(i), np.complex64, (m, n)), want), i
     ctx.close()
+
+
+def test_split_products_beyond_32_bit_offsets_same_bits(ctx):
+    """Odd k and an A of more than 2 GiB (rows in equal blocks): the split
+    kernels with 64-bit addressing give each block of rows the bits that the
+    pipelined ones give it alone."""
+    rows, blocks, n, k = 1024, 512, 48, 517
+    rng = np.random.default_rng(10)
+    rand = lambda *s: (rng.standard_normal(s) + 1j * rng.standard_normal(s)).astype(np.complex64)
+    part, B = ctx.upload(rand(rows, k)), ctx.upload(rand(k, n))
+    A, C, C1 = ctx.alloc(8 * rows * blocks * k), ctx.alloc(8 * rows * blocks * n), ctx.alloc(8 * rows * n)
+
+    class At:
+        def __init__(self, block):
+            self.ptr = A.ptr + 8 * rows * k * block
+    for block in range(blocks):
+        ctx.copy(At(block), part, 8 * rows * k)
+    for prec in (capi.SPLIT_FP16, capi.SPLIT_BF16, capi.SPLIT_BF16X3):
+        ctx.zero(C)
+        ctx.cgemm(prec, rows * blocks, n, k, A, B, C)
+        ctx.cgemm(prec, rows, n, k, part, B, C1)
+        want = ctx.download(C1, np.uint64, (1, rows, n))
+        assert want.any()
+        assert (ctx.download(C, np.uint64, (blocks, rows, n)) == want).all(), prec
+    for buf in (part, A, B, C, C1):
+        buf.free()
