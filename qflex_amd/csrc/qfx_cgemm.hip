@@ -7,8 +7,8 @@
 // matrix Ahat[m x 2k].  B[k x n] is expanded, while staging from LDS, into
 // the real matrix Bhat[2k x 2n] with 2x2 blocks [[Br, Bi], [-Bi, Br]], so
 // that Ahat . Bhat = [Cr Ci] interleaved, i.e. exactly C in memory order.
-// One v_mfma_f32_32x32x2_f32 then consumes one complex k for 32 rows and
-// 16 complex columns.  FLOPs are the textbook 8*m*n*k.
+// FLOPs are the textbook 8*m*n*k.  (The FP32 matrix-core form of the same is
+// in qfx_f32.hip.)
 //
 // Split-BF16 form.  Each real operand value x is split into BF16 terms
 // hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid); products of the
@@ -52,15 +52,10 @@ __global__ void cgemm_scalar_kernel(const float2* __restrict__ A, const float2* 
   }
 }
 
-// ------------------------------------------------------------ FP32 MFMA path
-constexpr int kBM = 128;  // complex rows per block
-constexpr int kBN = 64;   // complex cols per block
-constexpr int kBK = 16;   // complex k per stage
-constexpr int kAStride = 2 * kBK + 1;  // floats per LDS row of the A tile
-
 // ------------------------------------------------------------ split-BF16 MFMA
-// Same block tile as the FP32 kernel.  Operands are split once, while they
-// are staged into LDS, into NT BF16 planes (hi, mid[, lo]):
+// For operands beyond 32-bit offsets that the large tiles below don't take.
+// Operands are split once, while they are staged into LDS, into NT BF16
+// planes (hi, mid[, lo]):
 //   As[t][row][32 reals]          A rows, interleaved (re, im) along k;
 //   Bs[t][part*64 + n][32 reals]  Bhat columns: part 0 (the Cr column of
 //                                 complex column n) holds (Br_k, -Bi_k),
@@ -74,6 +69,9 @@ __device__ __forceinline__ void split3(float x, __bf16& h, __bf16& m, __bf16& l)
   l = static_cast<__bf16>(r - static_cast<float>(m));
 }
 
+constexpr int kBM = 128;   // complex rows per block
+constexpr int kBN = 64;    // complex cols per block
+constexpr int kBK = 16;    // complex k per stage
 constexpr int kRowB = 40;  // BF16 per LDS row: 32 + 8 pad (80 B, 16-byte aligned)
 
 template <int TERMS>
@@ -1043,7 +1041,8 @@ __global__ __launch_bounds__(64 * WM * WN) void cgemm_split_chain_kernel(
       int(L % gy) * 16 * J * WN, L, gridDim.x, ntiles, gy);
 }
 
-// One problem of a grouped launch: row-major operands, 256 x 128 tiles.
+// One problem of a grouped launch: row-major operands, 256 x 128 tiles (those
+// of odd sizes or 8-byte operands 128 x 64).
 struct GroupTile {
   const float2* A;
   const float2* B;
