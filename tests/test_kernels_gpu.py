@@ -543,3 +543,36 @@ def test_small_k_products_beyond_one_grid(m, n, k):
         got = ctx.download(At(C, spot, n), np.complex64, (1000, n))
         assert np.array_equal(got, (part.astype(np.complex128) @ b).astype(np.complex64)), spot
     ctx.close()
+
+
+# Edges of the waves and blocks that share a dot product and its partial sums;
+# whole numbers: every order of the sums is exact.
+@pytest.mark.parametrize("n", [1, 63, 65, 255, 257, 1000, 65537, 262144, 300001])
+def test_cdotu_exact(ctx, n):
+    rng = np.random.default_rng(n)
+    x, y = ((rng.integers(-3, 4, n) + 1j * rng.integers(-3, 4, n)).astype(np.complex64)
+            for _ in range(2))
+    X, Y, O = ctx.upload(x), ctx.upload(y), ctx.alloc(16)
+    ctx.zero(O)
+    ctx.cdotu(n, X, Y, O)
+    got = ctx.download(O, np.complex64, (2,))
+    assert got[0] == np.sum(x.astype(np.complex128) * y) and got[1] == 0
+    for buf in (X, Y, O):
+        buf.free()
+
+
+# Partial sums of several row splits: 16 columns per block and fewer, 64.
+@pytest.mark.parametrize("m,k", [(70000, 1), (66000, 2), (70001, 3), (20000, 17), (5000, 33), (9000, 63),
+                                 (66000, 5), (300, 70000), (70000, 16)])
+def test_cgemv_t_partial_sums_exact(ctx, m, k):
+    rng = np.random.default_rng(m + k)
+    a = (rng.integers(-3, 4, (m, k)) + 1j * rng.integers(-3, 4, (m, k))).astype(np.complex64)
+    x = (rng.integers(-3, 4, m) + 1j * rng.integers(-3, 4, m)).astype(np.complex64)
+    A, X, Y = ctx.upload(a), ctx.upload(x), ctx.alloc((k + 1) * 8)
+    ctx.zero(Y)
+    ctx.cgemv(1, m, k, A, X, Y)
+    got = ctx.download(Y, np.complex64, (k + 1,))
+    want = x.astype(np.complex128) @ a.astype(np.complex128)
+    assert np.array_equal(got[:-1], want.astype(np.complex64)) and got[-1] == 0
+    for buf in (A, X, Y):
+        buf.free()
