@@ -298,15 +298,22 @@ template <int V>
 void launch_n(hipStream_t s, uint64_t m, uint64_t k, const float2* A, const float2* x, float2* y) {
   const uint64_t units = k / V;
   // Few rows: a block per row, if the row has enough loads to fill it (four
-  // per thread; below 512 rows one).  Otherwise the largest group of lanes
-  // that a row keeps four fifths busy (33 columns: 8 lanes, 5 loads each).
+  // per thread; below 512 rows one).  Otherwise groups of lanes.
   if ((m < 4096 && units >= 1024) || (m < 512 && units >= 256)) {
     const unsigned threads = units >= 4096 && m <= 1024 ? 1024 : 256;
     gemv_n_block_kernel<V><<<unsigned(m), threads, 0, s>>>(A, x, y, m, k);
     return;
   }
+  // Many rows: the largest group that a row keeps four fifths busy (33
+  // columns: 8 lanes, 5 loads each).  Up to 3072 rows (three waves per SIMD,
+  // were each row a wave's) idle lanes cost nothing and rounds of loads do: a
+  // lane per load, up to a wave (1000 x 100: 2.9 us with 8 lanes, 2.5 so; 8000
+  // x 100 3.0 and 3.3).
   int llog = 6;
-  while (llog > 0 && 5 * units < 4 * ((((units - 1) >> llog) + 1) << llog)) --llog;
+  if (m <= 3072)
+    llog = log2_ceil(units, 6);
+  else
+    while (llog > 0 && 5 * units < 4 * ((((units - 1) >> llog) + 1) << llog)) --llog;
   // rows per lane group: four share each load of x where there are enough rows
   const uint64_t per_block = 256 >> llog;
   const bool four = m >= 4 * per_block * 512;

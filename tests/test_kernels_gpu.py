@@ -576,3 +576,21 @@ def test_cgemv_t_partial_sums_exact(ctx, m, k):
     assert np.array_equal(got[:-1], want.astype(np.complex64)) and got[-1] == 0
     for buf in (A, X, Y):
         buf.free()
+
+
+# Lanes per row of A x: as many as loads up to 3072 rows, whole rounds beyond;
+# units just below and above powers of two, odd k, one load per row.
+@pytest.mark.parametrize("m", [1, 3, 255, 3072, 3073])
+@pytest.mark.parametrize("k", [1, 2, 3, 31, 34, 63, 64, 65, 100, 128, 130, 200])
+def test_cgemv_n_lanes_exact(ctx, m, k):
+    rng = np.random.default_rng(m + k)
+    a = (rng.integers(-3, 4, (m, k)) + 1j * rng.integers(-3, 4, (m, k))).astype(np.complex64)
+    x = (rng.integers(-3, 4, k) + 1j * rng.integers(-3, 4, k)).astype(np.complex64)
+    A, X, Y = ctx.upload(a), ctx.upload(x), ctx.alloc((m + 1) * 8)
+    ctx.zero(Y)
+    ctx.cgemv(0, m, k, A, X, Y)
+    got = ctx.download(Y, np.complex64, (m + 1,))
+    want = a.astype(np.complex128) @ x.astype(np.complex128)
+    assert np.array_equal(got[:-1], want.astype(np.complex64)) and got[-1] == 0
+    for buf in (A, X, Y):
+        buf.free()
