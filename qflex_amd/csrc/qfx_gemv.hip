@@ -158,23 +158,40 @@ __global__ __launch_bounds__(1024) void gemv_n_block_kernel(const float2* __rest
   }
 }
 
-// Sum over the groups of a block of one value per thread, in a fixed tree:
+// Sums over the groups of a block of V values per thread, in a fixed tree:
 // thread t belongs to group t / CL (CL threads each, G = T / CL groups of the
-// block's T; the threads past G * CL take no part).  The result is in group 0.
-template <int T = 256>
-__device__ __forceinline__ float2 group_sum(float2 v, float2* red, int CL, int G) {
+// block's T; the threads past G * CL take no part).  The sums are in group 0.
+// Eight groups become one per step: halving them, for one value after the
+// other, took ten barriers of 16 waves (100 x 100 5.5 us, now 4.2; 256 x 64 6.1
+// and 4.8).
+template <int T, int V>
+__device__ __forceinline__ void group_sums(float2 (&v)[V], float2* red, int CL, int G) {
   const int t = threadIdx.x;
-  red[t] = v;
+#pragma unroll
+  for (int i = 0; i < V; ++i) red[i * T + t] = v[i];
   __syncthreads();
-  int w = T / 2;
-  while (w >= G && w > 1) w >>= 1;
-  for (; w > 0; w >>= 1) {  // group g takes over group g + w
-    if (t < w * CL && t + w * CL < G * CL) red[t] = cadd(red[t], red[t + w * CL]);
+  while (G > 1) {
+    const int left = (G + 7) / 8;  // group g < left takes over g + left, g + 2 left, ...
+    if (t < left * CL) {
+      float2 x[V][8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+          x[i][j] = t + j * left * CL < G * CL ? red[i * T + t + j * left * CL] : make_float2(0.f, 0.f);
+#pragma unroll
+      for (int i = 0; i < V; ++i)
+        v[i] = cadd(cadd(cadd(x[i][0], x[i][1]), cadd(x[i][2], x[i][3])),
+                    cadd(cadd(x[i][4], x[i][5]), cadd(x[i][6], x[i][7])));
+    }
+    G = left;
+    if (G == 1) break;
+    __syncthreads();
+    if (t < left * CL)
+#pragma unroll
+      for (int i = 0; i < V; ++i) red[i * T + t] = v[i];
     __syncthreads();
   }
-  const float2 r = red[t];
-  __syncthreads();
-  return r;
 }
 
 // y[c] = sum_r x[r] A[r][c] (A is m x k, row-major).  Block (x, y, z): column
@@ -189,7 +206,7 @@ __global__ __launch_bounds__(T) void gemv_t_kernel(const float2* __restrict__ A,
                                                      const float2* __restrict__ x,
                                                      float2* __restrict__ out, uint64_t M,
                                                      uint64_t K, uint64_t rows_per, int CL) {
-  __shared__ float2 red[T];
+  __shared__ float2 red[V * T];
   const int G = T / CL;
   const int rg = threadIdx.x / CL, cl = threadIdx.x - rg * CL;
   const uint64_t c = ((uint64_t(blockIdx.z) * gridDim.x + blockIdx.x) * CL + cl) * V;
@@ -222,17 +239,19 @@ __global__ __launch_bounds__(T) void gemv_t_kernel(const float2* __restrict__ A,
       for (int v = 0; v < V; ++v) acc[0][v] = cfma(x[r], a.e[v], acc[0][v]);
     }
   }
+  float2 sum[V];
 #pragma unroll
-  for (int v = 0; v < V; ++v) {
-    const float2 t = group_sum<T>(cadd(cadd(acc[0][v], acc[1][v]), cadd(acc[2][v], acc[3][v])), red,
-                               CL, G);
-    if (rg == 0 && in) out[blockIdx.y * K + c + v] = t;
-  }
+  for (int v = 0; v < V; ++v)
+    sum[v] = cadd(cadd(acc[0][v], acc[1][v]), cadd(acc[2][v], acc[3][v]));
+  group_sums<T, V>(sum, red, CL, G);
+  if (rg == 0 && in)
+#pragma unroll
+    for (int v = 0; v < V; ++v) out[blockIdx.y * K + c + v] = sum[v];
 }
 
 // The same for 256 threads and CL a power of two up to 64: in registers
-// within a wave, then over the four waves.  (With eight barriers of the tree
-// above a dot product of 100 values, two launches, took 4.5 us, 3.8 now.)
+// within a wave, then over the four waves.  (With a barrier per halving a dot
+// product of 100 values, two launches, took 4.5 us, 3.8 so.)
 __device__ __forceinline__ float2 lane_group_sum(float2 v, float2 (*red)[64], int CL) {
   const int lane = threadIdx.x & 63;
   for (int off = 32; off >= CL; off >>= 1) {
