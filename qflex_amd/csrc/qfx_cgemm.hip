@@ -1055,14 +1055,16 @@ struct GroupTile {
 
 // The operand maxima of all problems of a grouped launch: block b runs its
 // block of A or B of the problem whose partial maxima `first` + b is among.
-// (One launch per problem cost 3 us each.)
+// (One launch per problem cost 3 us each.)  A single problem comes as `one`,
+// without a list.
 __global__ __launch_bounds__(256) void amax_grouped_kernel(const GroupTile* __restrict__ probs,
-                                                           int count, float* __restrict__ part,
+                                                           GroupTile one, int count,
+                                                           float* __restrict__ part,
                                                            uint64_t first) {
   __shared__ float red[4];
   const uint64_t t = first + blockIdx.x;
-  const GroupTile& g =
-      probs[group_entry(&probs[0].first_part, sizeof(GroupTile), count, t)];
+  GroupTile g = one;
+  if (count > 1) g = probs[group_entry(&probs[0].first_part, sizeof(GroupTile), count, t)];
   const int b = int(t - g.first_part);
   const bool is_a = b < g.amax.na;
   const uint64_t m = uint64_t(g.M), n = uint64_t(g.N), k = uint64_t(g.K);
@@ -1074,14 +1076,16 @@ __global__ __launch_bounds__(256) void amax_grouped_kernel(const GroupTile* __re
 // (problems of any shape, tiles numbered problem by problem), each block
 // taking every gridDim.x-th tile; the blocks of an XCD take neighbouring ones,
 // which share B or A in its L2 (192 products of 512 x 128 x 64 48.6 -> 45.6 us, 150
-// of 300 x 99 x 101 57.8 -> 52.0, 200 of 700 x 250 x 32 143 -> 132).
+// of 300 x 99 x 101 57.8 -> 52.0, 200 of 700 x 250 x 32 143 -> 132).  A single
+// problem comes as `one`: the upload of its list took 3.5 us (one of 300 x 17 x
+// 33 15.3 -> 11.5, of 512 x 128 x 64 21.7 -> 18.2).
 template <int MODE, int WM, int WN, int J, bool ODD>
-__global__ __launch_bounds__(64 * WM * WN) void cgemm_split_grouped_kernel(const GroupTile* __restrict__ probs,
-                                                                  int count, uint64_t total) {
+__global__ __launch_bounds__(64 * WM * WN) void cgemm_split_grouped_kernel(
+    const GroupTile* __restrict__ probs, GroupTile one, int count, uint64_t total) {
   const qfx_index_map none{};
   for (uint64_t t = xcd_tile(blockIdx.x, gridDim.x); t < total; t += gridDim.x) {
-    const GroupTile g =
-        probs[group_entry(&probs[0].first_tile, sizeof(GroupTile), count, t)];
+    GroupTile g = one;
+    if (count > 1) g = probs[group_entry(&probs[0].first_tile, sizeof(GroupTile), count, t)];
     const uint64_t local = t - g.first_tile;
     const int tm = int(local % uint64_t(g.tiles_m)), tn = int(local / uint64_t(g.tiles_m));
     split_big_tile<MODE, WM, WN, J, 0, 2, false, false, ODD>(
@@ -2475,11 +2479,13 @@ static int launch_split_grouped(qfx_context* ctx, int precision, const qfx_gemm_
     t.amax = AmaxRef{part + off, ba, part + off + ba, bb};
     off += uint64_t(ba + bb);
   }
-  st = qfx_upload_problems(ctx, dev, host.data(), desc_bytes);
-  if (st != QFX_OK) return st;
+  if (host.size() > 1) {
+    st = qfx_upload_problems(ctx, dev, host.data(), desc_bytes);
+    if (st != QFX_OK) return st;
+  }
   for (uint64_t at = 0; at < nparts; at += kMaxBlocks)
     amax_grouped_kernel<<<unsigned(std::min<uint64_t>(kMaxBlocks, nparts - at)), 256, 0,
-                          ctx->stream>>>(dev, int(host.size()), part, at);
+                          ctx->stream>>>(dev, host[0], int(host.size()), part, at);
   QFX_HIP(hipGetLastError());
   if (ctx->cus <= 0) {
     int cus = 0;
@@ -2496,7 +2502,7 @@ static int launch_split_grouped(qfx_context* ctx, int precision, const qfx_gemm_
     const unsigned per_cu = unsigned(std::max<int>(1, int(kMaxLds) / kLds));
     const unsigned grid = unsigned(std::min<uint64_t>(tile, uint64_t(ctx->cus) * per_cu));
     cgemm_split_grouped_kernel<MODE, WM, WN, J, ODD><<<grid, 64 * WM * WN, kLds, ctx->stream>>>(
-        dev, int(grouped.size()), tile);
+        dev, host[0], int(host.size()), tile);
     return hipGetLastError();
   };
   if (precision == QFX_PREC_SPLIT_BF16X3) QFX_HIP(go(std::integral_constant<int, 0>{}));
