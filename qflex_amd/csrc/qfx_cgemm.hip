@@ -1738,10 +1738,12 @@ __device__ __forceinline__ void rows_tile(const float2* __restrict__ A,
   if constexpr (AROW) {
     const int per_row = K >> 1;  // 16-byte pieces per row; all of a thread's in flight
     float4 v[kSmallK / 2];
+    int at[kSmallK / 2];  // (kept: the divisions are most of a small product)
 #pragma unroll
     for (int h = 0; h < kSmallK / 2; ++h) {
       if (h >= per_row) break;
       const int q = threadIdx.x + 256 * h, r = q / per_row, p = q - r * per_row;
+      at[h] = r * kAPitch + 2 * p;
       const uint64_t grow = m0 + r;
       v[h] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (grow < M) {
@@ -1752,8 +1754,7 @@ __device__ __forceinline__ void rows_tile(const float2* __restrict__ A,
 #pragma unroll
     for (int h = 0; h < kSmallK / 2; ++h) {
       if (h >= per_row) break;
-      const int q = threadIdx.x + 256 * h, r = q / per_row, p = q - r * per_row;
-      *reinterpret_cast<float4*>(&X[r * kAPitch + 2 * p]) = v[h];
+      *reinterpret_cast<float4*>(&X[at[h]]) = v[h];
     }
   }
   __syncthreads();
