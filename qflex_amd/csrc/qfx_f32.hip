@@ -10,18 +10,19 @@
 // negated between them.  Lanes 0-31 hold the first two k of a group of four,
 // lanes 32-63 the other two.
 //
-// What bounds it: the MFMAs for large products (2048^3 runs at 119 TFLOP/s
-// and 2.1 GHz, where they could do 139), the chain of stages (1 us each, load
+// What bounds it: the MFMAs for large products (2048^3 ran at 119 TFLOP/s on
+// a card at 2.1 GHz, where they could do 139), the chain of stages (1 us each, load
 // to use) for small ones, which is why those take smaller tiles, deeper stages
 // and splits of k.  Measured against one 128 x 64 tile with selects between
 // the MFMAs, vector-ALU partial sums over 16 k each for up to 2^16 outputs,
-// and one thread per output for n < 16 or m < 64 (us):
-//   2048^3                    615 -> 584     300 x 300 x 300       52.4 -> 8.3
-//   65536 x 256 x 256         362 -> 350     256 x 256 x 4096      64.0 -> 31.6
-//   6145 x 515 x 333          105 ->  99     16 x 4096 x 4096       128 -> 60.3
-//   3719 x 642 x 516          156 -> 119     65536 x 8 x 1024       750 -> 360
-//   13066 x 36 x 948          160 ->  74     3000 x 2 x 900        99.4 -> 11.9
-//   57 x 104 x 3384           461 -> 10.7    86 x 169 x 470        80.7 -> 7.3
+// and one thread per output for n < 16 or m < 64 (us, in recorded sequences
+// over inputs that no cache holds):
+//   2048^3                    593 -> 556     300 x 300 x 300       53.2 -> 8.8
+//   65536 x 256 x 256         312 -> 300     256 x 256 x 4096      65.5 -> 30.2
+//   6145 x 515 x 333          106 ->  99     16 x 4096 x 4096       124 -> 55.6
+//   3719 x 642 x 516          157 -> 119     65536 x 8 x 1024       541 -> 125
+//   13066 x 36 x 948          163 ->  75     3000 x 2 x 900         253 -> 14.8
+//   57 x 104 x 3384          1050 -> 11.3    86 x 169 x 470        80.8 -> 7.5
 // Errors against complex128 are the same (128 x 64 tile) or lower (the other
 // tiles add their sums up once per stage): 57 x 104 x 3384 1e-6 -> 1e-7.
 #include <algorithm>

@@ -7,11 +7,13 @@
 // 256 CUs, for every aspect ratio: tall and narrow, short and wide.
 // Reductions run in a fixed order (no atomics): results are deterministic.
 // Measured against one wave per row (N) and against blocks that walked all
-// columns of 4 to 16 rows, 64 at a time (T), a plain copy running at 5.0 TB/s:
-//   T 4096 x 4096 (134 MB)   144 -> 23.0 us     N 4096 x 4096    36.7 -> 24.4 us
-//   T 227 x 37463 (68 MB)    842 -> 16.2 us     N 81 x 12430     51 -> 4.3 us
-//   T 16384 x 256 (34 MB)    74 -> 12.2 us      N 1000000 x 4    122 -> 7.8 us
-//   T 1000000 x 4 (32 MB)    141 -> 12.6 us     N 20000 x 2048   73.4 -> 62.1 us
+// columns of 4 to 16 rows, 64 at a time (T), in recorded sequences over inputs
+// that no cache holds (a 1 GiB copy runs at 5.2 TB/s):
+//   T 4096 x 4096 (134 MB)   145 -> 28.9 us     N 4096 x 4096    38.2 -> 26.1 us
+//   T 227 x 37463 (68 MB)    1220 -> 21.0 us    N 81 x 12430     89 -> 7.0 us
+//   T 16384 x 256 (34 MB)    78 -> 13.3 us      N 1000000 x 4    130 -> 10.1 us
+//   T 1000000 x 4 (32 MB)    172 -> 14.3 us     N 20000 x 2048   73.8 -> 63.0 us
+// The figures below are of the same kind where they name no other.
 #include <algorithm>
 
 #include "qfx_internal.h"
@@ -363,16 +365,16 @@ int qfx_launch_gemv_n(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
 int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A, const float2* x,
                       float2* y) {
   const int V = k % 2 == 0 && aligned16(A) ? 2 : 1;
-  // column lanes: the whole row up to 128 loads (300000 x 33: 44 -> 20 us
+  // column lanes: the whole row up to 128 loads (300000 x 33: 36.6 -> 26.9 us
   // against 64 lanes, 31 of them idle), else tiles of 64
   const uint64_t units = (k + V - 1) / V;
   const int CL = units <= 128 ? int(units) : 64;
   const uint64_t tile = uint64_t(V) * CL, tiles = (k + tile - 1) / tile;
   // Row splits: about 2048 blocks in all (8 per CU), each row group of a
-  // block with at least 16 rows (four rounds of the four in flight: with 8,
-  // 16384 x 256 took 29 instead of 12 us, most of it adding up 1024
-  // partials), at most 1024 splits of at least 16 rows (the scratch is then
-  // never more than 1024 x k values).
+  // block with at least 16 rows (four rounds of the four in flight; with 8,
+  // 16384 x 256 takes the same 13.3 us and twice the scratch), at most 1024
+  // splits of at least 16 rows (the scratch is then never more than 1024 x k
+  // values).
   const uint64_t G = 256 / CL;
   const uint64_t want = (2048 + tiles - 1) / tiles;
   uint64_t nsplit = std::min<uint64_t>({want, uint64_t(1024), (m + 16 * G - 1) / (16 * G),
@@ -386,11 +388,12 @@ int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
   if (tiles > tiles_x * 65535) return qfx_set_error(QFX_ERR_UNSUPPORTED, "gemv: too many columns");
   // Blocks of 1024 threads that take all rows of fewer columns save the
   // partials and their launch.  Taken with at most 32 rows per thread in at
-  // least 128 blocks (4096 x 4096: 28.2 -> 23.0 us, 5.8 TB/s; 1024 x 65536 98.2 ->
-  // 87.6; 227 x 37463 18.8 -> 16.2; with 63 blocks 1000 x 4000 took 13.0 instead
-  // of 8.7) and otherwise with at most 8 (100 x 100: 6.3 -> 5.2; with 23,
-  // 1409 x 17 took 8.1 instead of 6.2).  8-byte loads of many rows want the
-  // widest blocks (2047 x 8191: 37.8 with 16 columns, 27.6 split).
+  // least 128 blocks (4096 x 4096: 33.0 -> 28.9 us, 4.6 TB/s; 1024 x 65536 100 ->
+  // 90; 227 x 37463 22.2 -> 21.0; with 63 blocks 1000 x 4000 took 17.2 instead
+  // of 11.1) and otherwise with at most 8 (100 x 100: 5.0 -> 4.2; 1000 x 4000
+  // 11.1 -> 10.4; with 23, 1409 x 17 took 8.5 instead of 5.8).  8-byte loads of
+  // many rows want the widest blocks (2047 x 8191: 39.7 with 16 columns, 35.7
+  // split).
   for (uint64_t cl = units <= 64 ? units : 64; nsplit > 1 && cl > 0; cl /= 2) {
     const uint64_t cols = (units + cl - 1) / cl, rows = (m * cl + 1023) / 1024;
     const bool few = rows <= 8 && (cl == units || cl * V >= 16);
