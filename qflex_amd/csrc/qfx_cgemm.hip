@@ -2521,13 +2521,25 @@ extern "C" int qfx_cgemm_grouped_c64(qfx_context* ctx, int precision, int count,
     return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: invalid problem list");
   if (precision < QFX_PREC_FP32 || precision > QFX_PREC_FP8)
     return qfx_set_error(QFX_ERR_INVALID, "qfx_cgemm_grouped_c64: unknown precision");
-  // Every route's operands are checked here, before the first launch.
+  // Every route's operands are checked here, before the first launch (those in
+  // the arena: nothing is known about a caller's own memory).
+  const char *lo = nullptr, *hi = nullptr;
+  for (const auto& c : ctx->chunks) {
+    lo = lo ? std::min<const char*>(lo, c.base) : c.base;
+    hi = std::max<const char*>(hi, c.base + c.size);
+  }
+  auto check = [&](const qfx_c64* p, uint64_t rows, uint64_t cols, const char* what) {
+    const char* a = reinterpret_cast<const char*>(p);
+    return a < lo || a >= hi ? QFX_OK
+                             : qfx_check_extent(ctx, p, 8.0 * double(rows) * double(cols), what);
+  };
   for (int i = 0; i < count; ++i) {
     const qfx_gemm_desc& d = descs[i];
     if (d.m == 0 || d.n == 0 || d.k == 0 || !d.A || !d.B || !d.C) continue;  // qfx_cgemm_c64's cases
-    QFX_EXTENT(ctx, d.A, 8.0 * double(d.m) * double(d.k), "qfx_cgemm_grouped_c64: A");
-    QFX_EXTENT(ctx, d.B, 8.0 * double(d.k) * double(d.n), "qfx_cgemm_grouped_c64: B");
-    QFX_EXTENT(ctx, d.C, 8.0 * double(d.m) * double(d.n), "qfx_cgemm_grouped_c64: C");
+    int st = check(d.A, d.m, d.k, "qfx_cgemm_grouped_c64: A");
+    if (st == QFX_OK) st = check(d.B, d.k, d.n, "qfx_cgemm_grouped_c64: B");
+    if (st == QFX_OK) st = check(d.C, d.m, d.n, "qfx_cgemm_grouped_c64: C");
+    if (st != QFX_OK) return st;
   }
   const bool split = split_precision(precision);
   // One launch each for the problems of the large tiles, of the odd ones, of

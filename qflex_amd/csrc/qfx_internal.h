@@ -30,6 +30,17 @@ struct qfx_context {
   size_t chunk_bytes = size_t(1) << 30;
   std::map<size_t, std::vector<void*>> free_lists;
   std::map<void*, size_t> live;  // pointer -> rounded size
+  // Some of `live` by address, for operands that start their block (nearly
+  // all): the map's search took 50 ns of every check, 30 of the 865 us of a
+  // 4 x 4 circuit of depth 16 once its grouped products were checked.
+  struct LiveBlock {
+    const void* p;
+    size_t size;
+  };
+  std::array<LiveBlock, 1024> live_at{};
+  LiveBlock& live_slot(const void* p) {
+    return live_at[(reinterpret_cast<uintptr_t>(p) >> 8) % live_at.size()];
+  }
   size_t in_use = 0;
   // Device workspace for split reductions (grows on demand).
   void* work = nullptr;

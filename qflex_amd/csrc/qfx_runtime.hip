@@ -141,6 +141,7 @@ extern "C" int qfx_alloc(qfx_context* ctx, size_t bytes, void** dptr) {
     *dptr = p;
   }
   ctx->live[*dptr] = sz;
+  ctx->live_slot(*dptr) = {*dptr, sz};
   ctx->in_use += sz;
   return QFX_OK;
 }
@@ -163,6 +164,7 @@ extern "C" int qfx_free(qfx_context* ctx, void* dptr) {
   ctx->free_lists[it->second].push_back(dptr);
   ctx->in_use -= it->second;
   ctx->live.erase(it);
+  if (ctx->live_slot(dptr).p == dptr) ctx->live_slot(dptr) = {};
   return QFX_OK;
 }
 
@@ -177,6 +179,8 @@ extern "C" int qfx_arena_stats(qfx_context* ctx, size_t* reserved, size_t* in_us
 
 int qfx_check_extent(qfx_context* ctx, const void* p, double bytes, const char* what) {
   if (bytes <= 0) return QFX_OK;
+  const qfx_context::LiveBlock& at = ctx->live_slot(p);
+  if (at.p == p && bytes <= double(at.size)) return QFX_OK;
   const char* a = static_cast<const char*>(p);
   bool in_arena = false;
   for (const auto& c : ctx->chunks)

@@ -594,3 +594,31 @@ def test_cgemv_n_lanes_exact(ctx, m, k):
     assert np.array_equal(got[:-1], want.astype(np.complex64)) and got[-1] == 0
     for buf in (A, X, Y):
         buf.free()
+
+
+def test_operands_are_checked_against_live_blocks(ctx):
+    """More blocks than the table of their starts holds: each is accepted whole
+    while it lives, from its start and from inside, and refused when freed."""
+    class At:
+        def __init__(self, ptr):
+            self.ptr = ptr
+    bufs = [ctx.alloc(256) for _ in range(3000)]
+    starts = [b.ptr for b in bufs]
+    for p in starts:
+        ctx.zero(At(p), 256)
+        ctx.zero(At(p + 64), 192)
+    for p in starts[::100]:
+        for at, size in ((p, 257), (p + 64, 193)):
+            with pytest.raises(capi.QfxError, match="qfx_zero: dst"):
+                ctx.zero(At(at), size)
+    for b in bufs[::2]:
+        b.free()
+    for p, freed in zip(starts, [True, False] * 1500):
+        for at in (p, p + 64):
+            if freed:
+                with pytest.raises(capi.QfxError, match="qfx_zero: dst"):
+                    ctx.zero(At(at), 8)
+            else:
+                ctx.zero(At(at), 8)
+    for b in bufs[1::2]:
+        b.free()
