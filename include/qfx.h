@@ -45,7 +45,10 @@ enum qfx_status {
   QFX_ERR_UNSUPPORTED = 4
 };
 
-/* Arithmetic forms of the complex GEMM. */
+/* Arithmetic forms of the complex GEMM.  Products too small for the split
+ * tiles run in FP32 in the split precisions as well, which is the more exact
+ * form: k <= 16, m < 64 or n < 16, m*n <= 2^16 with k a multiple of 16 up to
+ * 4096, and even sizes of few tiles where FP32 is estimated to be faster. */
 enum qfx_precision {
   QFX_PREC_FP32 = 0,       /* FP32 MFMA, FP32 accumulate */
   QFX_PREC_SPLIT_BF16 = 1, /* A,B = hi+mid BF16; hi*hi + hi*mid + mid*hi, FP32 acc */
@@ -159,20 +162,22 @@ int qfx_cgemm_noalloc_c64(qfx_context* ctx, int precision, uint64_t m, uint64_t 
  * such products (numbered product by product), so many small or uneven
  * products fill the GPU together; each result is bit-identical to that
  * product computed alone on the 256 x 128 tile (split FP16: one max-abs
- * launch over all of them precedes the grouped launch).  The products with an
- * odd k or n or 8-byte aligned operands that qfx_cgemm_c64 would run split
- * share a second such launch, on 128 x 64 tiles (same bits).  Products with k <= 16
- * and n <= 16 (any precision) also share one launch, of the exact-FP32 row
- * kernel qfx_cgemm_c64 runs them on (same bits), and those with k <= 16 and
- * n > 16 another (same bits).  The products that are FP32 in the precision
- * share one launch per tile of the FP32 kernel, not split over k as small
- * ones are alone (the order of their sums, and so their last bits, may
- * differ; of 512 or more 128 x 64 tiles: run alone, same bits).  A
- * launch's problem list goes up as a kernel argument (up to 32) or through the
- * staged uploads.  All other products
- * run one by one through qfx_cgemm_c64.  The C_i must not overlap each other or
- * any A_j, B_j.  Not allowed while recording a graph.  No counterpart in the
- * reference (one cblas_cgemm per pairwise contraction, src/tensor.cpp:973). */
+ * launch over all of them precedes the grouped launch), also where alone it
+ * would run in FP32.  The products with an odd k or n or 8-byte aligned
+ * operands that qfx_cgemm_c64 would run split share a second such launch, on
+ * 128 x 64 tiles (same bits).  Products with k <= 16 and n <= 16 (any
+ * precision) also share one launch, of the exact-FP32 row kernel
+ * qfx_cgemm_c64 runs them on (same bits), and those with k <= 16 and n > 16
+ * another (same bits).  The products that are FP32 in the precision share one
+ * launch per tile of the FP32 kernel, not split over k as small ones are alone
+ * (the order of their sums, and so their last bits, may differ; of 512 or more
+ * 128 x 64 tiles: run alone, same bits).  A launch's problem list goes up as a
+ * kernel argument (up to 32, a single split product) or through the staged
+ * uploads.  All other products run one by one through qfx_cgemm_c64.  Every
+ * product's operands are checked against the arena's live blocks before the
+ * first launch.  The C_i must not overlap each other or any A_j, B_j.  Not
+ * allowed while recording a graph.  No counterpart in the reference (one
+ * cblas_cgemm per pairwise contraction, src/tensor.cpp:973). */
 typedef struct qfx_gemm_desc {
   uint64_t m, n, k;
   const qfx_c64* A;
@@ -199,9 +204,10 @@ typedef struct qfx_index_map {
  * orders of A and B, replacing the reorders of A to (left, common) and of
  * B to (common, right) plus _multiply_MM (src/tensor.cpp:1100-1128 and
  * :960-980).  m, n, k are the products of the maps' digit sizes.
- * Supported: the split precisions when m, n, k are large enough for the
- * MFMA tiles, any precision when k <= 16, and the non-exact precisions for
- * at most 8 x 8 outputs with k >= 1024; the operand read along its
+ * Supported: the split precisions and FP8 when m, n, k are large enough for
+ * their MFMA tiles, any precision when k <= 16, and the non-exact precisions
+ * for at most 8 x 8 outputs with k >= 1024 and, in FP32, for m*n <= 2^16 with
+ * k a multiple of 16 up to 4096; on the split tiles the operand read along its
  * contiguous axis needs digit 0 of that map at stride 1 with at least 3
  * bits.  Otherwise returns QFX_ERR_UNSUPPORTED without touching C (the
  * caller then reorders and calls qfx_cgemm_c64). */

@@ -365,8 +365,8 @@ int qfx_launch_gemv_n(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A,
 int qfx_launch_gemv_t(qfx_context* ctx, uint64_t m, uint64_t k, const float2* A, const float2* x,
                       float2* y) {
   const int V = k % 2 == 0 && aligned16(A) ? 2 : 1;
-  // column lanes: the whole row up to 128 loads (300000 x 33: 36.6 -> 26.9 us
-  // against 64 lanes, 31 of them idle), else tiles of 64
+  // column lanes: the whole row up to 128 loads (300000 x 33: 27 to 29 us,
+  // 36.6 with 64 lanes, 31 of them idle), else tiles of 64
   const uint64_t units = (k + V - 1) / V;
   const int CL = units <= 128 ? int(units) : 64;
   const uint64_t tile = uint64_t(V) * CL, tiles = (k + tile - 1) / tile;
